@@ -28,6 +28,7 @@
 #include <string>
 
 #include "../../include/cuwave_amd.h"
+#include "common.hpp"
 
 namespace cwh {
 int fail(const std::string &what);
@@ -41,8 +42,6 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kThreads = 256;
-constexpr int kBM = 128; // pixels a forward block takes (4 waves x 32)
-constexpr int kBK = 16;  // reduction step: 16 channels of one tap
 
 __device__ __forceinline__ uint16_t to_bf16(float v) {
   const uint32_t bits = __float_as_uint(v);
@@ -73,76 +72,156 @@ __device__ __forceinline__ int64_t shifted(const Image &im, int64_t p, int tap) 
 }
 
 // ------------------------------------------------------------ forward
-// one block: 128 pixels x BN output channels (BN = cout, 32 / 64 / 128);
-// wave w takes pixels 32 w .. 32 w + 31 and every channel
-template <int BN>
+// One block: a tile of kTH x kTW pixels of one image and every output channel
+// (BN = cout, 32 / 64 / 128). What bounds it is the LDS, then HBM: a 32 -> 32
+// layer has 36 flops a byte of activations, so the input has to reach the
+// block once. The tile's input with its one-pixel halo is staged KC channels
+// at a time and read nine times from LDS, with the KC channels' weights beside
+// it; the nine taps need no further load and no barrier between them. A wave
+// holds RW rows of 32 pixels by NT tiles of 32 channels and keeps the RW + 2
+// input rows of a column shift in registers for the three taps that share
+// them, so a tap costs a wave NT weight reads and a third of RW + 2 input
+// reads for RW NT matrix instructions.
+//
+// The matrix instruction's rows are channels and its columns pixels, so a lane
+// ends with runs of four channels of one pixel; the two halves of the wave
+// trade runs and store 16 bytes each. Blocks go to the XCDs in contiguous runs
+// of tiles: the halo a tile shares with its neighbours is in the same L2.
+constexpr int kTH = 8, kTW = 32;
+constexpr int kHaloW = kTW + 2, kHaloPixels = (kTH + 2) * kHaloW;
+
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  const bf16x2 v = {(__bf16)lo, (__bf16)hi};
+  return __builtin_bit_cast(uint32_t, v);
+}
+
+// the 16-byte slot of chunk c of staged pixel p: the chunks of a pixel are
+// permuted by its place among 16, so 16 neighbouring pixels' same chunk sits
+// in 16 different slots of the 64 banks
+template <int S> __device__ __forceinline__ int staged(int p, int c) {
+  return p * S + (c ^ (S == 4 ? (p >> 2) & 3 : (p >> 3) & 1));
+}
+
+template <int BN, int KC>
 __global__ void __launch_bounds__(kThreads)
-conv3x3_fwd(Image im, int cin, const uint4 *__restrict__ x, const uint4 *__restrict__ wt,
-            const float *__restrict__ bias, int relu, uint16_t *__restrict__ y) {
-  __shared__ uint4 sa[2][kBM * 2];  // [m][k]: 16 bf16 a row, two uint4
-  __shared__ uint4 sb[2][BN * 2];   // [n][k]
+conv3x3_fwd(Image im, int tiles_x, int tiles_y, int cin, const uint4 *__restrict__ x,
+            const uint4 *__restrict__ wt, const float *__restrict__ bias, int relu,
+            uint16_t *__restrict__ y) {
+  constexpr int S = KC / 8;                     // 16-byte chunks a pixel a stage
+  constexpr int WN = BN == 128 ? 2 : 1;         // waves along the channels
+  constexpr int RW = kTH * WN / 4;              // pixel rows a wave
+  constexpr int NT = BN / WN / 32;              // channel tiles a wave
+  __shared__ uint4 sx[kHaloPixels * S];
+  __shared__ uint4 sw[9 * S * BN];              // [tap][chunk][channel]
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-  const int64_t m0 = (int64_t)blockIdx.x * kBM;
-  const int steps = 9 * (cin / kBK);
-  const int cin8 = cin / 8;      // uint4 chunks a pixel
-  const int krow8 = 9 * cin8;    // uint4 chunks a weight row
-  // the chunk this thread stages: pixel am, half ah; weight row bn, half bh
-  const int am = tid / 2, ah = tid % 2;
-  const int bn = tid / 2, bh = tid % 2;
-  uint4 ra = {0, 0, 0, 0}, rb = {0, 0, 0, 0};
-  auto load = [&](int s) {
-    const int tap = s / (cin / kBK), c0 = (s % (cin / kBK)) * kBK;
-    const int64_t p = m0 + am;
-    ra = uint4{0, 0, 0, 0};
-    if (p < im.pixels) {
-      const int64_t q = shifted(im, p, tap);
-      if (q >= 0)
-        ra = x[q * cin8 + c0 / 8 + ah];
+  const int tile = cw::xcd_tile(blockIdx.x, gridDim.x);
+  const int x0 = tile % tiles_x * kTW, y0 = tile / tiles_x % tiles_y * kTH;
+  const int base = tile / (tiles_x * tiles_y) * im.h * im.w;  // the image's first pixel
+  const int cin8 = cin / 8, krow8 = 9 * cin8;
+  const int row0 = wave / WN * RW, n0 = wave % WN * (32 * NT);
+  f32x16 acc[RW][NT];
+#pragma unroll
+  for (int i = 0; i < RW; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        acc[i][j][r] = 0.0f;
+  for (int c0 = 0; c0 < cin8; c0 += S) {
+    if (c0)
+      __syncthreads();
+#pragma unroll
+    for (int k = 0; k < (kHaloPixels * S + kThreads - 1) / kThreads; ++k) {
+      const int t = tid + k * kThreads;
+      const int c = t % S, p = t / S;
+      const int py = y0 + p / kHaloW - 1, px = x0 + p % kHaloW - 1;
+      if (p < kHaloPixels) {
+        uint4 v = {0, 0, 0, 0};
+        if (py >= 0 && py < im.h && px >= 0 && px < im.w)
+          v = x[(int64_t)(base + py * im.w + px) * cin8 + c0 + c];
+        sx[staged<S>(p, c)] = v;
+      }
     }
-    if (bn < BN)
-      rb = wt[(int64_t)bn * krow8 + tap * cin8 + c0 / 8 + bh];
-  };
-  f32x16 acc[BN / 32];
 #pragma unroll
-  for (int j = 0; j < BN / 32; ++j)
-#pragma unroll
-    for (int r = 0; r < 16; ++r)
-      acc[j][r] = 0.0f;
-  load(0);
-  for (int s = 0; s < steps; ++s) {
-    const int buf = s & 1;
-    sa[buf][am * 2 + ah] = ra;
-    if (bn < BN)
-      sb[buf][bn * 2 + bh] = rb;
+    for (int k = 0; k < (9 * S * BN + kThreads - 1) / kThreads; ++k) {
+      const int t = tid + k * kThreads;
+      const int c = t % S, n = t / S % BN, tap = t / (S * BN);
+      if (tap < 9)
+        sw[(tap * S + c) * BN + n] = wt[n * krow8 + tap * cin8 + c0 + c];
+    }
     __syncthreads();
-    if (s + 1 < steps)
-      load(s + 1);
-    const uint4 a = sa[buf][(wave * 32 + lane % 32) * 2 + lane / 32];
-    const bf16x8 av = __builtin_bit_cast(bf16x8, a);
 #pragma unroll
-    for (int j = 0; j < BN / 32; ++j) {
-      const uint4 b = sb[buf][(j * 32 + lane % 32) * 2 + lane / 32];
-      acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, __builtin_bit_cast(bf16x8, b),
-                                                      acc[j], 0, 0, 0);
+    for (int kk = 0; kk < KC / 16; ++kk) {
+      const int c = 2 * kk + lane / 32;
+#pragma unroll
+      for (int dw = 0; dw < 3; ++dw) {
+        bf16x8 in[RW + 2];
+#pragma unroll
+        for (int i = 0; i < RW + 2; ++i)
+          in[i] = __builtin_bit_cast(
+              bf16x8, sx[staged<S>((row0 + i) * kHaloW + lane % 32 + dw, c)]);
+#pragma unroll
+        for (int dh = 0; dh < 3; ++dh)
+#pragma unroll
+          for (int j = 0; j < NT; ++j) {
+            const bf16x8 w = __builtin_bit_cast(
+                bf16x8, sw[((3 * dh + dw) * S + c) * BN + n0 + 32 * j + lane % 32]);
+#pragma unroll
+            for (int i = 0; i < RW; ++i)
+              acc[i][j] =
+                  __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, in[i + dh], acc[i][j], 0, 0, 0);
+          }
+      }
     }
   }
-  // epilogue: bias, activation, bfloat16
+  // epilogue: bias, activation, bfloat16; accumulator register r of a lane is
+  // channel 8 (r / 4) + 4 (lane / 32) + r % 4 of pixel lane % 32
+  const int px = x0 + lane % 32, half = lane / 32;
 #pragma unroll
-  for (int j = 0; j < BN / 32; ++j) {
-    const int n = j * 32 + lane % 32;
-    const float b = bias ? bias[n] : 0.0f;
+  for (int j = 0; j < NT; ++j) {
+    const int n = n0 + 32 * j;
+    float4 b[4];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int m = wave * 32 + 8 * (r / 4) + 4 * (lane / 32) + r % 4;
-      const int64_t p = m0 + m;
-      if (p >= im.pixels)
-        continue;
-      float v = acc[j][r] + b;
-      if (relu)
-        v = v > 0.0f ? v : 0.0f;
-      y[p * BN + n] = to_bf16(v);
+    for (int q = 0; q < 4; ++q)
+      b[q] = bias ? *reinterpret_cast<const float4 *>(bias + n + 8 * q + 4 * half)
+                  : float4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+      const int py = y0 + row0 + i;
+      uint2 v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float f[4] = {acc[i][j][4 * q] + b[q].x, acc[i][j][4 * q + 1] + b[q].y,
+                      acc[i][j][4 * q + 2] + b[q].z, acc[i][j][4 * q + 3] + b[q].w};
+        if (relu)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            f[e] = f[e] > 0.0f ? f[e] : 0.0f;
+        v[q] = uint2{pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3])};
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q += 2) {
+        // the low half keeps run q and takes the high half's, the high half
+        // run q + 1: eight channels in order each
+        const uint2 give = half ? v[q] : v[q + 1];
+        const uint2 got = {__shfl_xor(give.x, 32), __shfl_xor(give.y, 32)};
+        const uint4 out = half ? uint4{got.x, got.y, v[q + 1].x, v[q + 1].y}
+                               : uint4{v[q].x, v[q].y, got.x, got.y};
+        if (px < im.w && py < im.h)
+          *reinterpret_cast<uint4 *>(y + (int64_t)(base + py * im.w + px) * BN + n + 8 * q +
+                                     8 * half) = out;
+      }
     }
   }
+}
+
+template <int BN, int KC>
+void launch_fwd(const cw_conv3x3_args &a, const Image &im, hipStream_t s) {
+  const int tx = (a.w + kTW - 1) / kTW, ty = (a.h + kTH - 1) / kTH;
+  hipLaunchKernelGGL((conv3x3_fwd<BN, KC>), dim3(tx * ty * a.n), dim3(kThreads), 0, s, im, tx, ty,
+                     a.cin, (const uint4 *)a.x, (const uint4 *)a.weight, (const float *)a.bias,
+                     a.relu, (uint16_t *)a.y);
 }
 
 // ------------------------------------------------------- backward weight
@@ -336,15 +415,17 @@ int cw_conv3x3_bf16_fwd(const cw_conv3x3_args *a, void *stream) {
   if (!a->x || !a->weight || !a->y)
     return fail("the forward needs x, weight and y");
   const Image im{a->n, a->h, a->w, (int64_t)a->n * a->h * a->w};
-  const int blocks = (int)((im.pixels + kBM - 1) / kBM);
   const auto s = (hipStream_t)stream;
-  const uint4 *x = (const uint4 *)a->x, *w = (const uint4 *)a->weight;
-  const float *bias = (const float *)a->bias;
-  uint16_t *y = (uint16_t *)a->y;
+  const bool wide = a->cin % 32 == 0;
   switch (a->cout) {
-  case 32: hipLaunchKernelGGL(conv3x3_fwd<32>, dim3(blocks), dim3(kThreads), 0, s, im, a->cin, x, w, bias, a->relu, y); break;
-  case 64: hipLaunchKernelGGL(conv3x3_fwd<64>, dim3(blocks), dim3(kThreads), 0, s, im, a->cin, x, w, bias, a->relu, y); break;
-  default: hipLaunchKernelGGL(conv3x3_fwd<128>, dim3(blocks), dim3(kThreads), 0, s, im, a->cin, x, w, bias, a->relu, y); break;
+  case 32:
+    wide ? launch_fwd<32, 32>(*a, im, s) : launch_fwd<32, 16>(*a, im, s);
+    break;
+  case 64:
+    launch_fwd<64, 16>(*a, im, s);
+    break;
+  default:
+    launch_fwd<128, 16>(*a, im, s);
   }
   return hip_status("conv3x3_fwd");
 }

@@ -128,3 +128,39 @@ def test_training_fits_a_target_on_the_gpu():
         losses.append(loss.item())
     assert np.isfinite(losses).all()
     assert losses[-1] < 0.3 * losses[0]
+
+
+@pytest.mark.parametrize("n, h, w, cin, cout", [
+    (1, 1, 1, 32, 32),      # smaller than any tile
+    (3, 8, 32, 32, 64),     # whole tiles of pixels
+    (2, 7, 31, 64, 32),     # one short of a tile
+    (1, 9, 65, 16, 128),    # one past a tile, half a channel chunk
+    (2, 17, 33, 48, 64),    # a channel count of the 16-channel chunks only
+    (1, 40, 130, 96, 128),  # several tiles and chunks each way
+])
+def test_a_convolution_at_its_tiles_edges(n, h, w, cin, cout):
+    print(f"case conv3x3 {n}x{h}x{w} {cin}->{cout}", flush=True)
+    g = torch.Generator().manual_seed(h * 100 + w)
+    x = _bf(torch.randn(n, h, w, cin, generator=g))
+    conv = unet.Conv3x3(cin, cout, True)
+    with torch.no_grad():
+        conv.weight.copy_(_bf(conv.weight))
+    ref_x = x.clone().double().requires_grad_(True)
+    ref_w = conv.weight.detach().clone().double().requires_grad_(True)
+    ref_b = conv.bias.detach().clone().double().requires_grad_(True)
+    ref = O.conv3x3(ref_x, ref_w, ref_b, True)
+    conv = conv.cuda()
+    xg = x.cuda().to(torch.bfloat16).requires_grad_(cin in (32, 64, 128))
+    y = conv(xg)
+    # half an ulp of bfloat16 (2^-9) and the float32 sums of 9 cin terms
+    err = (y.detach().double().cpu() - ref.detach()).abs()
+    assert float((err - ref.detach().abs() * 2.0**-8).max()) <= 1e-5
+    dy = _bf(torch.randn(n, h, w, cout, generator=g))
+    # outputs whose sign the rounding could turn carry no gradient
+    dy = torch.where(ref.detach().abs() < 1e-4, torch.zeros_like(dy), dy)
+    y.backward(dy.cuda().to(torch.bfloat16))
+    ref.backward(dy.double())
+    assert _rel(conv.weight.grad, ref_w.grad) < 1e-4
+    assert _rel(conv.bias.grad, ref_b.grad) < 1e-5
+    if xg.requires_grad:  # bfloat16 outputs: 2^-9 relative each
+        assert _rel(xg.grad, ref_x.grad) < 4e-3
