@@ -178,26 +178,27 @@ conv3x3_fwd(Image im, int tiles_x, int tiles_y, int cin, const uint4 *__restrict
   // epilogue: bias, activation, bfloat16; accumulator register r of a lane is
   // channel 8 (r / 4) + 4 (lane / 32) + r % 4 of pixel lane % 32
   const int px = x0 + lane % 32, half = lane / 32;
+  const bool wide = (reinterpret_cast<uintptr_t>(y) & 15) == 0; // else two bytes a store
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     const int n = n0 + 32 * j;
-    float4 b[4];
+    float b[16];
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      b[q] = bias ? *reinterpret_cast<const float4 *>(bias + n + 8 * q + 4 * half)
-                  : float4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int r = 0; r < 16; ++r)
+      b[r] = bias ? bias[n + 8 * (r / 4) + 4 * half + r % 4] : 0.0f;
 #pragma unroll
     for (int i = 0; i < RW; ++i) {
       const int py = y0 + row0 + i;
       uint2 v[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        float f[4] = {acc[i][j][4 * q] + b[q].x, acc[i][j][4 * q + 1] + b[q].y,
-                      acc[i][j][4 * q + 2] + b[q].z, acc[i][j][4 * q + 3] + b[q].w};
-        if (relu)
+        float f[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
+        for (int e = 0; e < 4; ++e) {
+          f[e] = acc[i][j][4 * q + e] + b[4 * q + e];
+          if (relu)
             f[e] = f[e] > 0.0f ? f[e] : 0.0f;
+        }
         v[q] = uint2{pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3])};
       }
 #pragma unroll
@@ -208,9 +209,16 @@ conv3x3_fwd(Image im, int tiles_x, int tiles_y, int cin, const uint4 *__restrict
         const uint2 got = {__shfl_xor(give.x, 32), __shfl_xor(give.y, 32)};
         const uint4 out = half ? uint4{got.x, got.y, v[q + 1].x, v[q + 1].y}
                                : uint4{v[q].x, v[q].y, got.x, got.y};
-        if (px < im.w && py < im.h)
-          *reinterpret_cast<uint4 *>(y + (int64_t)(base + py * im.w + px) * BN + n + 8 * q +
-                                     8 * half) = out;
+        if (px >= im.w || py >= im.h)
+          continue;
+        uint16_t *to = y + (int64_t)(base + py * im.w + px) * BN + n + 8 * q + 8 * half;
+        if (wide) {
+          *reinterpret_cast<uint4 *>(to) = out;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            to[e] = (uint16_t)((&out.x)[e / 2] >> (16 * (e & 1)));
+        }
       }
     }
   }
@@ -225,126 +233,228 @@ void launch_fwd(const cw_conv3x3_args &a, const Image &im, hipStream_t s) {
 }
 
 // ------------------------------------------------------- backward weight
-// one block: 128 rows of the (tap, ci) axis x BN output channels, summed
-// over its run of pixels 32 at a time; the partial goes to part[split]
-template <int BN>
-__global__ void __launch_bounds__(kThreads)
-conv3x3_wgrad(Image im, int cin, const uint4 *__restrict__ x, const uint4 *__restrict__ dy,
-              int64_t run, float *__restrict__ part) {
-  constexpr int P = 32; // pixels a step
-  __shared__ __attribute__((aligned(16))) uint16_t sx[2][128][P + 8];
-  __shared__ __attribute__((aligned(16))) uint16_t sd[2][BN][P + 8];
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-  const int krows = 9 * cin;
-  const int r0 = blockIdx.x * 128;
-  const int split = blockIdx.y;
-  const int64_t p_begin = (int64_t)split * run;
-  const int64_t p_end = p_begin + run < im.pixels ? p_begin + run : im.pixels;
-  const int cin8 = cin / 8;
-  constexpr int cout8 = BN / 8;
-  constexpr int DPT = (P * cout8 + kThreads - 1) / kThreads; // dy chunks a thread
-  // staging: x chunk (pixel xp, rows xr .. xr + 7) twice; dy chunks (pixel dp,
-  // channels dc .. dc + 7)
-  uint4 rx[2], rd[DPT];
-  auto load = [&](int64_t q0) {
+// dw[co][tap][ci] = sum over pixels of dy[co] x shifted by the tap: a product
+// whose reduction runs along the pixels, so both operands are wanted with
+// eight neighbouring pixels of one channel a lane where memory has eight
+// channels of one pixel. A thread takes four pixels by eight channels and
+// writes them to LDS transposed (two packed pixels an instruction).
+//
+// A block marches down the rows of a strip of kWStrip columns, CI input and CO
+// output channels wide, two input rows in LDS (one being filled) and a ring of
+// four gradient rows. An input row meets the gradient rows below, at and above
+// it, and its eight-pixel runs shifted by -1, 0 and +1 pixel come from one
+// 16-byte read and the words either side: nine matrix instructions for four
+// and a half LDS reads, every tap of a (CI, CO) tile accumulated in one pass
+// over the data. What bounds it is HBM: x and dy are read once for every 64
+// channels of the other. The nine tiles of sums are 144 registers, so two
+// blocks a CU; the host asks for splits that give each CU its two.
+//
+// The waves take the (32, 32) channel tiles, and where there are fewer than
+// four the strip's 16-column steps between them, summed through LDS at the
+// end. Each split's sums go to its own workspace slice and a second kernel
+// adds the slices in a fixed order (deterministic, no atomics).
+constexpr int kWStrip = 64;
+
+// the 16-byte slot of eight-pixel run k of channel c, a row of eight runs: 16
+// neighbouring channels' same run, and the same run of channels eight apart,
+// fall in different slots of the 64 banks
+__device__ __forceinline__ int run_slot(int c, int k) {
+  return c * 8 + (k ^ ((c >> 1 ^ c >> 3) & 7));
+}
+
+// four pixels of eight channels (one uint4 a pixel) into a transposed row:
+// pixels 4 q .. 4 q + 3 of channels 8 cg .. 8 cg + 7
+__device__ __forceinline__ void put_transposed(uint4 *row, int cg, int q, const uint4 *v) {
+  const uint32_t *w[4] = {&v[0].x, &v[1].x, &v[2].x, &v[3].x};
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int t = tid + h * kThreads;       // 512 chunks: 32 pixels x 16
-      const int xp = t / 16, xr = r0 + (t % 16) * 8;
-      rx[h] = uint4{0, 0, 0, 0};
-      const int64_t p = q0 + xp;
-      if (p < p_end && xr < krows) {
-        const int tap = xr / cin, ci = xr % cin;
-        const int64_t q = shifted(im, p, tap);
-        if (q >= 0)
-          rx[h] = x[q * cin8 + ci / 8];
-      }
-    }
-#pragma unroll
-    for (int h = 0; h < DPT; ++h) {
-      const int t = tid + h * kThreads;
-      const int dp = t / cout8, dc = (t % cout8) * 8;
-      rd[h] = uint4{0, 0, 0, 0};
-      const int64_t p = q0 + dp;
-      if (dp < P && p < p_end)
-        rd[h] = dy[p * cout8 + dc / 8];
-    }
-  };
-  f32x16 acc[BN / 32];
-#pragma unroll
-  for (int j = 0; j < BN / 32; ++j)
-#pragma unroll
-    for (int r = 0; r < 16; ++r)
-      acc[j][r] = 0.0f;
-  const int64_t steps = (p_end - p_begin + P - 1) / P;
-  if (steps > 0)
-    load(p_begin);
-  for (int64_t s = 0; s < steps; ++s) {
-    const int buf = (int)(s & 1);
-    // transposed into LDS: [row][pixel], [channel][pixel]
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int t = tid + h * kThreads;
-      const int xp = t / 16, xr = (t % 16) * 8;
-      const uint16_t *v = reinterpret_cast<const uint16_t *>(&rx[h]);
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        sx[buf][xr + i][xp] = v[i];
-    }
-#pragma unroll
-    for (int h = 0; h < DPT; ++h) {
-      const int t = tid + h * kThreads;
-      const int dp = t / cout8, dc = (t % cout8) * 8;
-      if (dp < P) {
-        const uint16_t *v = reinterpret_cast<const uint16_t *>(&rd[h]);
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          sd[buf][dc + i][dp] = v[i];
-      }
-    }
-    __syncthreads();
-    if (s + 1 < steps)
-      load(p_begin + (s + 1) * P);
-    // rows of P + 8 bfloat16 (80 bytes), so a lane's eight pixels are one
-    // aligned 16-byte LDS read
-#pragma unroll
-    for (int k = 0; k < P; k += 16) {
-      const bf16x8 av = __builtin_bit_cast(
-          bf16x8, *reinterpret_cast<const uint4 *>(&sx[buf][wave * 32 + lane % 32][k + 8 * (lane / 32)]));
-#pragma unroll
-      for (int j = 0; j < BN / 32; ++j) {
-        const bf16x8 bv = __builtin_bit_cast(
-            bf16x8, *reinterpret_cast<const uint4 *>(&sd[buf][j * 32 + lane % 32][k + 8 * (lane / 32)]));
-        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc[j], 0, 0, 0);
-      }
-    }
-  }
-  // the partial: part[split][row][co]
-  float *out = part + (int64_t)split * krows * BN;
-#pragma unroll
-  for (int j = 0; j < BN / 32; ++j) {
-    const int n = j * 32 + lane % 32;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = r0 + wave * 32 + 8 * (r / 4) + 4 * (lane / 32) + r % 4;
-      if (row < krows)
-        out[(int64_t)row * BN + n] = acc[j][r];
-    }
+  for (int i = 0; i < 8; ++i) {
+    // the low or the high halves of two pixels' word i / 2
+    const uint32_t pick = i & 1 ? 0x07060302u : 0x05040100u;
+    const uint2 two = {__builtin_amdgcn_perm(w[1][i / 2], w[0][i / 2], pick),
+                       __builtin_amdgcn_perm(w[3][i / 2], w[2][i / 2], pick)};
+    reinterpret_cast<uint2 *>(&row[run_slot(8 * cg + i, q / 2)])[q & 1] = two;
   }
 }
 
-// dw[co][row] = sum over the splits in order of part[split][row][co]
-__global__ void __launch_bounds__(kThreads)
-conv3x3_wgrad_sum(int krows, int cout, int splits, const float *__restrict__ part,
-                  float *__restrict__ dw) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (int64_t)krows * cout)
+template <int CI, int CO>
+__global__ void __launch_bounds__(kThreads, 2)
+conv3x3_wgrad(Image im, int strips, int cin, int cout, const uint4 *__restrict__ x,
+              const uint4 *__restrict__ dy, int run, float *__restrict__ part) {
+  constexpr int TI = CI / 32, TO = CO / 32;
+  constexpr int KW = 4 / (TI * TO);       // waves that share a tile
+  constexpr int KS = kWStrip / 16 / KW;   // 16-column steps a wave takes
+  __shared__ uint4 sx[2][CI * 8];
+  __shared__ uint32_t halo[2][2][CI];     // the pixel left (high half) and right (low half)
+  __shared__ uint4 sd[4][CO * 8];
+  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64, half = lane / 32;
+  const int kw = wave % KW, ti = wave / KW % TI, to = wave / (KW * TI);
+  const int ciblocks = (cin + CI - 1) / CI;
+  const int ci0 = blockIdx.x % ciblocks * CI, co0 = blockIdx.x / ciblocks * CO;
+  const int split = blockIdx.y;
+  const int cin8 = cin / 8, cout8 = cout / 8;
+  // staging: threads 0 .. 127 four pixels of x each, the rest of dy (CI = 32
+  // or CO = 32 fill half of theirs), 2 CI / 8 threads a halo pixel too
+  const bool on_x = tid < 128;
+  const int task = on_x ? tid : tid - 128;
+  const int groups = on_x ? CI / 8 : CO / 8;
+  const int cg = task % groups, q = task / groups;
+  const bool mine = q < kWStrip / 4 && (!on_x || ci0 + 8 * cg < cin);
+  const bool zeroed = on_x && q < kWStrip / 4 && ci0 + 8 * cg >= cin; // channels past the last
+  const bool edge = tid < 2 * (CI / 8);
+  const int ecg = tid % (CI / 8), eside = tid / (CI / 8);
+  f32x16 acc[9];
+#pragma unroll
+  for (int j = 0; j < 9; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      acc[j][r] = 0.0f;
+  // the split's run of gradient rows, strip after strip of each image
+  const int64_t total = (int64_t)im.n * strips * im.h;
+  int64_t at = (int64_t)split * run;
+  const int64_t end = at + run < total ? at + run : total;
+  while (at < end) {
+    const int s = (int)(at / im.h);
+    const int a = (int)(at - (int64_t)s * im.h);
+    const int b = (int)(end - (int64_t)s * im.h < im.h ? end - (int64_t)s * im.h : im.h);
+    at += b - a;
+    const int c0 = s % strips * kWStrip;                 // the strip's first column
+    const int base = s / strips * im.h * im.w;           // the image's first pixel
+    uint4 v[4], ev;
+    // input row r into the x registers, gradient row r + 1 into the dy ones
+    auto fetch = [&](int r) {
+      const int row = on_x ? r : r + 1;
+      const bool there = on_x ? r >= 0 && r < im.h : row >= a && row < b;
+      const uint4 *src = on_x ? x + ci0 / 8 + cg : dy + co0 / 8 + cg;
+      const int step = on_x ? cin8 : cout8;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int col = c0 + 4 * q + i;
+        v[i] = uint4{0, 0, 0, 0};
+        if (mine && there && col < im.w)
+          v[i] = src[(int64_t)(base + row * im.w + col) * step];
+      }
+      const int col = eside ? c0 + kWStrip : c0 - 1;
+      ev = uint4{0, 0, 0, 0};
+      if (edge && r >= 0 && r < im.h && col >= 0 && col < im.w && ci0 + 8 * ecg < cin)
+        ev = x[(int64_t)(base + r * im.w + col) * cin8 + ci0 / 8 + ecg];
+    };
+    auto stage = [&](int r) {
+      if (mine || zeroed)
+        put_transposed(on_x ? sx[r & 1] : sd[(r + 1) & 3], cg, q, v);
+      if (edge) {
+        const uint32_t *w = &ev.x;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const uint32_t px = i & 1 ? w[i / 2] >> 16 : w[i / 2] & 0xffffu;
+          halo[r & 1][eside][8 * ecg + i] = eside ? px : px << 16;
+        }
+      }
+    };
+    __syncthreads(); // the rows of the segment before have been read
+    fetch(a - 1);
+    stage(a - 1);
+    for (int r = a - 1; r <= b; ++r) {
+      __syncthreads();
+      if (r < b)
+        fetch(r + 1);
+      const uint4 *xr = sx[r & 1];
+      const int ci = 32 * ti + lane % 32, co = 32 * to + lane % 32;
+#pragma unroll
+      for (int k = 0; k < KS; ++k) {
+        const int g = 2 * (kw + KW * k) + half; // this lane's run of eight pixels
+        const uint4 m = xr[run_slot(ci, g)];
+        const uint32_t left =
+            g ? xr[run_slot(ci, g ? g - 1 : 0)].w : halo[r & 1][0][ci];
+        const uint32_t right =
+            g < 7 ? xr[run_slot(ci, g < 7 ? g + 1 : 7)].x : halo[r & 1][1][ci];
+        const uint32_t a0 = __builtin_amdgcn_alignbit(m.x, left, 16);
+        const uint32_t a1 = __builtin_amdgcn_alignbit(m.y, m.x, 16);
+        const uint32_t a2 = __builtin_amdgcn_alignbit(m.z, m.y, 16);
+        const uint32_t a3 = __builtin_amdgcn_alignbit(m.w, m.z, 16);
+        const uint32_t a4 = __builtin_amdgcn_alignbit(right, m.w, 16);
+        const bf16x8 in[3] = {__builtin_bit_cast(bf16x8, uint4{a0, a1, a2, a3}),
+                              __builtin_bit_cast(bf16x8, m),
+                              __builtin_bit_cast(bf16x8, uint4{a1, a2, a3, a4})};
+#pragma unroll
+        for (int dh = 0; dh < 3; ++dh) {
+          const int row = r + 1 - dh; // the gradient row whose tap dh is input row r
+          if (row < a || row >= b)
+            continue;
+          const bf16x8 d = __builtin_bit_cast(bf16x8, sd[row & 3][run_slot(co, g)]);
+#pragma unroll
+          for (int dw = 0; dw < 3; ++dw)
+            acc[3 * dh + dw] =
+                __builtin_amdgcn_mfma_f32_32x32x16_bf16(d, in[dw], acc[3 * dh + dw], 0, 0, 0);
+        }
+      }
+      if (r < b)
+        stage(r + 1);
+    }
+  }
+  // the waves of a tile summed into its first, a tap at a time
+  if constexpr (KW > 1) {
+    float *sums = reinterpret_cast<float *>(sd); // (KW - 1) tiles' 4 KB fit the ring
+    static_assert(sizeof(sd) >= (size_t)TI * TO * (KW - 1) * 4096, "the sums need room");
+#pragma unroll
+    for (int j = 0; j < 9; ++j) {
+      __syncthreads();
+      if (kw)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          sums[(((ti + TI * to) * (KW - 1) + kw - 1) * 16 + r) * 64 + lane] = acc[j][r];
+      __syncthreads();
+      if (!kw)
+        for (int o = 0; o < KW - 1; ++o)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            acc[j][r] += sums[(((ti + TI * to) * (KW - 1) + o) * 16 + r) * 64 + lane];
+    }
+    if (kw)
+      return;
+  }
+  // the partial: part[split][co][tap][ci], dw's own order
+  const int ci = ci0 + 32 * ti + lane % 32;
+  if (ci >= cin)
     return;
-  const int row = (int)(t / cout), co = (int)(t % cout);
+  float *out = part + (int64_t)split * cout * 9 * cin;
+#pragma unroll
+  for (int j = 0; j < 9; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int co = co0 + 32 * to + 8 * (r / 4) + 4 * half + r % 4;
+      out[(co * 9 + j) * cin + ci] = acc[j][r];
+    }
+}
+
+// dw = the sum over the splits: a thread one value of every fourth split, eight
+// loads in flight, the four threads' sums then added in order
+__global__ void __launch_bounds__(kThreads)
+conv3x3_wgrad_sum(int total, int splits, const float *__restrict__ part,
+                  float *__restrict__ dw) {
+  __shared__ float sums[4][64];
+  const int lane = threadIdx.x % 64, group = threadIdx.x / 64;
+  const int t = blockIdx.x * 64 + lane;
   float s = 0.0f;
-  for (int k = 0; k < splits; ++k)
-    s += part[((int64_t)k * krows + row) * cout + co];
-  dw[(int64_t)co * krows + row] = s;
+  if (t < total) {
+#pragma unroll 8
+    for (int k = group; k < splits; k += 4)
+      s += part[(int64_t)k * total + t];
+  }
+  sums[group][lane] = s;
+  __syncthreads();
+  if (group || t >= total)
+    return;
+  dw[t] = s + sums[1][lane] + sums[2][lane] + sums[3][lane];
+}
+
+template <int CI, int CO>
+void launch_wgrad(const cw_conv3x3_args &a, const Image &im, hipStream_t s) {
+  const int strips = (a.w + kWStrip - 1) / kWStrip;
+  const int64_t rows = (int64_t)a.n * strips * a.h;
+  const int run = (int)((rows + a.splits - 1) / a.splits);
+  hipLaunchKernelGGL((conv3x3_wgrad<CI, CO>), dim3((a.cin + CI - 1) / CI * (a.cout / CO), a.splits),
+                     dim3(kThreads), 0, s, im, strips, a.cin, a.cout, (const uint4 *)a.x,
+                     (const uint4 *)a.dy, run, (float *)a.workspace);
 }
 
 // the kernels' weights from the float32 master: wt (cout, 9 cin) as is and
@@ -455,23 +565,16 @@ int cw_conv3x3_bf16_bwd_weight(const cw_conv3x3_args *a, void *stream) {
   if (!a->x || !a->dy || !a->dweight || !a->workspace || a->splits < 1)
     return fail("the backward weight pass needs x, dy, dweight, a workspace and splits");
   const Image im{a->n, a->h, a->w, (int64_t)a->n * a->h * a->w};
-  const int krows = 9 * a->cin;
-  const int64_t run = (im.pixels + a->splits - 1) / a->splits;
-  const dim3 grid((krows + 127) / 128, a->splits);
   const auto s = (hipStream_t)stream;
-  const uint4 *x = (const uint4 *)a->x, *dy = (const uint4 *)a->dy;
-  float *part = (float *)a->workspace;
-  switch (a->cout) {
-  case 32: hipLaunchKernelGGL(conv3x3_wgrad<32>, grid, dim3(kThreads), 0, s, im, a->cin, x, dy, run, part); break;
-  case 64: hipLaunchKernelGGL(conv3x3_wgrad<64>, grid, dim3(kThreads), 0, s, im, a->cin, x, dy, run, part); break;
-  default: hipLaunchKernelGGL(conv3x3_wgrad<128>, grid, dim3(kThreads), 0, s, im, a->cin, x, dy, run, part); break;
-  }
+  if (a->cin <= 32)
+    a->cout == 32 ? launch_wgrad<32, 32>(*a, im, s) : launch_wgrad<32, 64>(*a, im, s);
+  else
+    a->cout == 32 ? launch_wgrad<64, 32>(*a, im, s) : launch_wgrad<64, 64>(*a, im, s);
   if (int e = hip_status("conv3x3_wgrad"))
     return e;
-  const int64_t total = (int64_t)krows * a->cout;
-  hipLaunchKernelGGL(conv3x3_wgrad_sum, dim3((int)((total + kThreads - 1) / kThreads)),
-                     dim3(kThreads), 0, s, krows, a->cout, a->splits, (const float *)part,
-                     (float *)a->dweight);
+  const int total = 9 * a->cin * a->cout;
+  hipLaunchKernelGGL(conv3x3_wgrad_sum, dim3((total + 63) / 64), dim3(kThreads), 0, s, total,
+                     a->splits, (const float *)a->workspace, (float *)a->dweight);
   return hip_status("conv3x3_wgrad_sum");
 }
 

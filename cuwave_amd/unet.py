@@ -40,9 +40,13 @@ def _bf16_weights(w: torch.Tensor, cout: int, cin: int, flipped: bool):
     return wt, wd
 
 
-def _splits(pixels: int) -> int:
-    """Pixel runs a weight gradient sums apart: about 2 k pixels each, 16 .. 256 runs."""
-    return max(16, min(256, pixels // 2048))
+def _splits(n: int, h: int, w: int, cin: int, cout: int) -> int:
+    """Pixel runs a weight gradient sums apart: its kernel takes two blocks a CU (256 CUs),
+    so 512 blocks over the channel tiles of 64, each of at least 12 rows of a 64-column
+    strip (shorter runs spend their time on the slices)."""
+    tiles = max(1, -(-cin // 64)) * max(1, cout // 64)
+    rows = n * h * -(-w // 64)
+    return max(1, min(512 // tiles, rows // 12))
 
 
 class _Conv3x3(torch.autograd.Function):
@@ -82,7 +86,7 @@ class _Conv3x3(torch.autograd.Function):
             dx = torch.empty_like(x)
             a.weight_flipped, a.dx = _abi.ptr(ctx.wflip), _abi.ptr(dx)
             _abi.call("cw_conv3x3_bf16_bwd_data", ctypes.byref(a), _abi.stream())
-        splits = _splits(n * h * w)
+        splits = _splits(n, h, w, cin, cout)
         work = torch.empty((splits, 9 * cin, cout), dtype=torch.float32, device=x.device)
         dweight = torch.empty((cout, 9 * cin), dtype=torch.float32, device=x.device)
         a.workspace, a.splits, a.dweight = _abi.ptr(work), splits, _abi.ptr(dweight)
