@@ -389,6 +389,9 @@ SIGNATURES = {
     "cw_conv3x3_bf16_bwd_data": ([ctypes.POINTER(Conv3x3Args), VP], I32),
     "cw_conv3x3_bf16_bwd_weight": ([ctypes.POINTER(Conv3x3Args), VP], I32),
     "cw_conv3x3_weights": ([I32, I32, VP, VP, VP, VP], I32),
+    "cw_relu_bias_grad": ([I64, I32, VP, VP, VP, VP, I32, VP, VP], I32),
+    "cw_head_fwd": ([I64, I32, VP, VP, VP, VP, VP], I32),
+    "cw_head_bwd": ([I64, I32, VP, VP, VP, VP, VP, I32, VP, VP], I32),
     "cw_adamw": ([ctypes.POINTER(AdamWArgs), VP], I32),
 }
 

@@ -426,11 +426,10 @@ conv3x3_wgrad(Image im, int strips, int cin, int cout, const uint4 *__restrict__
     }
 }
 
-// dw = the sum over the splits: a thread one value of every fourth split, eight
+// out = the sum over the slices: a thread one value of every fourth slice, eight
 // loads in flight, the four threads' sums then added in order
 __global__ void __launch_bounds__(kThreads)
-conv3x3_wgrad_sum(int total, int splits, const float *__restrict__ part,
-                  float *__restrict__ dw) {
+slices_sum(int total, int splits, const float *__restrict__ part, float *__restrict__ out) {
   __shared__ float sums[4][64];
   const int lane = threadIdx.x % 64, group = threadIdx.x / 64;
   const int t = blockIdx.x * 64 + lane;
@@ -444,7 +443,163 @@ conv3x3_wgrad_sum(int total, int splits, const float *__restrict__ part,
   __syncthreads();
   if (group || t >= total)
     return;
-  dw[t] = s + sums[1][lane] + sums[2][lane] + sums[3][lane];
+  out[t] = s + sums[1][lane] + sums[2][lane] + sums[3][lane];
+}
+
+void launch_slices_sum(int total, int slices, const void *part, void *out, hipStream_t s) {
+  hipLaunchKernelGGL(slices_sum, dim3((total + 63) / 64), dim3(kThreads), 0, s, total, slices,
+                     (const float *)part, (float *)out);
+}
+
+// ------------------------------------------------- passes over activations
+// Both run at HBM's rate with 16 bytes (eight channels of a pixel) a thread:
+// what they save is passes. Per-channel sums stay in registers over a block's
+// pixels, are added over the block's threads of a channel in a fixed order,
+// and leave as one slice a block for slices_sum.
+__device__ __forceinline__ void unpack8(const uint4 &v, float *f) {
+  const uint32_t *w = &v.x;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    f[2 * i] = __uint_as_float(w[i] << 16);
+    f[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+  }
+}
+
+// the N values a thread holds summed over the block's threads t % G equal,
+// thread t < G ending with its sums
+template <int N, int G>
+__device__ __forceinline__ void block_sums(float *s, float *lds) {
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+#pragma unroll
+    for (int m = G; m < 64; m <<= 1)
+      s[i] += __shfl_xor(s[i], m);
+    if (lane < G)
+      lds[(wave * N + i) * G + lane] = s[i];
+  }
+  __syncthreads();
+  if (threadIdx.x < G)
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      s[i] = lds[i * G + threadIdx.x];
+      for (int o = 1; o < kThreads / 64; ++o)
+        s[i] += lds[(o * N + i) * G + threadIdx.x];
+    }
+}
+
+// the gradient before the activation, dy where y > 0, and its sums over the
+// pixels (the bias' gradient) in the same pass: 6 bytes a value instead of the
+// 16 of a comparison, a select, a conversion and a sum. y NULL (no
+// activation): the sums alone
+template <int C>
+__global__ void __launch_bounds__(kThreads)
+relu_bias_grad(int64_t chunks, const uint4 *__restrict__ dy, const uint4 *__restrict__ y,
+               uint4 *__restrict__ dpre, float *__restrict__ part) {
+  constexpr int G = C / 8;
+  __shared__ float lds[kThreads / 64 * 8 * G];
+  float s[8] = {};
+  const int64_t step = (int64_t)gridDim.x * kThreads; // a multiple of G
+  for (int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x; t < chunks; t += step) {
+    uint4 d = dy[t];
+    if (y) {
+      float f[8];
+      const uint4 yy = y[t];
+      unpack8(yy, f);
+      uint32_t *w = &d.x;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        w[i] &= (f[2 * i] > 0.0f ? 0xffffu : 0u) | (f[2 * i + 1] > 0.0f ? 0xffff0000u : 0u);
+      dpre[t] = d;
+    }
+    float f[8];
+    unpack8(d, f);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      s[i] += f[i];
+  }
+  block_sums<8, G>(s, lds);
+  if (threadIdx.x < G)
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      part[(int64_t)blockIdx.x * C + threadIdx.x * 8 + i] = s[i];
+}
+
+// the 1x1 output layer on kHeadC channels: y[p][o] = b[o] + sum_c x[p][c] w[c][o],
+// float32 from bfloat16 activations, four threads a pixel
+constexpr int kHeadC = 32, kHeadG = kHeadC / 8;
+
+template <int O>
+__global__ void __launch_bounds__(kThreads)
+head_fwd(int64_t pixels, const uint4 *__restrict__ x, const float *__restrict__ w,
+         const float *__restrict__ b, float *__restrict__ y) {
+  const int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  const int c = 8 * (threadIdx.x % kHeadG);
+  const int64_t p = t / kHeadG;
+  float f[8] = {};
+  if (p < pixels)
+    unpack8(x[t], f);
+#pragma unroll
+  for (int o = 0; o < O; ++o) {
+    float s = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      s += f[i] * w[(c + i) * O + o];
+#pragma unroll
+    for (int m = 1; m < kHeadG; m <<= 1)
+      s += __shfl_xor(s, m);
+    if (p < pixels && c == 0)
+      y[p * O + o] = s + b[o];
+  }
+}
+
+// its gradients in one pass: dx = dy w^T in bfloat16, and the sums x^T dy and
+// dy over the pixels as slices (kHeadC O values of dw, then O of db)
+template <int O>
+__global__ void __launch_bounds__(kThreads)
+head_bwd(int64_t pixels, const uint4 *__restrict__ x, const float *__restrict__ w,
+         const float *__restrict__ dy, uint4 *__restrict__ dx, float *__restrict__ part) {
+  __shared__ float lds[kThreads / 64 * 9 * O * kHeadG];
+  const int c = 8 * (threadIdx.x % kHeadG);
+  float ws[8 * O], s[9 * O] = {};
+#pragma unroll
+  for (int i = 0; i < 8 * O; ++i)
+    ws[i] = w[c * O + i];
+  const int64_t step = (int64_t)gridDim.x * kThreads;
+  for (int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x; t / kHeadG < pixels; t += step) {
+    float f[8], d[O];
+#pragma unroll
+    for (int o = 0; o < O; ++o)
+      d[o] = dy[t / kHeadG * O + o];
+    unpack8(x[t], f);
+    float g[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      g[i] = 0.0f;
+#pragma unroll
+      for (int o = 0; o < O; ++o) {
+        g[i] += d[o] * ws[i * O + o];
+        s[i * O + o] += f[i] * d[o];
+      }
+    }
+#pragma unroll
+    for (int o = 0; o < O; ++o)
+      s[8 * O + o] += d[o];
+    if (dx)
+      dx[t] = uint4{pack_bf16(g[0], g[1]), pack_bf16(g[2], g[3]), pack_bf16(g[4], g[5]),
+                    pack_bf16(g[6], g[7])};
+  }
+  block_sums<9 * O, kHeadG>(s, lds);
+  if (threadIdx.x >= kHeadG)
+    return;
+  float *out = part + (int64_t)blockIdx.x * (kHeadC + 1) * O;
+#pragma unroll
+  for (int i = 0; i < 8 * O; ++i)
+    out[c * O + i] = s[i];
+  if (c == 0)
+#pragma unroll
+    for (int o = 0; o < O; ++o)
+      out[kHeadC * O + o] = s[8 * O + o];
 }
 
 template <int CI, int CO>
@@ -573,9 +728,8 @@ int cw_conv3x3_bf16_bwd_weight(const cw_conv3x3_args *a, void *stream) {
   if (int e = hip_status("conv3x3_wgrad"))
     return e;
   const int total = 9 * a->cin * a->cout;
-  hipLaunchKernelGGL(conv3x3_wgrad_sum, dim3((total + 63) / 64), dim3(kThreads), 0, s, total,
-                     a->splits, (const float *)a->workspace, (float *)a->dweight);
-  return hip_status("conv3x3_wgrad_sum");
+  launch_slices_sum(total, a->splits, a->workspace, a->dweight, s);
+  return hip_status("slices_sum");
 }
 
 int cw_conv3x3_weights(int32_t cout, int32_t cin, const void *w, void *wt, void *wd,
@@ -587,6 +741,70 @@ int cw_conv3x3_weights(int32_t cout, int32_t cin, const void *w, void *wt, void 
                      dim3(kThreads), 0, (hipStream_t)stream, cout, cin, (const float *)w,
                      (uint16_t *)wt, (uint16_t *)wd);
   return hip_status("conv3x3_weights");
+}
+
+int cw_relu_bias_grad(int64_t pixels, int32_t channels, const void *dy, const void *y, void *dpre,
+                      void *workspace, int32_t slices, void *dbias, void *stream) {
+  if (pixels < 1 || !dy || !workspace || !dbias || slices < 1)
+    return fail("the bias gradient needs pixels, dy, a workspace, slices and dbias");
+  if (channels != 32 && channels != 64 && channels != 128)
+    return fail("channels must be 32, 64 or 128");
+  if (y && !dpre)
+    return fail("a masked gradient needs dpre");
+  const int64_t chunks = pixels * (channels / 8);
+  const auto s = (hipStream_t)stream;
+  const uint4 *d = (const uint4 *)dy, *yy = (const uint4 *)y;
+  uint4 *out = (uint4 *)dpre;
+  float *part = (float *)workspace;
+  const dim3 grid(slices), block(kThreads);
+  switch (channels) {
+  case 32: hipLaunchKernelGGL(relu_bias_grad<32>, grid, block, 0, s, chunks, d, yy, out, part); break;
+  case 64: hipLaunchKernelGGL(relu_bias_grad<64>, grid, block, 0, s, chunks, d, yy, out, part); break;
+  default: hipLaunchKernelGGL(relu_bias_grad<128>, grid, block, 0, s, chunks, d, yy, out, part); break;
+  }
+  launch_slices_sum(channels, slices, workspace, dbias, s);
+  return hip_status("relu_bias_grad");
+}
+
+int cw_head_fwd(int64_t pixels, int32_t outputs, const void *x, const void *w, const void *b, void *y,
+                void *stream) {
+  if (pixels < 1 || !x || !w || !b || !y)
+    return fail("the output layer needs pixels, x, w, b and y");
+  const int64_t threads = pixels * kHeadG;
+  const dim3 grid((int)((threads + kThreads - 1) / kThreads)), block(kThreads);
+  const auto s = (hipStream_t)stream;
+  const uint4 *xx = (const uint4 *)x;
+  const float *ww = (const float *)w, *bb = (const float *)b;
+  float *yy = (float *)y;
+  switch (outputs) {
+  case 1: hipLaunchKernelGGL(head_fwd<1>, grid, block, 0, s, pixels, xx, ww, bb, yy); break;
+  case 2: hipLaunchKernelGGL(head_fwd<2>, grid, block, 0, s, pixels, xx, ww, bb, yy); break;
+  case 3: hipLaunchKernelGGL(head_fwd<3>, grid, block, 0, s, pixels, xx, ww, bb, yy); break;
+  case 4: hipLaunchKernelGGL(head_fwd<4>, grid, block, 0, s, pixels, xx, ww, bb, yy); break;
+  default: return fail("the output layer is built for 1 to 4 outputs");
+  }
+  return hip_status("head_fwd");
+}
+
+int cw_head_bwd(int64_t pixels, int32_t outputs, const void *x, const void *w, const void *dy, void *dx,
+                void *workspace, int32_t slices, void *dwb, void *stream) {
+  if (pixels < 1 || !x || !w || !dy || !workspace || !dwb || slices < 1)
+    return fail("the output layer's backward needs pixels, x, w, dy, a workspace, slices and dwb");
+  const dim3 grid(slices), block(kThreads);
+  const auto s = (hipStream_t)stream;
+  const uint4 *xx = (const uint4 *)x;
+  const float *ww = (const float *)w, *dd = (const float *)dy;
+  uint4 *out = (uint4 *)dx;
+  float *part = (float *)workspace;
+  switch (outputs) {
+  case 1: hipLaunchKernelGGL(head_bwd<1>, grid, block, 0, s, pixels, xx, ww, dd, out, part); break;
+  case 2: hipLaunchKernelGGL(head_bwd<2>, grid, block, 0, s, pixels, xx, ww, dd, out, part); break;
+  case 3: hipLaunchKernelGGL(head_bwd<3>, grid, block, 0, s, pixels, xx, ww, dd, out, part); break;
+  case 4: hipLaunchKernelGGL(head_bwd<4>, grid, block, 0, s, pixels, xx, ww, dd, out, part); break;
+  default: return fail("the output layer is built for 1 to 4 outputs");
+  }
+  launch_slices_sum((kHeadC + 1) * outputs, slices, workspace, dwb, s);
+  return hip_status("head_bwd");
 }
 
 int cw_adamw(const cw_adamw_args *a, void *stream) {

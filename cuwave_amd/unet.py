@@ -5,9 +5,10 @@ its weights) runs in the hand-written bfloat16 MFMA kernels of
 `csrc/unet.hip` with float32 accumulation, through the C ABI
 (`cw_conv3x3_bf16_fwd` / `_bwd_data` / `_bwd_weight`), and the optimiser step
 is the library's AdamW kernel (`cw_adamw`). Activations are NHWC bfloat16,
-master weights float32. The pooling, the 2x2 up-convolutions (plain GEMMs
-on the library's bfloat16 matrix multiply), the concatenations and the 1x1
-output stay in torch.
+master weights float32. The 1x1 output layer and the pass back through a
+ReLU (with the bias' gradient) are the library's too. The pooling, the 2x2
+up-convolutions (plain GEMMs on the library's bfloat16 matrix multiply) and
+the concatenations stay in torch.
 
 No reference counterpart: the reference has no learned preconditioner.
 There is no CPU path; without the library or a GPU the network raises.
@@ -42,11 +43,17 @@ def _bf16_weights(w: torch.Tensor, cout: int, cin: int, flipped: bool):
 
 def _splits(n: int, h: int, w: int, cin: int, cout: int) -> int:
     """Pixel runs a weight gradient sums apart: its kernel takes two blocks a CU (256 CUs),
-    so 512 blocks over the channel tiles of 64, each of at least 12 rows of a 64-column
-    strip (shorter runs spend their time on the slices)."""
+    so 512 blocks over the channel tiles of 64, each of at least 6 rows of a 64-column
+    strip (below that the slices cost more than the CUs they occupy give)."""
     tiles = max(1, -(-cin // 64)) * max(1, cout // 64)
     rows = n * h * -(-w // 64)
-    return max(1, min(512 // tiles, rows // 12))
+    return max(1, min(512 // tiles, rows // 6))
+
+
+def _slices(threads: int) -> int:
+    """Blocks of a summing pass over activations, a slice each: four a CU, fewer where
+    the pass has fewer than 256 threads a block."""
+    return max(1, min(1024, -(-threads // 256)))
 
 
 class _Conv3x3(torch.autograd.Function):
@@ -73,10 +80,17 @@ class _Conv3x3(torch.autograd.Function):
         x, y = ctx.saved_tensors
         n, h, w, cin = x.shape
         cout = y.shape[-1]
-        dy = dy.to(torch.bfloat16)
-        if ctx.relu:
-            dy = torch.where(y > 0, dy, torch.zeros((), dtype=dy.dtype, device=dy.device))
-        dy = dy.contiguous()
+        dy = dy.to(torch.bfloat16).contiguous()
+        # the gradient before the activation and the bias' gradient, one pass
+        pixels = n * h * w
+        slices = _slices(pixels * cout // 8)
+        dpre = torch.empty_like(dy) if ctx.relu else None
+        work = torch.empty((slices, cout), dtype=torch.float32, device=x.device)
+        dbias = torch.empty(cout, dtype=torch.float32, device=x.device)
+        _abi.call("cw_relu_bias_grad", pixels, cout, _abi.ptr(dy),
+                  _abi.ptr(y) if ctx.relu else None, _abi.ptr(dpre), _abi.ptr(work), slices,
+                  _abi.ptr(dbias), _abi.stream())
+        dy = dpre if ctx.relu else dy
         a = _args(n, h, w, cin, cout)
         a.x, a.dy = _abi.ptr(x), _abi.ptr(dy)
         dx = None
@@ -91,8 +105,35 @@ class _Conv3x3(torch.autograd.Function):
         dweight = torch.empty((cout, 9 * cin), dtype=torch.float32, device=x.device)
         a.workspace, a.splits, a.dweight = _abi.ptr(work), splits, _abi.ptr(dweight)
         _abi.call("cw_conv3x3_bf16_bwd_weight", ctypes.byref(a), _abi.stream())
-        dbias = dy.float().sum((0, 1, 2))
         return dx, dweight, dbias, None
+
+
+class _Head(torch.autograd.Function):
+    """y = x w + b in float32, x (n, h, w, 32) bfloat16, w (32, 1 .. 4)."""
+
+    @staticmethod
+    def forward(ctx, x: torch.Tensor, w: torch.Tensor, b: torch.Tensor):
+        x, w = x.contiguous(), w.contiguous()
+        n, h, wd, _ = x.shape
+        y = torch.empty((n, h, wd, w.shape[1]), dtype=torch.float32, device=x.device)
+        _abi.call("cw_head_fwd", n * h * wd, w.shape[1], _abi.ptr(x), _abi.ptr(w.detach()),
+                  _abi.ptr(b.detach()), _abi.ptr(y), _abi.stream())
+        ctx.save_for_backward(x, w)
+        return y
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dy: torch.Tensor):
+        x, w = ctx.saved_tensors
+        outputs, pixels = w.shape[1], x.numel() // x.shape[-1]
+        dy = dy.contiguous()
+        slices = _slices(pixels * 4)
+        dx = torch.empty_like(x) if ctx.needs_input_grad[0] else None
+        work = torch.empty((slices, 33 * outputs), dtype=torch.float32, device=x.device)
+        dwb = torch.empty(33 * outputs, dtype=torch.float32, device=x.device)
+        _abi.call("cw_head_bwd", pixels, outputs, _abi.ptr(x), _abi.ptr(w.detach()), _abi.ptr(dy),
+                  _abi.ptr(dx), _abi.ptr(work), slices, _abi.ptr(dwb), _abi.stream())
+        return dx, dwb[:32 * outputs].view(32, outputs), dwb[32 * outputs:]
 
 
 class Conv3x3(nn.Module):
@@ -164,6 +205,8 @@ class UNet(nn.Module):
         m = self.mid(_pool(e2))
         d2 = self.dec2(torch.cat([self.up2(m), e2], -1).contiguous())
         d1 = self.dec1(torch.cat([self.up1(d2), e1], -1).contiguous())
+        if d1.shape[-1] == 32 and self.out_w.shape[1] <= 4 and self.out_w.dtype == torch.float32:
+            return _Head.apply(d1, self.out_w, self.out_b)
         return d1.float() @ self.out_w + self.out_b
 
 

@@ -543,6 +543,24 @@ int cw_conv3x3_bf16_bwd_weight(const cw_conv3x3_args *args, void *stream);
 int cw_conv3x3_weights(int32_t cout, int32_t cin, const void *w, void *wt, void *wd,
                        void *stream);
 
+/* the gradient before a ReLU, dpre = dy where y > 0 (the dy of the convolution's
+ * backward passes), and its sum over the pixels (dbias, float32) in the same
+ * pass; y NULL: no activation, the sums of dy alone (dpre unused). dy, y and
+ * dpre (pixels, channels) bfloat16, 16-byte aligned, channels 32, 64 or 128;
+ * workspace slices x channels float32, a slice a block */
+int cw_relu_bias_grad(int64_t pixels, int32_t channels, const void *dy, const void *y, void *dpre,
+                      void *workspace, int32_t slices, void *dbias, void *stream);
+/* the 1x1 output layer on 32 channels, y = x w + b in float32: x (pixels, 32)
+ * bfloat16 (16-byte aligned), w (32, outputs), b (outputs), y (pixels,
+ * outputs), outputs 1 to 4 */
+int cw_head_fwd(int64_t pixels, int32_t outputs, const void *x, const void *w, const void *b, void *y,
+                void *stream);
+/* its gradients in one pass: dx (pixels, 32) bfloat16 (or NULL), and in dwb the
+ * (32, outputs) gradient at w, then the (outputs) one at b; workspace slices x
+ * 33 outputs float32 */
+int cw_head_bwd(int64_t pixels, int32_t outputs, const void *x, const void *w, const void *dy, void *dx,
+                void *workspace, int32_t slices, void *dwb, void *stream);
+
 /* one AdamW step over `count` float32 parameters (decoupled weight decay,
  * bias-corrected moments; the update torch.optim.AdamW makes) */
 typedef struct cw_adamw_args {

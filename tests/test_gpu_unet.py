@@ -164,3 +164,24 @@ def test_a_convolution_at_its_tiles_edges(n, h, w, cin, cout):
     assert _rel(conv.bias.grad, ref_b.grad) < 1e-5
     if xg.requires_grad:  # bfloat16 outputs: 2^-9 relative each
         assert _rel(xg.grad, ref_x.grad) < 4e-3
+
+
+@pytest.mark.parametrize("shape, outputs", [((1, 1, 1), 1), ((1, 7, 9), 2), ((2, 8, 8), 3),
+                                            ((3, 61, 67), 4), ((4, 260, 300), 1)])
+def test_the_output_layer_and_its_gradients(shape, outputs):
+    print(f"case head {shape} outputs={outputs}", flush=True)
+    g = torch.Generator().manual_seed(outputs)
+    x = _bf(torch.randn(*shape, 32, generator=g))
+    w, b = torch.randn(32, outputs, generator=g), torch.randn(outputs, generator=g)
+    dy = torch.randn(*shape, outputs, generator=g)
+    ref = [t.double().requires_grad_(True) for t in (x, w, b)]
+    out = ref[0] @ ref[1] + ref[2]
+    out.backward(dy.double())
+    ours = [t.cuda().requires_grad_(True) for t in (x.bfloat16(), w, b)]
+    y = unet._Head.apply(*ours)
+    y.backward(dy.cuda())
+    # float32 sums of 32 terms, then of the pixels in slices; dx rounded to bfloat16
+    assert _rel(y, out) < 1e-6
+    assert _rel(ours[1].grad, ref[1].grad) < 1e-5
+    assert _rel(ours[2].grad, ref[2].grad) < 1e-5
+    assert _rel(ours[0].grad, ref[0].grad) < 4e-3
