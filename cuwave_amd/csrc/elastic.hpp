@@ -134,32 +134,46 @@ __device__ __forceinline__ Line<T> field_line(const T *p, int64_t idx, const ElG
 }
 
 // ------------------------------------------- staggered SBP derivatives
-// closure rows off a wall (cuwave/kernels/common.cuh:214-242)
-template <int NDIM, typename Q, typename T>
-__device__ Q node_rows(const ElGeom<T> &g, const Line<T> &L, int k, int lo, int hi) {
+// closure rows off a wall (cuwave/kernels/common.cuh:214-242): the row's span
+// is read four points at a time (past its end the last point again, the term
+// dropped), so that a wall node waits on memory once for four points and not
+// once for each
+template <int NDIM, typename Q, typename T, typename At>
+__device__ __forceinline__ Q closure_row(const T *row, int span, bool low, At at) {
   Q acc((T)0);
-  if (lo < g.nc) {
-    for (int m = 0; m < g.nspan; ++m)
-      acc += g.rows[lo * g.nspan + m] * line_at<NDIM, Q>(L, k, m - lo);
-  } else {
-    for (int m = 0; m < g.nspan; ++m)
-      acc -= g.rows[hi * g.nspan + m] * line_at<NDIM, Q>(L, k, hi - 1 - m);
+  for (int m0 = 0; m0 < span; m0 += 4) {
+    T w[4];
+    Q v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int m = m0 + i < span ? m0 + i : span - 1;
+      w[i] = row[m];
+      v[i] = at(m);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const Q term = w[i] * v[i];
+      acc = m0 + i >= span ? acc : low ? acc + term : acc - term;
+    }
   }
   return acc;
 }
 
 template <int NDIM, typename Q, typename T>
+__device__ Q node_rows(const ElGeom<T> &g, const Line<T> &L, int k, int lo, int hi) {
+  const bool low = lo < g.nc;
+  return closure_row<NDIM, Q>(g.rows + (low ? lo : hi) * g.nspan, g.nspan, low, [&](int m) {
+    return line_at<NDIM, Q>(L, k, low ? m - lo : hi - 1 - m);
+  });
+}
+
+template <int NDIM, typename Q, typename T>
 __device__ Q half_rows(const ElGeom<T> &g, const Line<T> &L, int k, int lo, int hi) {
-  const T *rows = g.rows + g.nc * g.nspan;
-  Q acc((T)0);
-  if (lo < g.hc) {
-    for (int i = 0; i < g.hspan; ++i)
-      acc += rows[lo * g.hspan + i] * line_at<NDIM, Q>(L, k, i - lo);
-  } else {
-    for (int i = 0; i < g.hspan; ++i)
-      acc -= rows[hi * g.hspan + i] * line_at<NDIM, Q>(L, k, hi + 1 - i);
-  }
-  return acc;
+  const bool low = lo < g.hc;
+  return closure_row<NDIM, Q>(g.rows + g.nc * g.nspan + (low ? lo : hi) * g.hspan, g.hspan, low,
+                              [&](int m) {
+                                return line_at<NDIM, Q>(L, k, low ? m - lo : hi + 1 - m);
+                              });
 }
 
 // d/dx at node a of a half-point field (common.cuh:247-258)
