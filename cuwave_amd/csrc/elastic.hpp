@@ -643,17 +643,13 @@ el_prepare(ElGeom<T> g, const T *__restrict__ gamma, T rho, T *__restrict__ prep
 // fold, and in the adjoint pair (GRAD) the stiffness densities of u1 against
 // the forward field v1 (stiffness_density, elastic.cu:356-383)
 template <typename T, int NDIM, int R, int V, bool GRAD>
-__global__ void __launch_bounds__(kThreads)
-el_stress(ElGeom<T> g, ElLayer<T> P, const T *__restrict__ gamma, const T *__restrict__ prep,
-          const T *__restrict__ u1, T *__restrict__ sigma, T *__restrict__ g_normal,
-          T *__restrict__ g_shear, const T *__restrict__ v1) {
+__device__ __forceinline__ void
+stress_node(const ElGeom<T> &g, const ElLayer<T> &P, const T *__restrict__ gamma,
+            const T *__restrict__ prep, const T *__restrict__ u1, T *__restrict__ sigma,
+            T *__restrict__ g_normal, T *__restrict__ g_shear, const T *__restrict__ v1,
+            const int *A, int64_t idx, int lane0) {
   using Q = LanesOf<T, V>;
   constexpr int NV = nvoigt<NDIM>();
-  int A[3];
-  int64_t idx;
-  int lane0;
-  if (!node_of<NDIM, V>(g, A, &idx, &lane0))
-    return;
   const T *u = u1 + lane0;
   const T *shear = prep + NDIM * g.nodes;
   const T gn = gamma[idx];
@@ -685,18 +681,27 @@ el_stress(ElGeom<T> g, ElLayer<T> P, const T *__restrict__ gamma, const T *__res
     lanes_put(sigma + lane0, ((int64_t)w * g.nodes + idx) * g.lanes, sig[w]);
 }
 
-// fd_kernel (elastic.cu:798-853): u2 from u0, u1 and the stresses, the PML
-// fold, and in the adjoint pair the inertia density against v1; u2 may be u0
 template <typename T, int NDIM, int R, int V, bool GRAD>
 __global__ void __launch_bounds__(kThreads)
-el_update(ElGeom<T> g, ElLayer<T> P, const T *__restrict__ prep, const T *sigma, const T *u0,
-          const T *__restrict__ u1, T *u2, T *__restrict__ g_mass, const T *__restrict__ v1, T mf) {
-  using Q = LanesOf<T, V>;
+el_stress(ElGeom<T> g, ElLayer<T> P, const T *__restrict__ gamma, const T *__restrict__ prep,
+          const T *__restrict__ u1, T *__restrict__ sigma, T *__restrict__ g_normal,
+          T *__restrict__ g_shear, const T *__restrict__ v1) {
   int A[3];
   int64_t idx;
   int lane0;
-  if (!node_of<NDIM, V>(g, A, &idx, &lane0))
-    return;
+  if (node_of<NDIM, V>(g, A, &idx, &lane0))
+    stress_node<T, NDIM, R, V, GRAD>(g, P, gamma, prep, u1, sigma, g_normal, g_shear, v1, A, idx,
+                                     lane0);
+}
+
+// fd_kernel (elastic.cu:798-853): u2 from u0, u1 and the stresses, the PML
+// fold, and in the adjoint pair the inertia density against v1; u2 may be u0
+template <typename T, int NDIM, int R, int V, bool GRAD>
+__device__ __forceinline__ void
+update_node(const ElGeom<T> &g, const ElLayer<T> &P, const T *__restrict__ prep, const T *sigma,
+            const T *u0, const T *__restrict__ u1, T *u2, T *__restrict__ g_mass,
+            const T *__restrict__ v1, T mf, const int *A, int64_t idx, int lane0) {
+  using Q = LanesOf<T, V>;
 #pragma unroll
   for (int c = 0; c < NDIM; ++c) {
     if (A[c] > g.n[c] - 3)
@@ -723,6 +728,18 @@ el_update(ElGeom<T> g, ElLayer<T> P, const T *__restrict__ prep, const T *sigma,
       if (P.lo[e] + P.hi[e])
         settle_memory<NDIM, V>(g, P, sigma + lane0, idx, lane0, e, A);
   }
+}
+
+template <typename T, int NDIM, int R, int V, bool GRAD>
+__global__ void __launch_bounds__(kThreads)
+el_update(ElGeom<T> g, ElLayer<T> P, const T *__restrict__ prep, const T *sigma, const T *u0,
+          const T *__restrict__ u1, T *u2, T *__restrict__ g_mass, const T *__restrict__ v1, T mf) {
+  int A[3];
+  int64_t idx;
+  int lane0;
+  if (node_of<NDIM, V>(g, A, &idx, &lane0))
+    update_node<T, NDIM, R, V, GRAD>(g, P, prep, sigma, u0, u1, u2, g_mass, v1, mf, A, idx,
+                                     lane0);
 }
 
 // gradient_kernel (elastic_sensitivity.cu:115-158): both densities of the
