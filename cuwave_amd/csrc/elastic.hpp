@@ -20,6 +20,8 @@
 // the lanes (cw::shot_sum) into one per-node accumulator.
 #pragma once
 
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace cwe {
@@ -86,34 +88,46 @@ __device__ __forceinline__ int64_t slab_at(int a, int N, int lo, int hi, bool sl
   return slow ? (int64_t)row * plane + off : off * (int64_t)(lo + hi) + row;
 }
 
+// A thread's place in a component of a field or of the stresses, in bytes: 32
+// bits where a component can't pass 4 GiB (the stresses' element count is
+// under 2^31), so that a load takes a scalar base and this one register and a
+// tap's distance costs no vector instruction.
+template <int NDIM, typename T>
+using Place = std::conditional_t<NDIM == 3 || (NDIM == 2 && sizeof(T) == 4), uint32_t, uint64_t>;
+
+template <typename Q, typename T, typename Off>
+__device__ __forceinline__ Q at_bytes(const T *base, Off off) {
+  return *reinterpret_cast<const Q *>(reinterpret_cast<const char *>(base) + off);
+}
+template <typename Q, typename T, typename Off>
+__device__ __forceinline__ void put_bytes(T *base, Off off, const Q &v) {
+  *reinterpret_cast<Q *>(reinterpret_cast<char *>(base) + off) = v;
+}
+
 // A line of points a derivative reads: a field component (or a stress row)
 // along an axis, and optionally through the PML memory (the value coef *
 // (base + memory) of the reference's Memory accessor,
 // cuwave/kernels/common.cuh:421-437).
-template <typename T> struct Line {
-  const T *p;        // field or stresses, offset to the thread's first lane
-  int64_t idx;       // the node
-  int64_t nodes;     // nodes between components
-  int step;          // node stride of the axis
+template <typename T, typename Off> struct Line {
+  const T *p;        // field or stresses (the same for every thread)
+  Off off;           // the thread's place in a component
+  int64_t comp, step; // elements between components, and a step of the axis
   int lanes;
   int e;             // the axis
   bool stress;       // rows by stress_row(k, e)
   bool memory;
   const T *aux;      // offset to the thread's first lane
   const T *profile;
-  int64_t size, plane, off;
+  int64_t size, plane, slab;
   int row0, a, lo, hi, N;
   bool own_half, slow;
 };
 
-template <int NDIM, typename Q, typename T>
-__device__ __forceinline__ Q line_at(const Line<T> &L, int k, int j) {
-  const int row = L.stress ? stress_row<NDIM>(k, L.e) : k;
-  const Q base = lanes_at<Q>(L.p, ((int64_t)row * L.nodes + L.idx + (int64_t)j * L.step) * L.lanes);
-  if (!L.memory)
-    return base;
+// through the PML memory: the value `base` read j points away
+template <typename Q, typename T, typename Off>
+__device__ __forceinline__ Q through_memory(const Line<T, Off> &L, int k, int j, const Q &base) {
   const int at = L.a + j;
-  const int64_t i = slab_at(at, L.N, L.lo, L.hi, L.slow, L.plane, L.off);
+  const int64_t i = slab_at(at, L.N, L.lo, L.hi, L.slow, L.plane, L.slab);
   if (i < 0)
     return Q((T)0);
   const bool half = (k == L.e) == L.own_half;
@@ -121,13 +135,30 @@ __device__ __forceinline__ Q line_at(const Line<T> &L, int k, int j) {
   return coef * (base + lanes_at<Q>(L.aux, ((int64_t)(L.row0 + k) * L.size + i) * L.lanes));
 }
 
-template <typename T>
-__device__ __forceinline__ Line<T> field_line(const T *p, int64_t idx, const ElGeom<T> &g, int d) {
-  Line<T> L{};
+// the point j steps away, j the same for every thread ...
+template <int NDIM, typename Q, typename T, typename Off>
+__device__ __forceinline__ Q line_at(const Line<T, Off> &L, int k, int j) {
+  const int row = L.stress ? stress_row<NDIM>(k, L.e) : k;
+  const Q base = at_bytes<Q>(L.p + (row * L.comp + j * L.step), L.off);
+  return L.memory ? through_memory(L, k, j, base) : base;
+}
+// ... and j the thread's own
+template <int NDIM, typename Q, typename T, typename Off>
+__device__ __forceinline__ Q line_var(const Line<T, Off> &L, int k, int j) {
+  const int row = L.stress ? stress_row<NDIM>(k, L.e) : k;
+  const Q base = at_bytes<Q>(L.p + row * L.comp,
+                             L.off + (Off)j * (Off)(L.step * (int64_t)sizeof(T)));
+  return L.memory ? through_memory(L, k, j, base) : base;
+}
+
+template <typename T, typename Off>
+__device__ __forceinline__ Line<T, Off> field_line(const T *p, Off off, const ElGeom<T> &g,
+                                                   int d) {
+  Line<T, Off> L{};
   L.p = p;
-  L.idx = idx;
-  L.nodes = g.nodes;
-  L.step = g.s[d];
+  L.off = off;
+  L.comp = g.nodes * g.lanes;
+  L.step = (int64_t)g.s[d] * g.lanes;
   L.lanes = g.lanes;
   L.e = d;
   return L;
@@ -159,26 +190,26 @@ __device__ __forceinline__ Q closure_row(const T *row, int span, bool low, At at
   return acc;
 }
 
-template <int NDIM, typename Q, typename T>
-__device__ Q node_rows(const ElGeom<T> &g, const Line<T> &L, int k, int lo, int hi) {
+template <int NDIM, typename Q, typename T, typename Off>
+__device__ Q node_rows(const ElGeom<T> &g, const Line<T, Off> &L, int k, int lo, int hi) {
   const bool low = lo < g.nc;
   return closure_row<NDIM, Q>(g.rows + (low ? lo : hi) * g.nspan, g.nspan, low, [&](int m) {
-    return line_at<NDIM, Q>(L, k, low ? m - lo : hi - 1 - m);
+    return line_var<NDIM, Q>(L, k, low ? m - lo : hi - 1 - m);
   });
 }
 
-template <int NDIM, typename Q, typename T>
-__device__ Q half_rows(const ElGeom<T> &g, const Line<T> &L, int k, int lo, int hi) {
+template <int NDIM, typename Q, typename T, typename Off>
+__device__ Q half_rows(const ElGeom<T> &g, const Line<T, Off> &L, int k, int lo, int hi) {
   const bool low = lo < g.hc;
   return closure_row<NDIM, Q>(g.rows + g.nc * g.nspan + (low ? lo : hi) * g.hspan, g.hspan, low,
                               [&](int m) {
-                                return line_at<NDIM, Q>(L, k, low ? m - lo : hi + 1 - m);
+                                return line_var<NDIM, Q>(L, k, low ? m - lo : hi + 1 - m);
                               });
 }
 
 // d/dx at node a of a half-point field (common.cuh:247-258)
-template <int NDIM, int R, typename Q, typename T>
-__device__ __forceinline__ Q node_derivative(const ElGeom<T> &g, const Line<T> &L, int k, int a,
+template <int NDIM, int R, typename Q, typename T, typename Off>
+__device__ __forceinline__ Q node_derivative(const ElGeom<T> &g, const Line<T, Off> &L, int k, int a,
                                              int N) {
   const int lo = a - 1, hi = N - 2 - a;
   if (lo < g.nc || hi < g.nc)
@@ -191,8 +222,8 @@ __device__ __forceinline__ Q node_derivative(const ElGeom<T> &g, const Line<T> &
 }
 
 // d/dx at half point a of a nodal field (common.cuh:261-271)
-template <int NDIM, int R, typename Q, typename T>
-__device__ __forceinline__ Q half_derivative(const ElGeom<T> &g, const Line<T> &L, int k, int a,
+template <int NDIM, int R, typename Q, typename T, typename Off>
+__device__ __forceinline__ Q half_derivative(const ElGeom<T> &g, const Line<T, Off> &L, int k, int a,
                                              int N) {
   const int lo = a - 1, hi = N - 3 - a;
   if (lo < g.hc || hi < g.hc)
@@ -205,8 +236,8 @@ __device__ __forceinline__ Q half_derivative(const ElGeom<T> &g, const Line<T> &
 }
 
 // the divergence of a nodal stress at half point a (common.cuh:276-288)
-template <int NDIM, int R, typename Q, typename T>
-__device__ __forceinline__ Q node_divergence(const ElGeom<T> &g, const Line<T> &L, int k, int a,
+template <int NDIM, int R, typename Q, typename T, typename Off>
+__device__ __forceinline__ Q node_divergence(const ElGeom<T> &g, const Line<T, Off> &L, int k, int a,
                                              int N) {
   const int lo = a - 1, hi = N - 3 - a;
   if (lo < g.hc || hi < g.hc)
@@ -221,8 +252,8 @@ __device__ __forceinline__ Q node_divergence(const ElGeom<T> &g, const Line<T> &
 }
 
 // the divergence of a half-point stress at node a (common.cuh:292-304)
-template <int NDIM, int R, typename Q, typename T>
-__device__ __forceinline__ Q half_divergence(const ElGeom<T> &g, const Line<T> &L, int k, int a,
+template <int NDIM, int R, typename Q, typename T, typename Off>
+__device__ __forceinline__ Q half_divergence(const ElGeom<T> &g, const Line<T, Off> &L, int k, int a,
                                              int N) {
   const int lo = a - 1, hi = N - 2 - a;
   if (lo < g.nc || hi < g.nc)
@@ -252,9 +283,25 @@ __device__ __forceinline__ int zeroed_axes(const ElGeom<T> &g, const int *A) {
   return zeroed;
 }
 
-// the normal strains of u at node idx, zero on a traction wall (elastic.cu:121-141)
-template <int NDIM, int R, typename Q, typename T>
-__device__ __forceinline__ int normal_strains(const ElGeom<T> &g, const T *u, int64_t idx,
+// the derivative of u_k along axis e at its strain point, zero where there is
+// none (a traction wall's normal strain, a shear point past the last);
+// strain_term (elastic.cu:417-431) is f[e] times it
+template <int NDIM, int R, typename Q, typename T, typename L>
+__device__ __forceinline__ Q strain_derivative(const ElGeom<T> &g, const L &line, int k, int e,
+                                               const int *A) {
+  if (k == e) {
+    if (traction_zero<NDIM>(g, A, e))
+      return Q((T)0);
+    return node_derivative<NDIM, R, Q>(g, line, e, A[e], g.n[e]);
+  }
+  if (A[k] > g.n[k] - 3 || A[e] > g.n[e] - 3)
+    return Q((T)0);
+  return half_derivative<NDIM, R, Q>(g, line, k, A[e], g.n[e]);
+}
+
+// the normal strains of u at a node, zero on a traction wall (elastic.cu:121-141)
+template <int NDIM, int R, typename Q, typename T, typename Off>
+__device__ __forceinline__ int normal_strains(const ElGeom<T> &g, const T *u, Off off,
                                               const int *A, Q *eps) {
   int zeroed = 0;
 #pragma unroll
@@ -263,8 +310,7 @@ __device__ __forceinline__ int normal_strains(const ElGeom<T> &g, const T *u, in
       eps[d] = Q((T)0);
       zeroed |= 1 << d;
     } else {
-      const Line<T> L = field_line(u, idx, g, d);
-      eps[d] = g.f[d] * node_derivative<NDIM, R, Q>(g, L, d, A[d], g.n[d]);
+      eps[d] = g.f[d] * node_derivative<NDIM, R, Q>(g, field_line(u, off, g, d), d, A[d], g.n[d]);
     }
   }
   return zeroed;
@@ -282,13 +328,11 @@ __device__ __forceinline__ T condensed_lame(const ElGeom<T> &g, int zeroed) {
 }
 
 // the engineering shear strain (k, l) at its point (elastic.cu:159-170)
-template <int NDIM, int R, typename Q, typename T>
-__device__ __forceinline__ Q shear_strain(const ElGeom<T> &g, const T *u, int64_t idx, int k,
-                                          int l, const int *A) {
-  const Line<T> Lk = field_line(u, idx, g, k);
-  const Line<T> Ll = field_line(u, idx, g, l);
-  const Q dk = half_derivative<NDIM, R, Q>(g, Lk, l, A[k], g.n[k]);
-  const Q dl = half_derivative<NDIM, R, Q>(g, Ll, k, A[l], g.n[l]);
+template <int NDIM, int R, typename Q, typename T, typename Off>
+__device__ __forceinline__ Q shear_strain(const ElGeom<T> &g, const T *u, Off off, int k, int l,
+                                          const int *A) {
+  const Q dk = half_derivative<NDIM, R, Q>(g, field_line(u, off, g, k), l, A[k], g.n[k]);
+  const Q dl = half_derivative<NDIM, R, Q>(g, field_line(u, off, g, l), k, A[l], g.n[l]);
   return fmat(g.f[k], dk, g.f[l] * dl);
 }
 
@@ -297,18 +341,20 @@ __device__ __forceinline__ bool shear_point(const ElGeom<T> &g, int k, int l, co
   return A[k] <= g.n[k] - 3 && A[l] <= g.n[l] - 3;
 }
 
-// every strain of u at node idx (elastic.cu:216-233)
-template <int NDIM, int R, typename Q, typename T>
-__device__ __forceinline__ int strain_point(const ElGeom<T> &g, const T *u, int64_t idx,
-                                            const int *A, Q *eps) {
-  const int zeroed = normal_strains<NDIM, R>(g, u, idx, A, eps);
+// every strain of u from its derivatives D[k][e] = d u_k / d x_e
+// (elastic.cu:216-233)
+template <int NDIM, typename Q, typename T>
+__device__ __forceinline__ void strains_of(const ElGeom<T> &g, const Q (*D)[NDIM], const int *A,
+                                           Q *eps) {
+#pragma unroll
+  for (int d = 0; d < NDIM; ++d)
+    eps[d] = traction_zero<NDIM>(g, A, d) ? Q((T)0) : g.f[d] * D[d][d];
 #pragma unroll
   for (int k = 0; k < NDIM - 1; ++k)
 #pragma unroll
     for (int l = k + 1; l < NDIM; ++l)
       eps[stress_row<NDIM>(k, l)] =
-          shear_point(g, k, l, A) ? shear_strain<NDIM, R, Q>(g, u, idx, k, l, A) : Q((T)0);
-  return zeroed;
+          shear_point(g, k, l, A) ? fmat(g.f[k], D[l][k], g.f[l] * D[k][l]) : Q((T)0);
 }
 
 // the stresses of the strains (elastic.cu:236-263); the shear gamma of the
@@ -334,22 +380,14 @@ __device__ __forceinline__ void stress_of(const ElGeom<T> &g, const Q *eps, int 
     }
 }
 
-// the force on component c at its point: the divergence of the stresses
-// (elastic.cu:281-303)
-template <int NDIM, int R, typename Q, typename T>
-__device__ __forceinline__ Q nodal_force(const ElGeom<T> &g, const T *sigma, int64_t idx, int c,
-                                         const int *A) {
-  const Line<T> Lc = field_line(sigma, idx, g, c);
-  Q force = g.f[c] * node_divergence<NDIM, R, Q>(g, Lc, c, A[c], g.n[c]);
-#pragma unroll
-  for (int l = 0; l < NDIM; ++l) {
-    if (l == c)
-      continue;
-    const Line<T> Lv = field_line(sigma, idx, g, l);
-    force = fmat(g.f[l], half_divergence<NDIM, R, Q>(g, Lv, stress_row<NDIM>(c, l), A[l], g.n[l]),
-                 force);
-  }
-  return force;
+// the divergence of the stresses of component c along axis e at its point;
+// divergence_term (elastic.cu:434-442) is f[e] times it
+template <int NDIM, int R, typename Q, typename T, typename L>
+__device__ __forceinline__ Q stress_divergence(const ElGeom<T> &g, const L &line, int c, int e,
+                                               int row, const int *A) {
+  if (c == e)
+    return node_divergence<NDIM, R, Q>(g, line, c, A[c], g.n[c]);
+  return half_divergence<NDIM, R, Q>(g, line, row, A[e], g.n[e]);
 }
 
 // the normal-strain energy form of two strain sets (elastic.cu:339-351)
@@ -388,29 +426,6 @@ __device__ __forceinline__ void slab_geometry(const ElGeom<T> &g, int e, int lo,
   *off = o;
 }
 
-// d u_k / d x_e at the strain point (k, e) (elastic.cu:417-431)
-template <int NDIM, int R, typename Q, typename T>
-__device__ __forceinline__ Q strain_term(const ElGeom<T> &g, const Line<T> &L, int k, int e,
-                                         const int *A) {
-  if (k == e) {
-    if (traction_zero<NDIM>(g, A, e))
-      return Q((T)0);
-    return g.f[e] * node_derivative<NDIM, R, Q>(g, L, e, A[e], g.n[e]);
-  }
-  if (A[k] > g.n[k] - 3 || A[e] > g.n[e] - 3)
-    return Q((T)0);
-  return g.f[e] * half_derivative<NDIM, R, Q>(g, L, k, A[e], g.n[e]);
-}
-
-// elastic.cu:434-442
-template <int NDIM, int R, typename Q, typename T>
-__device__ __forceinline__ Q divergence_term(const ElGeom<T> &g, const Line<T> &L, int c, int e,
-                                             const int *A, T fe) {
-  if (c == e)
-    return fe * node_divergence<NDIM, R, Q>(g, L, c, A[c], g.n[c]);
-  return fe * half_divergence<NDIM, R, Q>(g, L, c, A[e], g.n[e]);
-}
-
 // the stresses of the memory strains t of axis e (elastic.cu:445-467)
 template <int NDIM, typename Q, typename T>
 __device__ __forceinline__ void add_stress(const ElGeom<T> &g, Q *sig, T gn, const T *shear,
@@ -432,11 +447,12 @@ __device__ __forceinline__ void add_stress(const ElGeom<T> &g, Q *sig, T gn, con
     }
 }
 
-// the strain memory of axis e (elastic.cu:486-528)
-template <int NDIM, int R, int V, typename T>
+// the strain memory of axis e (elastic.cu:486-528), D[k] = d u_k / d x_e
+template <int NDIM, int R, int V, typename T, typename Off>
 __device__ __forceinline__ void stress_memory(const ElGeom<T> &g, const ElLayer<T> &P, int e,
-                                              const T *u, T gn, const T *shear, int64_t idx,
-                                              int lane0, const int *A, LanesOf<T, V> *sig) {
+                                              const T *u, const LanesOf<T, V> (*D)[NDIM], T gn,
+                                              const T *shear, int64_t idx, Off place, int lane0,
+                                              const int *A, LanesOf<T, V> *sig) {
   using Q = LanesOf<T, V>;
   const int a = A[e], lo = P.lo[e], hi = P.hi[e];
   if (!in_slab<NDIM>(g, a, e, lo, hi, P.phase ? R : 0))
@@ -447,13 +463,13 @@ __device__ __forceinline__ void stress_memory(const ElGeom<T> &g, const ElLayer<
   const T *prof = P.profile[e];
   Q q[3];
   if (P.phase) {
-    Line<T> h = field_line(u, idx, g, e);
+    Line<T, Off> h = field_line(u, place, g, e);
     h.memory = true;
     h.aux = P.aux[e] + lane0;
     h.profile = prof;
     h.size = size;
     h.plane = plane;
-    h.off = off;
+    h.slab = off;
     h.row0 = NDIM;
     h.a = a;
     h.lo = lo;
@@ -463,26 +479,27 @@ __device__ __forceinline__ void stress_memory(const ElGeom<T> &g, const ElLayer<
     h.slow = e < NDIM - 1;
 #pragma unroll
     for (int k = 0; k < NDIM; ++k)
-      q[k] = strain_term<NDIM, R, Q>(g, h, k, e, A);
+      q[k] = g.f[e] * strain_derivative<NDIM, R, Q>(g, h, k, e, A);
   } else {
-    const Line<T> f = field_line(u, idx, g, e);
     const int64_t t = slab_at(a, N, lo, hi, e < NDIM - 1, plane, off);
     T *aux = P.aux[e] + lane0;
 #pragma unroll
     for (int k = 0; k < NDIM; ++k) {
       const int at = (k == e ? 0 : 2 * N) + a;
       const int64_t m = ((int64_t)k * size + t) * g.lanes;
-      q[k] = prof[N + at] * lanes_at<Q>(aux, m) + prof[at] * strain_term<NDIM, R, Q>(g, f, k, e, A);
+      q[k] = prof[N + at] * lanes_at<Q>(aux, m) + prof[at] * (g.f[e] * D[k][e]);
       lanes_put(aux, m, q[k]);
     }
   }
   add_stress<NDIM>(g, sig, gn, shear, idx, e, q, A);
 }
 
-// the divergence memory of component c along axis e (elastic.cu:532-573)
-template <int NDIM, int R, int V, typename T>
+// the divergence memory of component c along axis e (elastic.cu:532-573),
+// `term` the divergence term itself (the forward's)
+template <int NDIM, int R, int V, typename T, typename Off>
 __device__ __forceinline__ LanesOf<T, V> force_memory(const ElGeom<T> &g, const ElLayer<T> &P,
-                                                      const T *sigma, const T *u1, int64_t idx,
+                                                      const T *sigma, const LanesOf<T, V> &term,
+                                                      const LanesOf<T, V> &u1, Off place,
                                                       int lane0, int c, int e, const int *A) {
   using Q = LanesOf<T, V>;
   const int a = A[e], lo = P.lo[e], hi = P.hi[e];
@@ -497,15 +514,15 @@ __device__ __forceinline__ LanesOf<T, V> force_memory(const ElGeom<T> &g, const 
   const int at = (c == e ? 2 * N : 0) + a;
   T *aux = P.aux[e] + lane0;
   const int64_t z = ((int64_t)(NDIM + c) * size + t) * g.lanes;
-  Line<T> k = field_line(sigma, idx, g, e);
-  k.stress = true;
   if (P.phase) {
+    Line<T, Off> k = field_line(sigma, place, g, e);
+    k.stress = true;
     k.memory = true;
     k.aux = aux;
     k.profile = prof;
     k.size = size;
     k.plane = plane;
-    k.off = off;
+    k.slab = off;
     k.row0 = P.phase == 1 ? 0 : 2 * NDIM;
     k.a = a;
     k.lo = lo;
@@ -513,15 +530,12 @@ __device__ __forceinline__ LanesOf<T, V> force_memory(const ElGeom<T> &g, const 
     k.N = N;
     k.own_half = false;
     k.slow = slow;
-    const Q term = divergence_term<NDIM, R, Q>(g, k, c, e, A, g.f[e]);
-    if (t >= 0) {
-      const Q u = lanes_at<Q>(u1, ((int64_t)c * g.nodes + idx) * g.lanes);
-      lanes_put(aux, z, prof[N + at] * (lanes_at<Q>(aux, z) + u));
-    }
-    return term;
+    const Q back = g.f[e] * stress_divergence<NDIM, R, Q>(g, k, c, e, c, A);
+    if (t >= 0)
+      lanes_put(aux, z, prof[N + at] * (lanes_at<Q>(aux, z) + u1));
+    return back;
   }
-  const Q next = prof[N + at] * lanes_at<Q>(aux, z) +
-                 prof[at] * divergence_term<NDIM, R, Q>(g, k, c, e, A, g.f[e]);
+  const Q next = prof[N + at] * lanes_at<Q>(aux, z) + prof[at] * term;
   lanes_put(aux, z, next);
   return next;
 }
@@ -559,17 +573,18 @@ __device__ __forceinline__ void settle_memory(const ElGeom<T> &g, const ElLayer<
 // XCD's L2 by the blocks before it.
 template <int NDIM, int V, typename T>
 __device__ __forceinline__ bool node_of(const ElGeom<T> &g, int *A, int64_t *idx, int *lane0) {
-  const int per = g.lanes / V;
-  const int64_t t = (int64_t)cw::xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  const int64_t i = t / per;
-  if (i >= g.interior)
+  // threads are under 2^31: 32-bit arithmetic, the lanes a power of two
+  const int per = g.lanes / V, shift = __builtin_ctz(per);
+  const uint32_t t = (uint32_t)cw::xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const uint32_t i = t >> shift;
+  if (i >= (uint32_t)g.interior)
     return false;
-  *lane0 = (int)(t % per) * V;
-  int64_t rest = i;
+  *lane0 = (int)(t & (per - 1)) * V;
+  uint32_t rest = i;
 #pragma unroll
   for (int d = NDIM - 1; d >= 0; --d) {
-    const int w = g.n[d] - 2;
-    A[d] = 1 + (int)(rest % w);
+    const uint32_t w = g.n[d] - 2;
+    A[d] = 1 + (int)(d ? rest % w : rest);
     rest /= w;
   }
   int64_t at = 0;
@@ -578,6 +593,13 @@ __device__ __forceinline__ bool node_of(const ElGeom<T> &g, int *A, int64_t *idx
     at += (int64_t)A[d] * g.s[d];
   *idx = at;
   return true;
+}
+
+// the thread's place in a component
+template <int NDIM, typename T>
+__device__ __forceinline__ Place<NDIM, T> place_of(const ElGeom<T> &g, int64_t idx, int lane0) {
+  return ((Place<NDIM, T>)idx * (Place<NDIM, T>)g.lanes + (Place<NDIM, T>)lane0) *
+         (Place<NDIM, T>)sizeof(T);
 }
 
 // the per-node sum over the shots of a density, taken off accumulator `acc`
@@ -650,15 +672,22 @@ stress_node(const ElGeom<T> &g, const ElLayer<T> &P, const T *__restrict__ gamma
             const int *A, int64_t idx, int lane0) {
   using Q = LanesOf<T, V>;
   constexpr int NV = nvoigt<NDIM>();
-  const T *u = u1 + lane0;
+  const auto place = place_of<NDIM>(g, idx, lane0);
   const T *shear = prep + NDIM * g.nodes;
   const T gn = gamma[idx];
+  // each derivative once: the strains and the forward's memory both read it
+  Q D[NDIM][NDIM];
+#pragma unroll
+  for (int e = 0; e < NDIM; ++e)
+#pragma unroll
+    for (int k = 0; k < NDIM; ++k)
+      D[k][e] = strain_derivative<NDIM, R, Q>(g, field_line(u1, place, g, e), k, e, A);
   Q eps[NV], sig[NV];
-  const int zeroed = strain_point<NDIM, R, Q>(g, u, idx, A, eps);
+  const int zeroed = zeroed_axes<NDIM>(g, A);
+  strains_of<NDIM>(g, D, A, eps);
   if constexpr (GRAD) {
-    const T *v = v1 + lane0;
     Q eu[NDIM];
-    const int z2 = normal_strains<NDIM, R, Q>(g, v, idx, A, eu);
+    const int z2 = normal_strains<NDIM, R, Q>(g, v1, place, A, eu);
     take_off<T, V>(g_normal, idx, normal_form<NDIM, Q>(g, eps, eu, z2), g.lanes, lane0);
 #pragma unroll
     for (int k = 0; k < NDIM - 1; ++k)
@@ -667,7 +696,7 @@ stress_node(const ElGeom<T> &g, const ElLayer<T> &P, const T *__restrict__ gamma
         if (!shear_point(g, k, l, A))
           continue;
         const int w = stress_row<NDIM>(k, l);
-        const Q d = g.mu * eps[w] * shear_strain<NDIM, R, Q>(g, v, idx, k, l, A);
+        const Q d = g.mu * eps[w] * shear_strain<NDIM, R, Q>(g, v1, place, k, l, A);
         take_off<T, V>(g_shear, (int64_t)(w - NDIM) * g.nodes + idx, d, g.lanes, lane0);
       }
   }
@@ -675,10 +704,10 @@ stress_node(const ElGeom<T> &g, const ElLayer<T> &P, const T *__restrict__ gamma
 #pragma unroll
   for (int e = 0; e < NDIM; ++e)
     if (P.lo[e] + P.hi[e])
-      stress_memory<NDIM, R, V>(g, P, e, u, gn, shear, idx, lane0, A, sig);
+      stress_memory<NDIM, R, V>(g, P, e, u1, D, gn, shear, idx, place, lane0, A, sig);
 #pragma unroll
   for (int w = 0; w < NV; ++w)
-    lanes_put(sigma + lane0, ((int64_t)w * g.nodes + idx) * g.lanes, sig[w]);
+    put_bytes(sigma + w * (g.nodes * g.lanes), place, sig[w]);
 }
 
 template <typename T, int NDIM, int R, int V, bool GRAD>
@@ -702,25 +731,38 @@ update_node(const ElGeom<T> &g, const ElLayer<T> &P, const T *__restrict__ prep,
             const T *u0, const T *__restrict__ u1, T *u2, T *__restrict__ g_mass,
             const T *__restrict__ v1, T mf, const int *A, int64_t idx, int lane0) {
   using Q = LanesOf<T, V>;
+  const auto place = place_of<NDIM>(g, idx, lane0);
 #pragma unroll
   for (int c = 0; c < NDIM; ++c) {
     if (A[c] > g.n[c] - 3)
       continue;
-    const Q force = nodal_force<NDIM, R, Q>(g, sigma + lane0, idx, c, A);
+    // the force on component c at its point (nodal_force, elastic.cu:281-303),
+    // each divergence once: the forward's memory reads it too
+    Q D[NDIM];
+#pragma unroll
+    for (int e = 0; e < NDIM; ++e)
+      D[e] = stress_divergence<NDIM, R, Q>(g, field_line(sigma, place, g, e), c, e,
+                                           stress_row<NDIM>(c, e), A);
+    Q force = g.f[c] * D[c];
+#pragma unroll
+    for (int l = 0; l < NDIM; ++l)
+      if (l != c)
+        force = fmat(g.f[l], D[l], force);
     const int64_t n = (int64_t)c * g.nodes + idx;
-    const int64_t at = n * g.lanes + lane0;
+    const int64_t comp = c * (g.nodes * g.lanes);
     const T mi = prep[n];
-    const Q w0 = lanes_at<Q>(u0, at), w1 = lanes_at<Q>(u1, at);
+    const Q w0 = at_bytes<Q>(u0 + comp, place), w1 = at_bytes<Q>(u1 + comp, place);
     Q next = -w0 + (T)2.f * w1 + mi * force;
 #pragma unroll
     for (int e = 0; e < NDIM; ++e)
       if (P.lo[e] + P.hi[e])
-        next += mi * force_memory<NDIM, R, V>(g, P, sigma + lane0, u1 + lane0, idx, lane0, c, e, A);
+        next += mi * force_memory<NDIM, R, V>(g, P, sigma, Q(g.f[e] * D[e]), w1, place, lane0, c,
+                                              e, A);
     if constexpr (GRAD) {
-      const Q v = lanes_at<Q>(v1, at);
+      const Q v = at_bytes<Q>(v1 + comp, place);
       take_off<T, V>(g_mass, n, mf * v * (next - (T)2.f * w1 + w0), g.lanes, lane0);
     }
-    lanes_put(u2, at, next);
+    put_bytes(u2 + comp, place, next);
   }
   if (P.phase) {
 #pragma unroll
@@ -765,9 +807,10 @@ el_gradient(ElGeom<T> g, T *__restrict__ g_mass, T *__restrict__ g_normal,
     const Q w0 = lanes_at<Q>(u0, at), w1 = lanes_at<Q>(u1, at), w2 = lanes_at<Q>(u2, at);
     take_off<T, V>(g_mass, n, mf * l * (w2 - (T)2.f * w1 + w0), g.lanes, lane0);
   }
+  const auto place = place_of<NDIM>(g, idx, lane0);
   Q eu[NDIM], el[NDIM];
-  const int zeroed = normal_strains<NDIM, R, Q>(g, u1 + lane0, idx, A, eu);
-  normal_strains<NDIM, R, Q>(g, l1 + lane0, idx, A, el);
+  const int zeroed = normal_strains<NDIM, R, Q>(g, u1, place, A, eu);
+  normal_strains<NDIM, R, Q>(g, l1, place, A, el);
   take_off<T, V>(g_normal, idx, normal_form<NDIM, Q>(g, el, eu, zeroed), g.lanes, lane0);
 #pragma unroll
   for (int k = 0; k < NDIM - 1; ++k)
@@ -776,8 +819,8 @@ el_gradient(ElGeom<T> g, T *__restrict__ g_mass, T *__restrict__ g_normal,
       if (!shear_point(g, k, l, A))
         continue;
       const int w = stress_row<NDIM>(k, l);
-      const Q d = g.mu * shear_strain<NDIM, R, Q>(g, l1 + lane0, idx, k, l, A) *
-                  shear_strain<NDIM, R, Q>(g, u1 + lane0, idx, k, l, A);
+      const Q d = g.mu * shear_strain<NDIM, R, Q>(g, l1, place, k, l, A) *
+                  shear_strain<NDIM, R, Q>(g, u1, place, k, l, A);
       take_off<T, V>(g_shear, (int64_t)(w - NDIM) * g.nodes + idx, d, g.lanes, lane0);
     }
 }

@@ -70,26 +70,15 @@ __device__ __forceinline__ void frame_node(const ElGeom<T> &g, const ElFrame &f,
 
 // the frame node and first lane of thread `t`, false past the last
 template <int V, typename T>
-__device__ __forceinline__ bool frame_thread(const ElGeom<T> &g, const ElFrame &f, int64_t t,
+__device__ __forceinline__ bool frame_thread(const ElGeom<T> &g, const ElFrame &f, uint32_t t,
                                              int *A, int64_t *idx, int *lane0) {
-  const int per = g.lanes / V;
-  const int64_t i = t / per;
+  const int per = g.lanes / V, i = (int)(t >> __builtin_ctz(per));
   if (i >= f.nodes)
     return false;
-  *lane0 = (int)(t % per) * V;
-  frame_node(g, f, (int)i, A);
+  *lane0 = (int)(t & (per - 1)) * V;
+  frame_node(g, f, i, A);
   *idx = (int64_t)A[0] * g.s[0] + A[1];
   return true;
-}
-
-// the V lanes `off` bytes into an array (a scalar base, one 32-bit offset)
-template <typename Q, typename T>
-__device__ __forceinline__ Q at_bytes(const T *base, uint32_t off) {
-  return *reinterpret_cast<const Q *>(reinterpret_cast<const char *>(base) + off);
-}
-template <typename Q, typename T>
-__device__ __forceinline__ void put_bytes(T *base, uint32_t off, const Q &v) {
-  *reinterpret_cast<Q *>(reinterpret_cast<char *>(base) + off) = v;
 }
 
 // LDS of a core block of NT threads: two buffers of two displacement rows
@@ -273,7 +262,7 @@ el_core(ElGeom<T> g, T fu0, T fu1, ElBox box, ElFrame frame, ElLayer<T> P,
   int64_t idx;
   int lane0;
   const int b = cw::xcd_tile((int)blockIdx.x - blocks, (int)gridDim.x - blocks);
-  if (frame_thread<V>(g, frame, (int64_t)b * NT + threadIdx.x, A, &idx, &lane0))
+  if (frame_thread<V>(g, frame, (uint32_t)b * NT + threadIdx.x, A, &idx, &lane0))
     stress_node<T, 2, R, V, false>(g, P, gamma, prep, u1, sigma, (T *)nullptr, (T *)nullptr,
                                    (const T *)nullptr, A, idx, lane0);
 }
@@ -287,7 +276,7 @@ el_frame_update(ElGeom<T> g, ElFrame frame, ElLayer<T> P, const T *__restrict__ 
   int64_t idx;
   int lane0;
   if (frame_thread<V>(g, frame,
-                      (int64_t)cw::xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x, A,
+                      (uint32_t)cw::xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x, A,
                       &idx, &lane0))
     update_node<T, 2, R, V, false>(g, P, prep, sigma, u0, u1, u2, (T *)nullptr,
                                    (const T *)nullptr, (T)0, A, idx, lane0);
