@@ -86,10 +86,10 @@ class Traces(torch.autograd.Function):
         except StopIteration:
             pass
         if g_stiff is None:
-            grads = _zero_outside(_finalize(sim, {"g": g_mass}, run.dev), ~run.valid, run.dev)
+            grads = _zero_outside(_finalize(sim, {"g": g_mass}, run.dev), ~run.inside, run.dev)
             return grads["g"].to(device, dtype), None, None, None, None
         grads = _finalize(sim, {"mass": g_mass, "stiff": g_stiff}, run.dev)
-        grads = _zero_outside(grads, ~run.valid, run.dev)
+        grads = _zero_outside(grads, ~run.inside, run.dev)
         gi = _chain(sim, ind, grads["mass"], grads["stiff"])
         return gi.to(device, dtype), None, None, None, None
 

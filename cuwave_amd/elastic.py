@@ -22,10 +22,10 @@ innermost in every per-shot array as in the pressure path:
   kernel (cuwave/elastic.py:731-762);
 - `misfit_gradient`: every shot of a batch in one sweep, summed.
 
-The host-side parametrization (point inertia, excitation weights, the norms,
-the chain rule of `finalize_gradients`) runs in numpy in the simulation's
-precision, as the reference computes it, so what the kernels read is the
-reference's to the bit.
+The host-side parametrization (point inertia, excitation weights, the norms)
+runs in numpy in the simulation's precision, as the reference computes it, so
+what the kernels read is the reference's to the bit; the chain rule
+(`finalize_gradients`) runs the same operations where the densities are.
 """
 
 from __future__ import annotations
@@ -476,61 +476,72 @@ class ElasticEngine(ShotFields):
         _abi.call("cw_elastic_gradient", ctypes.byref(a), _abi.stream())
 
 # ------------------------------------------------------------------ gradients
-def _point_average_adjoint(sim: ElasticWave, density: np.ndarray, c: int) -> np.ndarray:
+# The chain rule runs where the densities are, in the simulation's precision and the
+# reference's order, an operation a pass.
+def _point_average_adjoint(density: torch.Tensor, c: int) -> torch.Tensor:
     """The transpose of the mean over the two nodes component c sits between."""
-    out = 0.5 * density
-    to = [slice(None)] * sim.ndim
-    fro = [slice(None)] * sim.ndim
-    to[c], fro[c] = slice(1, None), slice(0, -1)
-    out[tuple(to)] += 0.5 * density[tuple(fro)]
+    half = 0.5 * density
+    out = half.clone()
+    n = out.shape[c]
+    out.narrow(c, 1, n - 1).add_(half.narrow(c, 0, n - 1))
     return out
 
 
-def _pair_average(sim: ElasticWave, field: np.ndarray, axes) -> np.ndarray:
-    """The harmonic mean of `field` over the four nodes around a pair point of `axes`."""
-    out = np.zeros(sim.Nx_padded, dtype=sim.np_dtype)
-    safe = np.maximum(field, np.finfo(sim.np_dtype).tiny)
-    inner = tuple(slice(0, n - 1) if d in axes else slice(0, n) for d, n in enumerate(sim.Nx))
+def _pair_corners(sim: ElasticWave, axes):
+    """Per corner of a pair point of `axes`, the slices of its node over the points."""
     for bits in itertools.product((0, 1), repeat=2):
-        shifted = tuple(slice(bits[axes.index(d)], n - 1 + bits[axes.index(d)])
-                        if d in axes else slice(0, n) for d, n in enumerate(sim.Nx))
-        out[inner] += 1.0 / safe[shifted]
+        yield tuple(slice(bits[axes.index(d)], n - 1 + bits[axes.index(d)]) if d in axes
+                    else slice(0, n) for d, n in enumerate(sim.Nx))
+
+
+def _pair_average(sim: ElasticWave, field: torch.Tensor, axes) -> torch.Tensor:
+    """The harmonic mean of `field` over the four nodes around a pair point of `axes`."""
+    out = torch.zeros_like(field)
+    inverse = 1.0 / torch.clamp(field, min=float(np.finfo(sim.np_dtype).tiny))
+    inner = tuple(slice(0, n - 1) if d in axes else slice(0, n) for d, n in enumerate(sim.Nx))
+    for corner in _pair_corners(sim, axes):
+        out[inner] += inverse[corner]
     out[inner] = 4.0 / out[inner]
     return out
 
 
-def _pair_average_adjoint(sim: ElasticWave, density, field, axes) -> np.ndarray:
+def _pair_average_adjoint(sim: ElasticWave, density: torch.Tensor, field: torch.Tensor,
+                          axes) -> torch.Tensor:
     """The transpose of the harmonic pair mean's derivative, scattered onto the four nodes."""
-    safe = np.maximum(field, np.finfo(sim.np_dtype).tiny)
+    safe = torch.clamp(field, min=float(np.finfo(sim.np_dtype).tiny))
+    square = safe * safe
     mean = _pair_average(sim, field, axes)
     scattered = density * mean * mean * 0.25
-    out = np.zeros(sim.Nx_padded, dtype=sim.np_dtype)
+    out = torch.zeros_like(field)
     for bits in itertools.product((0, 1), repeat=2):
         to = [slice(None)] * sim.ndim
         fro = [slice(None)] * sim.ndim
         for d, b in zip(axes, bits):
-            to[d], fro[d] = slice(b, None), slice(0, -b if b else None)
-        out[tuple(to)] += scattered[tuple(fro)] / safe[tuple(to)] ** 2
+            n = field.shape[d]
+            to[d], fro[d] = slice(b, n), slice(0, n - b)
+        out[tuple(to)] += scattered[tuple(fro)] / square[tuple(to)]
     return out
 
 
 def finalize_gradients(sim: ElasticWave, grads: dict, gamma: np.ndarray) -> dict:
     """The point densities chained through the averages onto the nodal design field
-    (cuwave/elastic.py:716-729, cuwave/wave.py:386-475), on the host."""
-    host = {k: v.cpu().numpy() for k, v in grads.items()}
-    g_mass = np.zeros(sim.Nx_padded, dtype=sim.np_dtype)
+    (cuwave/elastic.py:716-729, cuwave/wave.py:386-475), on the densities' device."""
+    device = grads["normal"].device
+
+    def here(a):
+        return torch.as_tensor(a, device=device)
+
+    gamma = here(gamma)
+    g_mass = torch.zeros_like(grads["normal"])
+    density = float(sim.np_dtype(sim.density))
     for c in range(sim.ncomp):
-        density = host["mass"][c] * sim.point_weights((c,)) * sim.density
-        g_mass += _point_average_adjoint(sim, density, c)
-    g_stiff = host["normal"] * sim.point_weights(())
+        g_mass += _point_average_adjoint(grads["mass"][c] * here(sim.point_weights((c,))) * density,
+                                         c)
+    g_stiff = grads["normal"] * here(sim.point_weights(()))
     for p, axes in enumerate(PAIRS[sim.ndim][sim.ndim:]):
-        density = host["shear"][p] * sim.point_weights(axes)
-        g_stiff += _pair_average_adjoint(sim, density, gamma, axes)
+        shear = grads["shear"][p] * here(sim.point_weights(axes))
+        g_stiff += _pair_average_adjoint(sim, shear, gamma, axes)
     return {"mass": g_mass, "stiff": g_stiff}
-
-
-def _on_device(grads: dict, device) -> dict:
-    return {k: torch.as_tensor(np.ascontiguousarray(v), device=device) for k, v in grads.items()}
 
 
 def reconstruction_nodes(sim: ElasticWave):
@@ -624,10 +635,10 @@ def sensitivity(sim: ElasticWave, source: Source, indicator, sensors, objective)
         adj.adjoint_inject(l0, adjoint, m, grads["mass"], v1, mf)
     out = finalize_gradients(sim, grads, mat["gamma_host"])
     if sim.pml is not None:
-        layer = pml_nodes(sim)
+        layer = torch.as_tensor(pml_nodes(sim), device=eng.device)
         for f in out.values():
-            f[..., layer] = 0.0
-    return cost, _on_device(out, eng.device), um, {}
+            f[layer] = 0.0
+    return cost, out, um, {}
 
 
 class _Reconstruction:
@@ -676,6 +687,7 @@ class _Reconstruction:
         self.U = eng.levels(3)
         snapshot = 2 * self.U[0].nbytes + sum(a.nbytes for a in self.fwd.memory)
         strip, self.valid = reconstruction_nodes(sim)
+        self.inside = torch.as_tensor(self.valid, device=eng.device)  # where the fields are
         self.count = strip.shape[1]
         self.strip = eng.sensors(strip) if self.count else None
         segment = sim.N
@@ -745,8 +757,7 @@ class _Reconstruction:
             self.strip.replay(c, buffer, strip_row)
 
     def _valid_norm(self, level: torch.Tensor) -> float:
-        valid = torch.as_tensor(self.valid, device=self.eng.device)
-        return float(torch.linalg.vector_norm(self.eng.shots(level) * valid))
+        return float(torch.linalg.vector_norm(self.eng.shots(level) * self.inside))
 
     def leaf(self, k):
         sim, eng = self.sim, self.eng
@@ -808,7 +819,7 @@ class _Reconstruction:
     def gradients(self) -> dict:
         out = finalize_gradients(self.sim, self.grads, self.mat["gamma_host"])
         for f in out.values():
-            f[~self.valid] = 0.0
+            f[~self.inside] = 0.0
         return out
 
 
@@ -833,7 +844,7 @@ def reconstruction_sensitivity(sim: ElasticWave, source: Source, indicator, sens
     costs = run.run(objectives)
     info = {"strip": run.count, "drift": run.drift(), "segment": run.segment,
             "sweeps": run.steps / sim.N, "valid": run.valid}
-    return costs[0], _on_device(run.gradients(), run.eng.device), run.eng.shots(run.record)[0], info
+    return costs[0], run.gradients(), run.eng.shots(run.record)[0], info
 
 
 def misfit_gradient(sim: ElasticWave, sources, indicator, sensors, observed, objective,
@@ -847,7 +858,7 @@ def misfit_gradient(sim: ElasticWave, sources, indicator, sensors, observed, obj
     _require(sim, sources, nodes)
     step = min(batch or MAX_BATCH, MAX_BATCH)
     mat = sim.build_materials(indicator)
-    cost, total, valid, device = 0.0, None, None, None
+    cost, total, valid = 0.0, None, None
     for start in range(0, len(sources), step):
         chunk = sources[start:start + step]
         run = _Reconstruction(sim, mat, chunk, nodes, checkpoints)
@@ -862,12 +873,17 @@ def misfit_gradient(sim: ElasticWave, sources, indicator, sensors, observed, obj
 
         cost += sum(run.run(objectives))
         if total is None:
-            total, valid, device = run.grads, run.valid, run.eng.device
+            total, valid = run.grads, run.inside
         else:
             for k in total:
                 total[k] += run.grads[k]
     out = finalize_gradients(sim, total, mat["gamma_host"])
+    def chained(jacobian, density):
+        if np.ndim(jacobian) == 0:
+            return float(jacobian) * density
+        return torch.as_tensor(jacobian, device=density.device) * density
+
     jm, js = sim.parametrization_jacobian(indicator)
-    gradient = jm * out["mass"] + js * out["stiff"]
+    gradient = chained(jm, out["mass"]) + chained(js, out["stiff"])
     gradient[~valid] = 0.0
-    return cost, torch.as_tensor(gradient, device=device)
+    return cost, gradient

@@ -204,8 +204,10 @@ class MaxwellWave(Simulation):
                 w[tuple(wall)] *= 0.5
         return w
 
-    def _point_average(self, field: np.ndarray, c: int) -> np.ndarray:
-        out = np.zeros(self.Nx_padded, dtype=self.np_dtype)
+    # The materials' passes over the grid run in torch on the host, over its
+    # threads: the same operations in the same precision as numpy's, a pass each.
+    def _point_average(self, field: torch.Tensor, c: int) -> torch.Tensor:
+        out = torch.zeros(self.Nx_padded, dtype=self.dtype)
         lo = tuple(slice(0, n - 1) if d == c else slice(0, n) for d, n in enumerate(self.Nx))
         hi = tuple(slice(1, n) if d == c else slice(0, n) for d, n in enumerate(self.Nx))
         out[lo] = 0.5 * (field[lo] + field[hi])
@@ -214,9 +216,11 @@ class MaxwellWave(Simulation):
     def _point_harmonic(self, field: np.ndarray, c: int) -> np.ndarray:
         """The harmonic mean of the two nodes component c sits between
         (cuwave/wave.py:416-425)."""
-        tiny = np.finfo(self.np_dtype).tiny
-        mean = self._point_average(1.0 / np.maximum(field, tiny), c)
-        return np.where(mean > 0.0, 1.0 / np.maximum(mean, tiny), 0.0).astype(self.np_dtype)
+        tiny = float(np.finfo(self.np_dtype).tiny)
+        inverse = 1.0 / torch.clamp(torch.as_tensor(field), min=tiny)
+        mean = self._point_average(inverse, c)
+        return torch.where(mean > 0.0, 1.0 / torch.clamp(mean, min=tiny),
+                           torch.zeros((), dtype=self.dtype)).numpy()
 
     def _pair_average(self, field: np.ndarray, axes) -> np.ndarray:
         """The harmonic mean of the four nodes a pair point straddles (cuwave/wave.py:436-457)."""
@@ -233,11 +237,12 @@ class MaxwellWave(Simulation):
     def point_inverse_inertia(self, eps: np.ndarray) -> np.ndarray:
         """(ncomp, *Nx_padded): 1 / (W eps) on the component points, zero on a
         conductor's wall node for the tangential components (cuwave/maxwell.py:247-263)."""
-        tiny = np.finfo(self.np_dtype).tiny
-        minv = np.zeros((self.ncomp, *self.Nx_padded), dtype=self.np_dtype)
+        tiny = float(np.finfo(self.np_dtype).tiny)
+        minv = np.empty((self.ncomp, *self.Nx_padded), dtype=self.np_dtype)
         for c in range(self.ncomp):
-            mass = self._wall_weights((c,)) * self._point_harmonic(eps, c)
-            minv[c] = 1.0 / np.maximum(mass, tiny)
+            mass = torch.as_tensor(self._point_harmonic(eps, c))
+            mass.mul_(torch.as_tensor(self._wall_weights((c,)))).clamp_(min=tiny)
+            torch.div(torch.ones((), dtype=self.dtype), mass, out=torch.as_tensor(minv[c]))
         for face in faces_with(self, Conductor):
             wall = [slice(None)] * self.ndim
             wall[face // 2] = 1 if face % 2 == 0 else self.Nx[face // 2] - 2
@@ -403,14 +408,13 @@ class MaxwellEngine(ShotFields):
         return self.step(l0, l1, l0, grads["mass"], v1, mf, grads.get("nu"))
 
 
-def _point_average_adjoint(density: np.ndarray, c: int) -> np.ndarray:
+def _point_average_adjoint(density: torch.Tensor, c: int) -> torch.Tensor:
     """Transpose of the point mean: half of `density` back onto each node it spans
     (cuwave/wave.py:405-413)."""
-    out = 0.5 * density
-    to = [slice(None)] * density.ndim
-    fro = [slice(None)] * density.ndim
-    to[c], fro[c] = slice(1, None), slice(0, -1)
-    out[tuple(to)] += 0.5 * density[tuple(fro)]
+    half = 0.5 * density
+    out = half.clone()
+    n = out.shape[c]
+    out.narrow(c, 1, n - 1).add_(half.narrow(c, 0, n - 1))
     return out
 
 
@@ -436,14 +440,15 @@ def finalize_gradients(sim: MaxwellWave, grads: dict, mat: dict) -> dict:
     pair means onto the nodal 1 / mu (cuwave/maxwell.py:601-613, cuwave/wave.py:
     427-475); zero stiffness otherwise."""
     eps = mat["eps"]
-    g_mass = grads["mass"].cpu().numpy()
-    tiny = np.finfo(sim.np_dtype).tiny
-    safe = np.maximum(eps, tiny)
-    out = np.zeros(sim.Nx_padded, dtype=sim.np_dtype)
+    g_mass = grads["mass"].cpu()
+    safe = torch.clamp(torch.as_tensor(eps), min=float(np.finfo(sim.np_dtype).tiny))
+    square = safe * safe
+    total = torch.zeros(sim.Nx_padded, dtype=sim.dtype)
     for c in range(sim.ncomp):
-        density = g_mass[c] * sim._wall_weights((c,))
-        mean = sim._point_harmonic(eps, c)
-        out += _point_average_adjoint(density * mean * mean, c) / (safe * safe)
+        density = g_mass[c] * torch.as_tensor(sim._wall_weights((c,)))
+        mean = torch.as_tensor(sim._point_harmonic(eps, c))
+        total += _point_average_adjoint(density * mean * mean, c) / square
+    out = total.numpy()
     stiff = np.zeros(sim.Nx_padded, dtype=sim.np_dtype)
     if sim.magnetic:
         g_nu = grads["nu"].cpu().numpy()

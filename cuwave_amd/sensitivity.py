@@ -25,7 +25,7 @@ import numpy as np
 import scipy.ndimage as ndi
 import torch
 
-from .boundary import pml_nodes
+from .boundary import pml_nodes, pml_widths
 from .engine import Propagator, sensor_points, source_points
 from .wave import Simulation, Source, as_numpy, family_drivers
 
@@ -116,6 +116,24 @@ def _zero_outside(grads: dict, mask: np.ndarray, device) -> dict:
     return grads
 
 
+def _shell(outer, inner) -> np.ndarray:
+    """The nodes of the box `outer` off the box `inner` inside it (a (low, high) pair an
+    axis each), (ndim, num) in row-major order, without visiting the nodes inside."""
+    (o0, o1), (i0, i1) = outer[0], inner[0]
+    if len(outer) == 1:
+        return np.concatenate((np.arange(o0, i0), np.arange(i1, o1))).astype(np.int32)[None]
+    every = np.indices([b - a for a, b in outer[1:]], dtype=np.int32).reshape(len(outer) - 1, -1)
+    every = every + np.array([a for a, _ in outer[1:]], dtype=np.int32)[:, None]
+    ring = _shell(outer[1:], inner[1:])
+
+    def planes(a, b, rest):
+        rows = np.repeat(np.arange(a, b, dtype=np.int32), rest.shape[1])
+        return np.concatenate((rows[None], np.tile(rest, (1, max(b - a, 0)))))
+
+    return np.concatenate((planes(o0, i0, every), planes(i0, i1, ring), planes(i1, o1, every)),
+                          axis=1)
+
+
 def reconstruction_nodes(sim: Simulation, indicator=None, span: int | None = None):
     """The nodes a reverse march replays from a record, and those it rebuilds exactly.
 
@@ -128,17 +146,25 @@ def reconstruction_nodes(sim: Simulation, indicator=None, span: int | None = Non
     Returns the (ndim, num) record nodes in row-major order and the mask of the
     reversible interior nodes, where the rebuilt field is exact.
     """
+    if sim.damping is None:
+        # the reversible nodes are a box, its dilation a box too: nothing to search for
+        widths = [(0, 0)] * sim.ndim if sim.pml is None else pml_widths(sim)
+        box = [(1 + lo, n - 1 - hi) for (lo, hi), n in zip(widths, sim.Nx)]
+        exact = np.zeros(sim.Nx_padded, dtype=bool)
+        exact[tuple(slice(a, max(a, b)) for a, b in box)] = True
+        if sim.pml is None or any(a >= b for a, b in box):
+            return np.zeros((sim.ndim, 0), dtype=np.int32), exact
+        grown = [(max(1, a - sim.reach), min(n - 1, b + sim.reach))
+                 for (a, b), n in zip(box, sim.Nx)]
+        return _shell(grown, box), exact
     inside = np.zeros(sim.Nx_padded, dtype=bool)
     inside[tuple(slice(1, n - 1) for n in sim.Nx)] = True
-    if sim.pml is None and sim.damping is None:
-        return np.zeros((sim.ndim, 0), dtype=np.int32), inside
     exact = inside.copy()
     if sim.pml is not None:
         exact &= ~pml_nodes(sim)
-    if sim.damping is not None:
-        # a damped node runs back only where its growth stays bounded over the span
-        span = sim.N if span is None else span
-        exact &= ~(sim.damping > 0) | reversible_damping(sim, indicator, span)
+    # a damped node runs back only where its growth stays bounded over the span
+    span = sim.N if span is None else span
+    exact &= ~(sim.damping > 0) | reversible_damping(sim, indicator, span)
     # a box maximum is the dilation by the full square, taken `reach` times over
     seen = ndi.maximum_filter(exact.astype(np.uint8), size=2 * sim.reach + 1,
                               mode="constant", cval=0).astype(bool)
@@ -369,10 +395,11 @@ class _Reconstruction:
                              "there is nothing to reconstruct; set checkpoints, damp only the "
                              "faces with boundary.sponge, or use sensitivity")
         self.count = strip.shape[1]
-        smap = np.full(sim.Nx_padded, -1, dtype=np.int32)
+        self.strip_map = torch.full(sim.Nx_padded, -1, dtype=torch.int32, device=dev)
         if self.count:
-            smap.ravel()[sim.flatten_indices(strip)] = np.arange(self.count, dtype=np.int32)
-        self.strip_map = torch.as_tensor(smap, device=dev)
+            at = torch.as_tensor(sim.flatten_indices(strip), device=dev).long()
+            self.strip_map.view(-1)[at] = torch.arange(self.count, dtype=torch.int32, device=dev)
+        self.inside = torch.as_tensor(self.valid, device=dev)  # `valid` where the fields are
         self.src_back = self.src
         if sim.damping is not None:
             # backwards a reversible damping is negated (cuwave/sensitivity.py:592-598);
@@ -484,8 +511,7 @@ class _Reconstruction:
             prop.backward(self.lam, self.U, s, s + 1, reverse=False, **common)
 
     def _valid_norm(self, level: torch.Tensor) -> float:
-        valid = torch.as_tensor(self.valid, device=self.dev)
-        return float(torch.linalg.vector_norm(self.prop.shots(level) * valid))
+        return float(torch.linalg.vector_norm(self.prop.shots(level) * self.inside))
 
     def drift(self) -> float:
         """Norm of the rebuilt u^(-1), which is zero, over that of the top state."""
@@ -529,7 +555,7 @@ def reconstruction_sensitivity(sim: Simulation, source: Source, indicator, senso
 
     costs = run.run(objectives, dict(g_mass=acc["mass"], g_stiff=acc["stiff"], skip_layer=True))
     grads = _finalize(sim, acc, dev)
-    grads = _zero_outside(grads, ~run.valid, dev)
+    grads = _zero_outside(grads, ~run.inside, dev)
     info = {"strip": run.count, "drift": run.drift(), "segment": run.segment,
             "sweeps": run.steps / sim.N}
     return costs[0], grads, run.prop.shots(run.record)[0], info

@@ -266,7 +266,7 @@ def misfit_gradient(sim: Simulation, sources: Sequence[Source], indicator, senso
     for start, chunk in _batches(sources, batch):
         run = _Reconstruction(sim, mat, chunk, sensors.nodes, checkpoints=checkpoints,
                               illum=illum, indicator=indicator)
-        valid = run.valid
+        valid = run.inside
         if constant:  # the kernel chains the Jacobian as it sums: one accumulator
             acc = run.prop.accumulator()
             mode = dict(g_mass=acc, combine=(jm, js), skip_layer=True)
@@ -298,7 +298,7 @@ def misfit_gradient(sim: Simulation, sources: Sequence[Source], indicator, senso
             return torch.as_tensor(d, dtype=gradient.dtype, device=gradient.device)
 
         gradient = field(jm) * (gradient[0] * w) + field(js) * (gradient[1] * w)
-        gradient[torch.as_tensor(~valid, device=gradient.device)] = 0.0
+        gradient[~valid] = 0.0
         return cost, gradient
     grads = _finalize(sim, {"g": gradient}, gradient.device)
     grads = _zero_outside(grads, ~valid, gradient.device)
