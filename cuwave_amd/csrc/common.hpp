@@ -25,6 +25,29 @@ template <int NDIM> struct TileShape {
   static constexpr int TY = kThreads / TX;
 };
 
+// division of an unsigned under 2^31 by a number the host knows: a product's
+// high half, an addition and a shift where the general division takes about
+// twenty instructions, three times over to find a node
+struct Div {
+  uint32_t m, s, d;
+};
+inline Div make_div(int64_t by) {
+  Div v{0, 0, (uint32_t)(by < 1 ? 1 : by)};
+  while (((uint64_t)1 << v.s) < v.d)
+    ++v.s;
+  v.m = (uint32_t)((((uint64_t)1 << 32) * (((uint64_t)1 << v.s) - v.d)) / v.d + 1);
+  return v;
+}
+__device__ __forceinline__ uint32_t quot(const Div &v, uint32_t t) {
+  return (__umulhi(v.m, t) + t) >> v.s;
+}
+// the quotient, and the remainder in `rest`
+__device__ __forceinline__ uint32_t quot(const Div &v, uint32_t t, uint32_t &rest) {
+  const uint32_t q = quot(v, t);
+  rest = t - q * v.d;
+  return q;
+}
+
 // the grid and operator a kernel reads, all by value
 template <typename T> struct Geom {
   int n[3];          // logical extents (ghosts included)
@@ -38,6 +61,10 @@ template <typename T> struct Geom {
   int tf, tm, ts;    // point tiles along the fast, middle and slow axes
   int ntiles;
   int interior;      // interior nodes (every axis 1 .. n - 2)
+  Div row;           // interior columns of the fast axis
+  // 3D: a stripe of rows through every plane, its rows of one plane, and the
+  // last stripe's (general_node)
+  Div stripe, band, last;
   T op[4];           // op[k - 1], the full-radius cell weights
   T f[3];            // step factors per axis
 };
@@ -204,6 +231,18 @@ __device__ __forceinline__ void keep(Lanes<T, V> &x) {
     CW_KEEP(x.v[i]);
 }
 
+// the V lanes `off` bytes past a base every thread shares: the base's own
+// offsets (a tap's distance, a row of memory) are scalar arithmetic and the
+// load's address one addition, or none where off has 32 bits
+template <typename Q, typename T, typename Off>
+__device__ __forceinline__ Q at_bytes(const T *base, Off off) {
+  return *reinterpret_cast<const Q *>(reinterpret_cast<const char *>(base) + off);
+}
+template <typename Q, typename T, typename Off>
+__device__ __forceinline__ void put_bytes(T *base, Off off, const Q &v) {
+  *reinterpret_cast<Q *>(reinterpret_cast<char *>(base) + off) = v;
+}
+
 // the V lanes at element e of a per-shot array (e a multiple of V)
 template <typename Q, typename T>
 __device__ __forceinline__ Q lanes_at(const T *__restrict__ p, int64_t e) {
@@ -240,6 +279,16 @@ __device__ __forceinline__ int mirror_step(int a, int N, int odd, int j,
   const int b = a + j;
   neg = (b < 0 && (odd & 1)) || (b > N - 1 && (odd & 2));
   return (b < 0 ? 2 - b : b > N - 1 ? 2 * (N - 2) - b : b) - a;
+}
+
+// mirror_step for a tap that can only pass the wall on its own side: the low
+// one for j < 0, the high one for j > 0 (an axis has R + 3 nodes or more)
+__device__ __forceinline__ int mirror_side(int a, int N, int odd, int j,
+                                           bool &neg) {
+  const int b = a + j;
+  const bool past = j < 0 ? b < 0 : b > N - 1;
+  neg = past && (odd & (j < 0 ? 1 : 2));
+  return past ? (j < 0 ? 2 : 2 * (N - 2)) - b - a : j;
 }
 
 // tap j through the image about the wall node, for a field no refill keeps

@@ -26,10 +26,12 @@
 
 namespace cwe {
 
+using cw::at_bytes;
 using cw::fmat;
 using cw::lanes_at;
 using cw::lanes_put;
 using cw::LanesOf;
+using cw::put_bytes;
 
 constexpr int kThreads = 256;
 
@@ -94,15 +96,6 @@ __device__ __forceinline__ int64_t slab_at(int a, int N, int lo, int hi, bool sl
 // tap's distance costs no vector instruction.
 template <int NDIM, typename T>
 using Place = std::conditional_t<NDIM == 3 || (NDIM == 2 && sizeof(T) == 4), uint32_t, uint64_t>;
-
-template <typename Q, typename T, typename Off>
-__device__ __forceinline__ Q at_bytes(const T *base, Off off) {
-  return *reinterpret_cast<const Q *>(reinterpret_cast<const char *>(base) + off);
-}
-template <typename Q, typename T, typename Off>
-__device__ __forceinline__ void put_bytes(T *base, Off off, const Q &v) {
-  *reinterpret_cast<Q *>(reinterpret_cast<char *>(base) + off) = v;
-}
 
 // A line of points a derivative reads: a field component (or a stress row)
 // along an axis, and optionally through the PML memory (the value coef *

@@ -112,6 +112,15 @@ template <typename T> cw::Geom<T> make_geom(const cw_grid &gr) {
   g.interior = 1;
   for (int d = 0; d < nd; ++d)
     g.interior *= g.n[d] - 2;
+  const int64_t W = g.n[nd - 1] - 2;
+  g.row = cw::make_div(W);
+  if (nd == 3) {
+    const int H = g.n[1] - 2, rows = (H + cw::kXcds - 1) / cw::kXcds;
+    const int whole = H / rows; // stripes of `rows` rows; the last takes the rest
+    g.stripe = cw::make_div((int64_t)(g.n[0] - 2) * rows * W);
+    g.band = cw::make_div(rows * W);
+    g.last = cw::make_div((H - whole * rows) * W);
+  }
   for (int k = 0; k < 4; ++k)
     g.op[k] = (T)gr.op[k];
   for (int d = 0; d < 3; ++d)
@@ -247,6 +256,10 @@ inline cw::Region band_of(const cw_grid &g, const cw::Box &b) {
   const int W = g.n[1] - 2;
   r.count = (b.y0 - 1) * W + (g.n[0] - 1 - b.y1) * W +
             (b.y1 - b.y0) * ((b.x0 - 1) + (g.n[1] - 1 - b.x1));
+  r.by[0] = cw::make_div(W);
+  r.by[1] = cw::make_div(2 * r.q);
+  r.by[2] = cw::make_div(W - 2 * r.q);
+  r.by[3] = cw::make_div((b.x0 - 1 - r.q) + (g.n[1] - 1 - r.q - b.x1));
   return r;
 }
 

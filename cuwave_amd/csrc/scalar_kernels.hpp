@@ -76,6 +76,10 @@ struct Region {
   int count; // band nodes
   int q;     // (2D) the rows and columns by each wall that its folds reach, R + 1
   int z0, z1;
+  // the divisors of the enumeration: (2D) a row's columns, the wall columns,
+  // the columns off the side walls, the side columns; (3D) a row, a plane, a
+  // plane's rows off the box, a plane's columns off it, a row's
+  Div by[5];
 };
 
 template <typename T> struct FwdParams {
@@ -193,32 +197,49 @@ template <typename T> __device__ __forceinline__ T harmonic(T a, T b) {
   return a * b / (a + b);
 }
 
+// slab_index in 32 bits (a slab holds fewer nodes than a field)
+template <int NDIM, typename T>
+__device__ __forceinline__ uint32_t slab_place(const Geom<T> &g, const int *a,
+                                               int d, int row, int lo, int hi) {
+  uint32_t off = 0, plane = 1;
+#pragma unroll
+  for (int e = 0; e < NDIM; ++e)
+    if (e != d) {
+      off = off * g.np[e] + a[e];
+      plane *= g.np[e];
+    }
+  return d < NDIM - 1 ? row * plane + off : off * (uint32_t)(lo + hi) + row;
+}
+
+// the profile of an axis of N nodes at node a: a and b at the node, at the
+// half point above it and at the one below
+template <typename T>
+__device__ __forceinline__ void profile_at(const T *prof, int N, int a, T *v) {
+  const uint32_t at = (uint32_t)a * sizeof(T);
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    v[k] = at_bytes<T>(prof + k * N, at);
+  v[4] = at_bytes<T>(prof + 2 * N - 1, at);
+  v[5] = at_bytes<T>(prof + 3 * N - 1, at);
+}
+
 // the forward CPML of axis d at a slab node (cuwave/kernels/scalar.cu:
 // 499-532): the three memories, `size` elements apart, updated in place,
 // their share of the field returned. `an .. bh1` are the profile at the node
 // and at the half point below it.
-// `m` holds the three memories as read (so a caller may load them early)
+// `m` holds the three memories as read, `own` their place in bytes, `pr` the
+// profile (profile_at)
 template <typename T, typename Q = T>
-__device__ __forceinline__ Q pml_forward_from(const Q *m, T *aux,
+__device__ __forceinline__ Q pml_forward_from(const Q *m, T *aux, uint64_t own,
                                               int64_t size, Q Dp, Q Dm, T gp,
-                                              T gm, T f, T mi, T an, T bn,
-                                              T ah, T bh, T ah1, T bh1) {
-  const Q pp = bh * m[0] + ah * Dp;
-  const Q pm = bh1 * m[1] + ah1 * Dm;
-  const Q z = bn * m[2] + an * f * (gp * (Dp + pp) - gm * (Dm + pm));
-  lanes_put(aux, 0, pp);
-  lanes_put(aux, size, pm);
-  lanes_put(aux, 2 * size, z);
+                                              T gm, T f, T mi, const T *pr) {
+  const Q pp = pr[3] * m[0] + pr[2] * Dp;
+  const Q pm = pr[5] * m[1] + pr[4] * Dm;
+  const Q z = pr[1] * m[2] + pr[0] * f * (gp * (Dp + pp) - gm * (Dm + pm));
+  put_bytes(aux, own, pp);
+  put_bytes(aux + size, own, pm);
+  put_bytes(aux + 2 * size, own, z);
   return mi * (f * (gp * pp - gm * pm) + z);
-}
-template <typename T, typename Q = T>
-__device__ __forceinline__ Q pml_forward(T *aux, int64_t size, Q Dp, Q Dm,
-                                         T gp, T gm, T f, T mi, T an, T bn,
-                                         T ah, T bh, T ah1, T bh1) {
-  const Q m[3] = {lanes_at<Q>(aux, 0), lanes_at<Q>(aux, size),
-                  lanes_at<Q>(aux, 2 * size)};
-  return pml_forward_from(m, aux, size, Dp, Dm, gp, gm, f, mi, an, bn, ah, bh,
-                          ah1, bh1);
 }
 
 // the adjoint memory of a slab node stepped by lambda (scalar_sensitivity.cu:
@@ -415,42 +436,41 @@ template <typename T>
 __device__ __forceinline__ bool band_node(const Region &r, const Geom<T> &g,
                                           int t, int *a) {
   const int N0 = g.n[0], N1 = g.n[1], W = N1 - 2, q = r.q;
+  uint32_t k;
   const int rows = 2 * q * W;
   if (t < rows) {
-    const int k = t / W;
-    a[0] = k < q ? 1 + k : N0 - 1 - 2 * q + k;
-    a[1] = 1 + t % W;
+    const int row = (int)quot(r.by[0], t, k);
+    a[0] = row < q ? 1 + row : N0 - 1 - 2 * q + row;
+    a[1] = 1 + (int)k;
     return true;
   }
   t -= rows;
   if (t < (N0 - 2 - 2 * q) * 2 * q) {
-    const int k = t % (2 * q);
-    a[0] = q + 1 + t / (2 * q);
-    a[1] = k < q ? 1 + k : N1 - 1 - 2 * q + k;
+    a[0] = q + 1 + (int)quot(r.by[1], t, k);
+    a[1] = (int)k < q ? 1 + (int)k : N1 - 1 - 2 * q + (int)k;
     return true;
   }
   t -= (N0 - 2 - 2 * q) * 2 * q;
   const int Wi = W - 2 * q; // the columns off the side walls
   const int top = (r.y0 - 1 - q) * Wi;
   if (t < top) {
-    a[0] = q + 1 + t / Wi;
-    a[1] = q + 1 + t % Wi;
+    a[0] = q + 1 + (int)quot(r.by[2], t, k);
+    a[1] = q + 1 + (int)k;
     return true;
   }
   t -= top;
   const int bot = (N0 - 1 - q - r.y1) * Wi;
   if (t < bot) {
-    a[0] = r.y1 + t / Wi;
-    a[1] = q + 1 + t % Wi;
+    a[0] = r.y1 + (int)quot(r.by[2], t, k);
+    a[1] = q + 1 + (int)k;
     return true;
   }
   t -= bot;
   const int left = r.x0 - 1 - q, right = N1 - 1 - q - r.x1, per = left + right;
   if (per <= 0 || t >= per * (r.y1 - r.y0))
     return false;
-  const int k = t % per;
-  a[0] = r.y0 + t / per;
-  a[1] = k < left ? q + 1 + k : r.x1 + (k - left);
+  a[0] = r.y0 + (int)quot(r.by[3], t, k);
+  a[1] = (int)k < left ? q + 1 + (int)k : r.x1 + ((int)k - left);
   return true;
 }
 
@@ -462,21 +482,22 @@ __device__ __forceinline__ bool shell_node(const Region &r, const Geom<T> &g,
                                            int t, int *a) {
   const int H = g.n[1] - 2, W = g.n[2] - 2;
   const int before = r.z0 - 1, planes = before + (g.n[0] - 1 - r.z1);
+  uint32_t rest, k;
   if (t < planes * H * W) {
-    const int k = t / (H * W), rest = t % (H * W);
-    a[0] = k < before ? 1 + k : r.z1 + (k - before);
-    a[1] = 1 + rest / W;
-    a[2] = 1 + rest % W;
+    const int z = (int)quot(r.by[1], t, rest);
+    a[0] = z < before ? 1 + z : r.z1 + (z - before);
+    a[1] = 1 + (int)quot(r.by[0], rest, k);
+    a[2] = 1 + (int)k;
     return true;
   }
   t -= planes * H * W;
   const int depth = r.z1 - r.z0;
   const int above = r.y0 - 1, rows = above + (g.n[1] - 1 - r.y1);
   if (t < depth * rows * W) {
-    const int rest = t % (rows * W), k = rest / W;
-    a[0] = r.z0 + t / (rows * W);
-    a[1] = k < above ? 1 + k : r.y1 + (k - above);
-    a[2] = 1 + rest % W;
+    a[0] = r.z0 + (int)quot(r.by[2], t, rest);
+    const int y = (int)quot(r.by[0], rest, k);
+    a[1] = y < above ? 1 + y : r.y1 + (y - above);
+    a[2] = 1 + (int)k;
     return true;
   }
   t -= depth * rows * W;
@@ -484,10 +505,9 @@ __device__ __forceinline__ bool shell_node(const Region &r, const Geom<T> &g,
   const int span = r.y1 - r.y0;
   if (cols <= 0 || t >= depth * span * cols)
     return false;
-  const int rest = t % (span * cols), k = rest % cols;
-  a[0] = r.z0 + t / (span * cols);
-  a[1] = r.y0 + rest / cols;
-  a[2] = k < left ? 1 + k : r.x1 + (k - left);
+  a[0] = r.z0 + (int)quot(r.by[3], t, rest);
+  a[1] = r.y0 + (int)quot(r.by[4], rest, k);
+  a[2] = (int)k < left ? 1 + (int)k : r.x1 + ((int)k - left);
   return true;
 }
 
@@ -517,27 +537,25 @@ __device__ __forceinline__ bool general_node(const Region &r, const Geom<T> &g,
   const int t = xcd_tile(bid, nb) * per + (int)(threadIdx.x >> ts);
   if (t >= g.interior)
     return false;
+  uint32_t rest, k;
   if (NDIM == 1) {
     a[0] = 1 + t;
   } else if (NDIM == 2) {
-    const int W = g.n[1] - 2;
-    a[0] = 1 + t / W;
-    a[1] = 1 + t % W;
+    a[0] = 1 + (int)quot(g.row, t, k);
+    a[1] = 1 + (int)k;
   } else {
     // the rows cut into kXcds stripes, a stripe's nodes in (plane, row,
     // column) order: the run of items an XCD takes is one stripe marched
     // plane by plane, so the planes the slow-axis taps read (R either side)
     // are the stripe's share of them, which its L2 holds (whole planes it
     // would not)
-    const int W = g.n[2] - 2, H = g.n[1] - 2;
-    const int hs = (H + kXcds - 1) / kXcds;
-    const int64_t full = (int64_t)(g.n[0] - 2) * hs * W;
-    const int k = (int)(t / full);
-    const int rem = (int)(t - k * full);
-    const int rows = min(hs, H - k * hs);
-    a[0] = 1 + rem / (rows * W);
-    a[1] = 1 + k * hs + (rem % (rows * W)) / W;
-    a[2] = 1 + rem % W;
+    const int H = g.n[1] - 2, hs = (H + kXcds - 1) / kXcds;
+    const int stripe = (int)quot(g.stripe, t, rest);
+    const Div &plane = (stripe + 1) * hs <= H ? g.band : g.last;
+    uint32_t in;
+    a[0] = 1 + (int)quot(plane, rest, in);
+    a[1] = 1 + stripe * hs + (int)quot(g.row, in, k);
+    a[2] = 1 + (int)k;
   }
   return true;
 }
@@ -601,12 +619,15 @@ __device__ __forceinline__ void forward_general(const FwdParams<T> &p,
   }
   const int elem = (node << sh) + b;
   const int64_t e = elem;
-  const T mi = p.inv[idx];
+  // this node's and this thread's places in per-node and per-shot arrays
+  const uint64_t nat = (uint64_t)(uint32_t)node * sizeof(T);
+  const uint64_t at = (uint64_t)(uint32_t)elem * sizeof(T);
+  const T mi = at_bytes<T>(p.inv, nat);
   T gp[NDIM], gm[NDIM];
 #pragma unroll
   for (int d = 0; d < NDIM; ++d) {
-    gp[d] = p.cell[d * g.nodes + idx];
-    gm[d] = p.cell[d * g.nodes + idx - g.s[d]];
+    gp[d] = at_bytes<T>(p.cell + d * g.nodes, nat);
+    gm[d] = at_bytes<T>(p.cell + (d * g.nodes - g.s[d]), nat);
   }
   int prow[NDIM];
   bool layer = false;
@@ -631,22 +652,56 @@ __device__ __forceinline__ void forward_general(const FwdParams<T> &p,
   if ((layer || p.damp) && p.strip.map) // a damped node may be a strip node
     col = p.strip.map[idx];
   const T *__restrict__ u1 = p.u.at(t - 1);
+  // the layer memory this node owns and its profile: in flight with the taps
+  // where a lane group is small (a one-shot 298 x 298 step 6.0 us without, 5.2
+  // with), and only when it is used in 3D or where a group is 16 bytes (held
+  // through the taps it would halve the waves a SIMD holds)
+  constexpr bool kEarly = NDIM < 3 && sizeof(Q) <= 8;
+  Q mem[NDIM][3];
+  T pr[NDIM][6];
+  uint64_t own[NDIM];
+  auto load_layer = [&](int d) {
+    const int L = p.pml.lo[d], H = p.pml.hi[d];
+    const int64_t size = slab_size<NDIM>(g, d, L, H) << sh;
+    own[d] = (uint64_t)((slab_place<NDIM>(g, a, d, prow[d], L, H) << sh) + b) * sizeof(T);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      mem[d][k] = at_bytes<Q>(p.pml.aux[d] + k * size, own[d]);
+    profile_at(p.pml.profile[d], g.n[d], a[d], pr[d]);
+  };
+  if (kEarly && layer)
+#pragma unroll
+    for (int d = 0; d < NDIM; ++d)
+      if (prow[d] >= 0)
+        load_layer(d);
   Q taps[NDIM][2 * R + 1];
 #pragma unroll
   for (int d = 0; d < NDIM; ++d) {
-    const int se = g.s[d] << sh;
+    const int64_t se = (int64_t)g.s[d] << sh;
     // mirrored only along an axis near a wall (the same bits as along every
-    // axis), there by moving the one load of a tap and setting its sign
+    // axis), there by moving the one load of a tap and setting its sign; a
+    // wave with no node near this axis' walls (most are, along the slow axes
+    // nearly all) takes the taps at their distances as they are
     const bool wall = !(deep || (a[d] >= R && a[d] <= g.n[d] - 1 - R));
+    if (!__any(wall)) {
 #pragma unroll
-    for (int j = -R; j <= R; ++j) {
-      bool neg = false;
-      const int k =
-          wall ? mirror_step(a[d], g.n[d], g.dirichlet >> (2 * d), j, neg) : j;
-      const Q v = lanes_at<Q>(u1, elem + k * se);
-      taps[d][j + R] = neg ? -v : v;
+      for (int j = -R; j <= R; ++j)
+        taps[d][j + R] = at_bytes<Q>(u1 + j * se, at);
+    } else {
+#pragma unroll
+      for (int j = -R; j <= R; ++j) {
+        if (j >= -1 && j <= 1) { // within the ghosts of any interior node
+          taps[d][j + R] = at_bytes<Q>(u1 + j * se, at);
+          continue;
+        }
+        bool neg = false;
+        const int k = mirror_side(a[d], g.n[d], g.dirichlet >> (2 * d), j, neg);
+        const Q v = lanes_at<Q>(u1, elem + k * (int)se);
+        taps[d][j + R] = neg ? -v : v;
+      }
     }
   }
+  const Q before = at_bytes<Q>(p.u.at(t - 2), at);
   const Q uc = taps[0][R];
   Q lap;
   if (MASK && !(code & kDeepCells)) {
@@ -659,9 +714,8 @@ __device__ __forceinline__ void forward_general(const FwdParams<T> &p,
       div[d] = flux<T, R>(taps[d], gp[d], gm[d], g.op);
     lap = combine_axes<T, NDIM, R>(div, g.f);
   }
-  Q v = p.damp ? damped<T, Q>(uc, lanes_at<Q>(p.u.at(t - 2), e), mi * lap, mi,
-                              p.damp[idx], p.dt)
-               : -lanes_at<Q>(p.u.at(t - 2), e) + (T)2 * uc + mi * lap;
+  Q v = p.damp ? damped<T, Q>(uc, before, mi * lap, mi, p.damp[idx], p.dt)
+               : -before + (T)2 * uc + mi * lap;
   if (held)
     v = (T)0;
   if (layer) {
@@ -669,17 +723,13 @@ __device__ __forceinline__ void forward_general(const FwdParams<T> &p,
     for (int d = 0; d < NDIM; ++d) {
       if (prow[d] < 0)
         continue;
-      const int N = g.n[d], L = p.pml.lo[d], H = p.pml.hi[d], ad = a[d];
-      const T *an = p.pml.profile[d], *bn = an + N, *ah = an + 2 * N,
-              *bh = an + 3 * N;
-      const int64_t size = slab_size<NDIM>(g, d, L, H) << sh;
-      T *aux = p.pml.aux[d] +
-               (slab_index<NDIM>(g, a, d, prow[d], L, H) << sh) + b;
+      const int64_t size = slab_size<NDIM>(g, d, p.pml.lo[d], p.pml.hi[d]) << sh;
       Q Dp, Dm;
       cell_diffs<T, R>(taps[d], g.op, Dp, Dm);
-      const Q share =
-          pml_forward(aux, size, Dp, Dm, gp[d], gm[d], g.f[d], mi, an[ad],
-                      bn[ad], ah[ad], bh[ad], ah[ad - 1], bh[ad - 1]);
+      if (!kEarly)
+        load_layer(d);
+      const Q share = pml_forward_from(mem[d], p.pml.aux[d], own[d], size, Dp, Dm, gp[d], gm[d],
+                                       g.f[d], mi, pr[d]);
       if (!held)
         v += share;
     }
@@ -690,7 +740,7 @@ __device__ __forceinline__ void forward_general(const FwdParams<T> &p,
         if (p.src.takes(k, idx, b + i))
           lane(v, i) += p.src.weight[k] * p.signal[p.src.at(t, k, b + i)];
   T *__restrict__ u2 = p.u.at(t);
-  lanes_put(u2, e, v);
+  put_bytes(u2, at, v);
   if (p.illum) {
     // every thread of the node takes part in the sum; one writer a node
     const T s2 = shot_sum(v * v, g.lanes);
@@ -715,14 +765,14 @@ __device__ __forceinline__ void forward_general(const FwdParams<T> &p,
           p.record[p.rec.at(t, k, b + i)] = lane(v, i);
   {
     if (col >= 0) {
-      const int64_t at =
+      const int64_t to =
           (((int64_t)(t - p.strip.first) * p.strip.count + col) << sh) + b;
       if (p.strip.bf16) {
 #pragma unroll
         for (int i = 0; i < V; ++i)
-          ((uint16_t *)p.strip.record)[at + i] = bf16_bits((float)lane(v, i));
+          ((uint16_t *)p.strip.record)[to + i] = bf16_bits((float)lane(v, i));
       } else {
-        lanes_put((T *)p.strip.record, at, v);
+        lanes_put((T *)p.strip.record, to, v);
       }
     }
   }
