@@ -62,8 +62,10 @@ template <typename T> cwa::AnGeom<T> make_geom(const cw_aniso_grid &gr) {
   g.nodes = stride;
   g.lanes = gr.lanes;
   g.interior = 1;
-  for (int d = 0; d < gr.ndim; ++d)
+  for (int d = 0; d < gr.ndim; ++d) {
     g.interior *= gr.n[d] - 2;
+    g.by[d] = cw::make_div(gr.n[d] - 2);
+  }
   g.f = (T)gr.step;
   return g;
 }

@@ -17,13 +17,21 @@
 // (scalar) loads: every index into it is a compile-time constant.
 #pragma once
 
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace cwa {
 
-using cw::lanes_at;
-using cw::lanes_put;
+using cw::at_bytes;
 using cw::LanesOf;
+using cw::put_bytes;
+
+// A thread's place in a component, in bytes: 32 bits where a component stays
+// under 4 GiB (the batch's elements are under 2^31), so that a neighbour's
+// load is a scalar base and this register.
+template <int NDIM, typename T>
+using Place = std::conditional_t<sizeof(T) == 4 && (NDIM > 1), uint32_t, uint64_t>;
 
 constexpr int kThreads = 256;
 
@@ -32,40 +40,68 @@ template <typename T> struct AnGeom {
   int64_t nodes;  // nodes of one component
   int lanes;
   int interior;   // interior nodes, every axis 1 .. n - 2
+  cw::Div by[3];  // interior nodes of each axis
   T f;            // the update factor dt^2 (the spacing sits in K)
 };
 
 template <int NDIM> constexpr int corners() { return 1 << NDIM; }
 template <int NDIM> constexpr int nloc() { return corners<NDIM>() * NDIM; }
 
-// the interior node of this thread and the first of its V lanes
+// the interior node of this thread, the first of its V lanes and its places in
+// a node array and in a component
+template <int NDIM, typename T> struct AnNode {
+  int A[3];
+  int64_t idx;
+  int lane0;
+  Place<NDIM, T> nat, at;
+};
 template <int NDIM, int V, typename T>
-__device__ __forceinline__ bool an_node(const AnGeom<T> &g, int *A, int64_t *idx, int *lane0) {
+__device__ __forceinline__ bool an_node(const AnGeom<T> &g, AnNode<NDIM, T> &n) {
+  using P = Place<NDIM, T>;
   const int per = g.lanes / V;
-  const int64_t t = (int64_t)cw::xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  const int64_t i = t / per;
-  if (i >= g.interior)
+  const uint32_t t = (uint32_t)cw::xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const uint32_t i = t >> __builtin_ctz(per);
+  if (i >= (uint32_t)g.interior)
     return false;
-  *lane0 = (int)(t % per) * V;
-  int64_t rest = i;
+  n.lane0 = (int)(t & (per - 1)) * V;
+  uint32_t rest = i, k;
 #pragma unroll
-  for (int d = NDIM - 1; d >= 0; --d) {
-    const int w = g.n[d] - 2;
-    A[d] = 1 + (int)(rest % w);
-    rest /= w;
+  for (int d = NDIM - 1; d > 0; --d) {
+    rest = cw::quot(g.by[d], rest, k);
+    n.A[d] = 1 + (int)k;
   }
-  int64_t at = 0;
+  n.A[0] = 1 + (int)rest;
+  int at = 0;
 #pragma unroll
   for (int d = 0; d < NDIM; ++d)
-    at += (int64_t)A[d] * g.s[d];
-  *idx = at;
+    at += n.A[d] * g.s[d];
+  n.idx = at;
+  n.nat = (P)at * (P)sizeof(T);
+  n.at = ((P)at * (P)g.lanes + (P)n.lane0) * (P)sizeof(T);
   return true;
+}
+
+// the node steps from a node to corner l of the cell whose low corner is the
+// node itself moved by `low` (a bit an axis: one node back)
+template <int NDIM, typename T>
+__device__ __forceinline__ int corner_step(const AnGeom<T> &g, int low, int l) {
+  int off = 0;
+#pragma unroll
+  for (int d = 0; d < NDIM; ++d)
+    off += (((l >> d) & 1) - ((low >> d) & 1)) * g.s[d];
+  return off;
 }
 
 // fd_kernel without damping (anisotropic.cu:367-397): the cell-gathered force
 // on every component, then u2 = -u0 + 2 u1 + f minv force. The cells run in
 // block order (axis 0 fastest, the cell below the node first), then the
 // corners of a cell in the same order, then the components.
+//
+// In 2D its instructions bound it as much as HBM does: the gather is 64 products
+// with K a lane (each a rounding of its own, which the order of the reference
+// fixes) and the step moves 405 MB at 1026^2 nodes and 16 float lanes. A wave
+// off the walls loads the nodes around once (9 in 2D, where a cell after the
+// other reads 16) and gathers without a test a cell.
 template <typename T, int NDIM, int V>
 __global__ void __launch_bounds__(kThreads)
 an_step(AnGeom<T> g, const T *__restrict__ K, const T *__restrict__ minv,
@@ -73,56 +109,80 @@ an_step(AnGeom<T> g, const T *__restrict__ K, const T *__restrict__ minv,
         const T *__restrict__ damping, T dt) {
   using Q = LanesOf<T, V>;
   constexpr int NL = nloc<NDIM>();
-  int A[3];
-  int64_t idx;
-  int lane0;
-  if (!an_node<NDIM, V>(g, A, &idx, &lane0))
+  AnNode<NDIM, T> n;
+  if (!an_node<NDIM, V>(g, n))
     return;
   const int64_t comp = g.nodes * g.lanes;
-  const T *v = u1 + idx * g.lanes + lane0;
   Q force[NDIM];
 #pragma unroll
   for (int i = 0; i < NDIM; ++i)
     force[i] = (T)0;
+  bool wall = false;
 #pragma unroll
-  for (int c = 0; c < corners<NDIM>(); ++c) {
-    bool inside = true;
-    int base = 0;
+  for (int d = 0; d < NDIM; ++d)
+    wall |= n.A[d] < 2 || n.A[d] > g.n[d] - 3;
+  if (NDIM == 2 && !__any(wall)) {
+    Q around[3][3][NDIM]; // [axis 0][axis 1]
+    T gc[corners<NDIM>()];
 #pragma unroll
-    for (int d = 0; d < NDIM; ++d) {
-      const int e = ((c >> d) & 1) - 1; // the cell's low corner, from the node
-      inside &= A[d] + e >= 1 && A[d] + e <= g.n[d] - 3;
-      base += e * g.s[d];
+    for (int c = 0; c < corners<NDIM>(); ++c)
+      gc[c] = at_bytes<T>(cell + corner_step<NDIM>(g, corners<NDIM>() - 1 - c, 0), n.nat);
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+      for (int s = 0; s < 3; ++s)
+#pragma unroll
+        for (int j = 0; j < NDIM; ++j)
+          around[r][s][j] = at_bytes<Q>(
+              u1 + (j * comp + (int64_t)((r - 1) * g.s[0] + (s - 1) * g.s[1]) * g.lanes), n.at);
+#pragma unroll
+    for (int c = 0; c < corners<NDIM>(); ++c) {
+      const int self = corners<NDIM>() - 1 - c; // the node's corner in the cell
+#pragma unroll
+      for (int l = 0; l < corners<NDIM>(); ++l)
+#pragma unroll
+        for (int j = 0; j < NDIM; ++j) {
+          const Q uj = around[(c & 1) + (l & 1)][((c >> 1) & 1) + ((l >> 1) & 1)][j];
+#pragma unroll
+          for (int i = 0; i < NDIM; ++i)
+            force[i] = force[i] - (gc[c] * K[(self * NDIM + i) * NL + l * NDIM + j]) * uj;
+        }
     }
-    if (!inside)
-      continue;
-    const int self = corners<NDIM>() - 1 - c; // the node's corner in the cell
-    const T gc = cell[idx + base];
+  } else {
 #pragma unroll
-    for (int l = 0; l < corners<NDIM>(); ++l) {
-      int off = base;
+    for (int c = 0; c < corners<NDIM>(); ++c) {
+      bool inside = true;
 #pragma unroll
-      for (int d = 0; d < NDIM; ++d)
-        off += ((l >> d) & 1) * g.s[d];
+      for (int d = 0; d < NDIM; ++d) {
+        const int e = ((c >> d) & 1) - 1; // the cell's low corner, from the node
+        inside &= n.A[d] + e >= 1 && n.A[d] + e <= g.n[d] - 3;
+      }
+      if (!inside)
+        continue;
+      const int self = corners<NDIM>() - 1 - c; // the node's corner in the cell
+      const T gc = at_bytes<T>(cell + corner_step<NDIM>(g, self, 0), n.nat);
 #pragma unroll
-      for (int j = 0; j < NDIM; ++j) {
-        const Q uj = lanes_at<Q>(v, j * comp + (int64_t)off * g.lanes);
+      for (int l = 0; l < corners<NDIM>(); ++l) {
+        const int64_t off = (int64_t)corner_step<NDIM>(g, self, l) * g.lanes;
 #pragma unroll
-        for (int i = 0; i < NDIM; ++i)
-          force[i] = force[i] - (gc * K[(self * NDIM + i) * NL + l * NDIM + j]) * uj;
+        for (int j = 0; j < NDIM; ++j) {
+          const Q uj = at_bytes<Q>(u1 + (j * comp + off), n.at);
+#pragma unroll
+          for (int i = 0; i < NDIM; ++i)
+            force[i] = force[i] - (gc * K[(self * NDIM + i) * NL + l * NDIM + j]) * uj;
+        }
       }
     }
   }
-  const T mi = minv[idx];
+  const T mi = at_bytes<T>(minv, n.nat);
   // with a damping field the damped update (anisotropic.cu:380-389), nodal beta
-  const T beta = damping ? (T)0.5 * mi * damping[idx] * dt : (T)0;
+  const T beta = damping ? (T)0.5 * mi * damping[n.idx] * dt : (T)0;
 #pragma unroll
   for (int i = 0; i < NDIM; ++i) {
-    const int64_t at = (i * g.nodes + idx) * g.lanes + lane0;
-    const Q w0 = lanes_at<Q>(u0, at), w1 = lanes_at<Q>(u1, at);
+    const Q w0 = at_bytes<Q>(u0 + i * comp, n.at), w1 = at_bytes<Q>(u1 + i * comp, n.at);
     const Q next = damping ? ((T)2 * w1 - w0 * ((T)1 - beta) + g.f * mi * force[i]) / ((T)1 + beta)
                            : -w0 + (T)2 * w1 + (g.f * mi) * force[i];
-    lanes_put(u2, at, next);
+    put_bytes(u2 + i * comp, n.at, next);
   }
 }
 
@@ -137,55 +197,45 @@ an_gradient(AnGeom<T> g, const T *__restrict__ K, T *__restrict__ g_mass,
             const T *__restrict__ u2, const T *__restrict__ l1, T mass_factor) {
   using Q = LanesOf<T, V>;
   constexpr int NL = nloc<NDIM>();
-  int A[3];
-  int64_t idx;
-  int lane0;
-  if (!an_node<NDIM, V>(g, A, &idx, &lane0))
+  AnNode<NDIM, T> n;
+  if (!an_node<NDIM, V>(g, n))
     return;
   const int64_t comp = g.nodes * g.lanes;
-  const int64_t e = idx * g.lanes + lane0;
   Q acc = (T)0;
 #pragma unroll
-  for (int i = 0; i < NDIM; ++i) {
-    const int64_t at = i * comp + e;
-    acc = acc + lanes_at<Q>(l1, at) *
-                    (lanes_at<Q>(u2, at) - (T)2 * lanes_at<Q>(u1, at) + lanes_at<Q>(u0, at));
-  }
+  for (int i = 0; i < NDIM; ++i)
+    acc = acc + at_bytes<Q>(l1 + i * comp, n.at) *
+                    (at_bytes<Q>(u2 + i * comp, n.at) - (T)2 * at_bytes<Q>(u1 + i * comp, n.at) +
+                     at_bytes<Q>(u0 + i * comp, n.at));
   const T mass = cw::shot_sum(mass_factor * acc, g.lanes);
   bool own = true;
 #pragma unroll
   for (int d = 0; d < NDIM; ++d)
-    own &= A[d] <= g.n[d] - 3;
+    own &= n.A[d] <= g.n[d] - 3;
   Q bilinear = (T)0;
   if (own) {
 #pragma unroll
     for (int l = 0; l < corners<NDIM>(); ++l) {
-      int lo = 0;
-#pragma unroll
-      for (int d = 0; d < NDIM; ++d)
-        lo += ((l >> d) & 1) * g.s[d];
+      const int64_t lo = (int64_t)corner_step<NDIM>(g, 0, l) * g.lanes;
 #pragma unroll
       for (int m = 0; m < corners<NDIM>(); ++m) {
-        int mo = 0;
-#pragma unroll
-        for (int d = 0; d < NDIM; ++d)
-          mo += ((m >> d) & 1) * g.s[d];
+        const int64_t mo = (int64_t)corner_step<NDIM>(g, 0, m) * g.lanes;
 #pragma unroll
         for (int i = 0; i < NDIM; ++i)
 #pragma unroll
           for (int j = 0; j < NDIM; ++j)
-            bilinear = bilinear + (lanes_at<Q>(l1, i * comp + e + (int64_t)lo * g.lanes) *
+            bilinear = bilinear + (at_bytes<Q>(l1 + (i * comp + lo), n.at) *
                                    K[(l * NDIM + i) * NL + m * NDIM + j]) *
-                                      lanes_at<Q>(u1, j * comp + e + (int64_t)mo * g.lanes);
+                                      at_bytes<Q>(u1 + (j * comp + mo), n.at);
       }
     }
   }
   // every thread of the node takes part in both sums; one writer a node
   const T stiff = cw::shot_sum(bilinear, g.lanes);
-  if (lane0 == 0) {
-    g_mass[idx] -= mass;
+  if (n.lane0 == 0) {
+    g_mass[n.idx] -= mass;
     if (own)
-      g_cell[idx] -= stiff;
+      g_cell[n.idx] -= stiff;
   }
 }
 
