@@ -62,10 +62,11 @@ template <typename T> cwa::AnGeom<T> make_geom(const cw_aniso_grid &gr) {
   g.nodes = stride;
   g.lanes = gr.lanes;
   g.interior = 1;
-  for (int d = 0; d < gr.ndim; ++d) {
+  for (int d = 0; d < gr.ndim; ++d)
     g.interior *= gr.n[d] - 2;
-    g.by[d] = cw::make_div(gr.n[d] - 2);
-  }
+  g.row = cw::make_div(gr.n[gr.ndim - 1] - 2);
+  if (gr.ndim == 3)
+    g.stripes = cw::make_stripes(gr.n);
   g.f = (T)gr.step;
   return g;
 }

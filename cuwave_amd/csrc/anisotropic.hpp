@@ -40,7 +40,8 @@ template <typename T> struct AnGeom {
   int64_t nodes;  // nodes of one component
   int lanes;
   int interior;   // interior nodes, every axis 1 .. n - 2
-  cw::Div by[3];  // interior nodes of each axis
+  cw::Div row;    // interior nodes of the fast axis
+  cw::Stripes stripes; // 3D
   T f;            // the update factor dt^2 (the spacing sits in K)
 };
 
@@ -64,13 +65,14 @@ __device__ __forceinline__ bool an_node(const AnGeom<T> &g, AnNode<NDIM, T> &n) 
   if (i >= (uint32_t)g.interior)
     return false;
   n.lane0 = (int)(t & (per - 1)) * V;
-  uint32_t rest = i, k;
-#pragma unroll
-  for (int d = NDIM - 1; d > 0; --d) {
-    rest = cw::quot(g.by[d], rest, k);
-    n.A[d] = 1 + (int)k;
+  if (NDIM == 3) {
+    cw::stripe_node(g.stripes, i, n.A);
+  } else {
+    uint32_t k = i;
+    n.A[0] = 1 + (int)(NDIM == 2 ? cw::quot(g.row, i, k) : i);
+    if (NDIM == 2)
+      n.A[1] = 1 + (int)k;
   }
-  n.A[0] = 1 + (int)rest;
   int at = 0;
 #pragma unroll
   for (int d = 0; d < NDIM; ++d)

@@ -112,15 +112,9 @@ template <typename T> cw::Geom<T> make_geom(const cw_grid &gr) {
   g.interior = 1;
   for (int d = 0; d < nd; ++d)
     g.interior *= g.n[d] - 2;
-  const int64_t W = g.n[nd - 1] - 2;
-  g.row = cw::make_div(W);
-  if (nd == 3) {
-    const int H = g.n[1] - 2, rows = (H + cw::kXcds - 1) / cw::kXcds;
-    const int whole = H / rows; // stripes of `rows` rows; the last takes the rest
-    g.stripe = cw::make_div((int64_t)(g.n[0] - 2) * rows * W);
-    g.band = cw::make_div(rows * W);
-    g.last = cw::make_div((H - whole * rows) * W);
-  }
+  g.row = cw::make_div(g.n[nd - 1] - 2);
+  if (nd == 3)
+    g.stripes = cw::make_stripes(g.n);
   for (int k = 0; k < 4; ++k)
     g.op[k] = (T)gr.op[k];
   for (int d = 0; d < 3; ++d)

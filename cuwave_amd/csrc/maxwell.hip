@@ -69,10 +69,11 @@ template <typename T> cwm::MxGeom<T> make_geom(const cw_maxwell_grid &gr, const 
   g.lanes = gr.lanes;
   g.conductor = gr.conductor;
   g.interior = 1;
-  for (int d = 0; d < gr.ndim; ++d) {
+  for (int d = 0; d < gr.ndim; ++d)
     g.interior *= gr.n[d] - 2;
-    g.by[d] = cw::make_div(gr.n[d] - 2);
-  }
+  g.row = cw::make_div(gr.n[gr.ndim - 1] - 2);
+  if (gr.ndim == 3)
+    g.stripes = cw::make_stripes(gr.n);
   for (int k = 0; k < 4; ++k)
     g.sg[k] = (T)gr.stag[k];
   g.nu = (T)gr.nu;

@@ -537,25 +537,14 @@ __device__ __forceinline__ bool general_node(const Region &r, const Geom<T> &g,
   const int t = xcd_tile(bid, nb) * per + (int)(threadIdx.x >> ts);
   if (t >= g.interior)
     return false;
-  uint32_t rest, k;
   if (NDIM == 1) {
     a[0] = 1 + t;
   } else if (NDIM == 2) {
+    uint32_t k;
     a[0] = 1 + (int)quot(g.row, t, k);
     a[1] = 1 + (int)k;
   } else {
-    // the rows cut into kXcds stripes, a stripe's nodes in (plane, row,
-    // column) order: the run of items an XCD takes is one stripe marched
-    // plane by plane, so the planes the slow-axis taps read (R either side)
-    // are the stripe's share of them, which its L2 holds (whole planes it
-    // would not)
-    const int H = g.n[1] - 2, hs = (H + kXcds - 1) / kXcds;
-    const int stripe = (int)quot(g.stripe, t, rest);
-    const Div &plane = (stripe + 1) * hs <= H ? g.band : g.last;
-    uint32_t in;
-    a[0] = 1 + (int)quot(plane, rest, in);
-    a[1] = 1 + stripe * hs + (int)quot(g.row, in, k);
-    a[2] = 1 + (int)k;
+    stripe_node(g.stripes, t, a);
   }
   return true;
 }
