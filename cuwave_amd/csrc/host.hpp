@@ -28,9 +28,9 @@ inline int hip_status(const char *where) {
   return 0;
 }
 
-// The second stream a 2D sweep runs its edge launches on, beside the core
+// The second stream a 2D sweep runs its general launches on, beside the core
 // launches on the caller's stream, and the two events that order them. A
-// step's core and edge launches write disjoint nodes and read only levels
+// step's core and general launches write disjoint nodes and read only levels
 // the step before finished, so each waits only for the other's previous
 // step. The stream is non-blocking, so the legacy null stream does not
 // serialise it.
@@ -204,37 +204,22 @@ inline cw::Box stream_box(const cw_grid &g, const cw_pml &pml) {
   box.y1 = hi[0];
   box.x0 = lo[1];
   box.x1 = hi[1];
-  // every block of the box is a core block: the second launch's stream
-  // blocks are those holding sources or sensors
   const int C = cw::kThreads / g.lanes;
   const int xa = box.x0 / C * C;
-  box.c0 = 0;
-  box.c1 = (box.y1 - box.y0 + box.chunk - 1) / box.chunk;
-  box.k0 = 0;
-  box.k1 = (box.x1 - xa + C - 1) / C;
+  box.nc = (box.y1 - box.y0 + box.chunk - 1) / box.chunk;
+  box.nk = (box.x1 - xa + C - 1) / C;
   // a box of few blocks marches few long chunks, each one row at a time: a
   // small grid steps faster with one independent thread a node everywhere
-  if ((box.c1 - box.c0) * (box.k1 - box.k0) < stream_threshold())
+  if (box.nc * box.nk < stream_threshold())
     return cw::Box{0, 0, 0, 0, kChunk};
   return box;
 }
 
-// the stream blocks of a sweep, and of its core, each padded to a multiple
-// of the XCD count (the second launch's general blocks then start on XCD 0)
+// the core blocks of a sweep, padded to a multiple of the XCD count
 inline int pad_xcds(int blocks) {
   return (blocks + cw::kXcds - 1) / cw::kXcds * cw::kXcds;
 }
-inline int box_blocks(const cw::Box &b, int lanes) {
-  if (b.y0 >= b.y1)
-    return 0;
-  const int cols = cw::kThreads / lanes;
-  const int xa = b.x0 / cols * cols;
-  const int nchunk = (b.y1 - b.y0 + b.chunk - 1) / b.chunk;
-  return pad_xcds(nchunk * ((b.x1 - xa + cols - 1) / cols));
-}
-inline int core_blocks(const cw::Box &b) {
-  return pad_xcds((b.c1 - b.c0) * (b.k1 - b.k0));
-}
+inline int core_blocks(const cw::Box &b) { return pad_xcds(b.nc * b.nk); }
 
 // where the general kernels run: the band around the box, or every node
 inline cw::Region band_of(const cw_grid &g, const cw::Box &b) {

@@ -25,10 +25,15 @@
 // Blocks are dealt to the XCDs in contiguous runs, rows of blocks across
 // the box, so vertically neighbouring chunks share one L2.
 //
-// The box holds no layer node, so the core kernel carries no layer, point
-// or strip code. A box block holding a source or sensor runs in the second
-// launch of the step instead, with the point code (the layer code there is
-// never reached).
+// The box holds no layer node, so the core kernel carries no layer and no
+// strip code. It does carry the points: a block learns once which of its rows
+// hold any, and a row without skips them on one scalar bit. Blocks with points
+// used to run in the second launch, which tested every block of the box for
+// them and then marched the few 32 rows long on a nearly empty chip: on
+// 1090 x 1090 with 32 shots a step took 201 us and an adjoint level 421,
+// against 173 and 352 now (and 169 and 340 then with no point in the box).
+// The core needs 7 to 8 registers more for it, one wave a SIMD in the forward
+// step, which the memory rate does not show.
 //
 // The arithmetic is the general kernels' term by term, in the same order,
 // so both paths give the same bits; the cell weight of every node here is 1.
@@ -40,27 +45,25 @@ namespace cw {
 
 // The box of a sweep, rows [y0, y1) and columns [x0, x1), cut into blocks
 // of `chunk` rows by C columns (the first block column starting at the
-// multiple of C below x0). Blocks [c0, c1) x [k0, k1) are the core, which
-// the core kernel runs; with the box layer-free that is every block, and
-// the blocks holding points are handed to the second launch.
+// multiple of C below x0), nc by nk of them.
 struct Box {
   int y0, y1, x0, x1;
   int chunk;
-  int c0, c1, k0, k1;
+  int nc, nk;
 };
 
 // whether a point list holds a point in the tiles of rows [ya, yb) at tile
-// columns [tx0, tx1]: looked up once a block, so rows without points
-// (nearly all) skip the lists without waiting on a load
+// column tx: looked up once a block, so blocks without points (nearly all)
+// wait for one load of each list
 template <typename T>
 __device__ __forceinline__ bool chunk_has(const Points<T> &pts,
                                           const Geom<T> &g, int ya, int yb,
-                                          int tx0, int tx1) {
+                                          int tx) {
   if (!pts.starts)
     return false;
   int any = 0;
   for (int ty = ya / TileShape<2>::TY; ty <= (yb - 1) / TileShape<2>::TY; ++ty)
-    any |= pts.starts[ty * g.tf + tx1 + 1] - pts.starts[ty * g.tf + tx0];
+    any |= pts.starts[ty * g.tf + tx + 1] - pts.starts[ty * g.tf + tx];
   return __builtin_amdgcn_readfirstlane(any) != 0;
 }
 
@@ -89,44 +92,18 @@ __device__ __forceinline__ uint32_t point_rows(const Points<T> &pts,
   return __builtin_amdgcn_readfirstlane(mask);
 }
 
-// stream block `bid` of `nb` (a multiple of the XCD count) of the core or
-// of the second launch: its rows [ya, yb) and first column xb, or false for a
-// block the other kernel runs (or a padding block). A block starts at a
+// stream block `bid` of `nb` (a multiple of the XCD count): its rows [ya, yb)
+// and first column xb, or false for a padding block. A block starts at a
 // multiple of its width, so no wave straddles a point tile.
-template <bool EDGE, typename T>
-__device__ __forceinline__ bool box_item(const Box &box, const Geom<T> &g,
-                                         const Points<T> &src, bool use_src,
-                                         const Points<T> &rec, int cols,
-                                         int bid, int nb, int &ya, int &yb,
-                                         int &xb) {
-  const int xa = box.x0 / cols * cols;
-  const int ncx = (box.x1 - xa + cols - 1) / cols;
-  const int nchunk = (box.y1 - box.y0 + box.chunk - 1) / box.chunk;
+__device__ __forceinline__ bool box_item(const Box &box, int cols, int bid,
+                                         int nb, int &ya, int &yb, int &xb) {
   const int w = xcd_tile(bid, nb);
-  int c, k;
-  if (EDGE) {
-    if (w >= nchunk * ncx)
-      return false;
-    c = w / ncx;
-    k = w % ncx;
-  } else {
-    const int kw = box.k1 - box.k0;
-    if (w >= (box.c1 - box.c0) * kw)
-      return false;
-    c = box.c0 + w / kw;
-    k = box.k0 + w % kw;
-  }
-  ya = box.y0 + c * box.chunk;
+  if (w >= box.nc * box.nk)
+    return false;
+  ya = box.y0 + w / box.nk * box.chunk;
   yb = min(ya + box.chunk, box.y1);
-  xb = xa + k * cols;
-  const bool core = c >= box.c0 && c < box.c1 && k >= box.k0 && k < box.k1;
-  if (EDGE && !core)
-    return true;
-  const int tx0 = xb / TileShape<2>::TX;
-  const int tx1 = min(xb + cols - 1, g.np[1] - 1) / TileShape<2>::TX;
-  const bool points = (use_src && chunk_has(src, g, ya, yb, tx0, tx1)) ||
-                      chunk_has(rec, g, ya, yb, tx0, tx1);
-  return EDGE == points;
+  xb = box.x0 / cols * cols + w % box.nk * cols;
+  return true;
 }
 
 // Copy `bytes` contiguous bytes from global `src` to LDS `dst` by DMA, the
@@ -179,7 +156,7 @@ __device__ __forceinline__ void stage_nodes(const T *a, int64_t node, int count,
 }
 
 // --------------------------------------------------------------- forward
-template <typename T, int R, int W, bool EDGE, bool ILLUM>
+template <typename T, int R, int W, bool ILLUM>
 __device__ __forceinline__ void forward_stream(const FwdParams<T> &p,
                                                const Box &box, const int t,
                                                int bid, int nb) {
@@ -187,7 +164,7 @@ __device__ __forceinline__ void forward_stream(const FwdParams<T> &p,
   constexpr int SH = S::SH, C = S::C;
   const Geom<T> &g = p.g;
   int ya, yb, xb;
-  if (!box_item<EDGE>(box, g, p.src, true, p.rec, C, bid, nb, ya, yb, xb))
+  if (!box_item(box, C, bid, nb, ya, yb, xb))
     return;
   // the staged rows of u^(t-1), and per material row slot (two alternating)
   // the slow-axis cells [C], the fast-axis cells of x - 1 .. [C + 1], 1 / m
@@ -208,8 +185,8 @@ __device__ __forceinline__ void forward_stream(const FwdParams<T> &p,
   // this thread's element at row ya, and its row stride
   const uint32_t frow = ((uint32_t)s0 << SH) * sizeof(T);
   const uint32_t e0 = ((((uint32_t)ya * s0 + xl) << SH) + b) * sizeof(T);
-  const bool has_src = EDGE && chunk_has(p.src, g, ya, yb, tx, tx);
-  const bool has_rec = EDGE && chunk_has(p.rec, g, ya, yb, tx, tx);
+  const bool has_src = chunk_has(p.src, g, ya, yb, tx);
+  const bool has_rec = chunk_has(p.rec, g, ya, yb, tx);
   const uint32_t src_rows = has_src ? point_rows(p.src, g, ya, yb, tx) : 0u;
   const uint32_t rec_rows = has_rec ? point_rows(p.rec, g, ya, yb, tx) : 0u;
   const int lane0 = ((xc + R) * W + b); // this thread in a staged row
@@ -297,7 +274,7 @@ __device__ __forceinline__ void forward_stream(const FwdParams<T> &p,
 }
 
 // --------------------------------------------------------------- adjoint
-template <typename T, int R, int W, bool STIFF, bool EDGE>
+template <typename T, int R, int W, bool STIFF>
 __device__ __forceinline__ void backward_stream(const BwdParams<T> &p,
                                                 const Box &box, const int n,
                                                 int bid, int nb) {
@@ -306,7 +283,7 @@ __device__ __forceinline__ void backward_stream(const BwdParams<T> &p,
   const Geom<T> &g = p.g;
   const bool reverse = p.reverse && n <= p.steps - 2;
   int ya, yb, xb;
-  if (!box_item<EDGE>(box, g, p.src, reverse, p.rec, C, bid, nb, ya, yb, xb))
+  if (!box_item(box, C, bid, nb, ya, yb, xb))
     return;
   // the staged rows of lambda^(n+1) and u^n; per material row slot the
   // fast-axis cells of x - R .. [C + 2R], 1 / m [C] and the slow-axis cell
@@ -338,8 +315,8 @@ __device__ __forceinline__ void backward_stream(const BwdParams<T> &p,
   const uint32_t e0 = ((((uint32_t)ya * s0 + xl) << SH) + b) * sizeof(T);
   const uint32_t n0 = ((uint32_t)ya * s0 + xl) * sizeof(T);
   const uint32_t nrow = (uint32_t)s0 * sizeof(T);
-  const bool has_rec = EDGE && chunk_has(p.rec, g, ya, yb, tx, tx);
-  const bool has_src = EDGE && reverse && chunk_has(p.src, g, ya, yb, tx, tx);
+  const bool has_rec = chunk_has(p.rec, g, ya, yb, tx);
+  const bool has_src = reverse && chunk_has(p.src, g, ya, yb, tx);
   const uint32_t rec_rows = has_rec ? point_rows(p.rec, g, ya, yb, tx) : 0u;
   const uint32_t src_rows = has_src ? point_rows(p.src, g, ya, yb, tx) : 0u;
   const int lane0 = ((xc + R) * W + b);
@@ -518,11 +495,9 @@ __device__ __forceinline__ void backward_stream(const BwdParams<T> &p,
 }
 
 // ------------------------------------------------------------ the steps
-// The edge launch of a step: the first `streams` blocks (a multiple of the
-// XCD count) march the stream box's blocks that hold sources or sensors,
-// the rest take the general nodes (the 2D frame around the box, or every
-// node in 1D and 3D), V shot lanes a thread. W is the shot lanes of a node
-// for the stream blocks (0 where there are none).
+// The second launch of a step takes the general nodes: the 2D frame around
+// the box, or every node in 1D and 3D (and in 2D without a box), V shot lanes
+// a thread.
 // the step a launch makes: `t`, offset by the device clock where one is given
 // (-1 outside 0 .. t_end - 1: the launch does nothing)
 template <typename T>
@@ -533,22 +508,13 @@ __device__ __forceinline__ int clocked_step(const FwdParams<T> &p, int t) {
   return tc >= 0 && tc < p.t_end ? tc : -1;
 }
 
-template <typename T, int NDIM, int R, int W, int V>
+template <typename T, int NDIM, int R, int V>
 __global__ __launch_bounds__(kThreads) void forward_step(const FwdParams<T> p,
-                                                         const Box box,
-                                                         const int step,
-                                                         const int streams) {
+                                                         const int step) {
   const int t = clocked_step(p, step);
   if (t < 0)
     return;
-  if constexpr (NDIM == 2 && W > 0) {
-    if ((int)blockIdx.x < streams) {
-      forward_stream<T, R, W, true, true>(p, box, t, blockIdx.x, streams);
-      return;
-    }
-  }
-  forward_general<T, NDIM, R, V>(p, t, blockIdx.x - streams,
-                                 gridDim.x - streams);
+  forward_general<T, NDIM, R, V>(p, t, blockIdx.x, gridDim.x);
 }
 
 // a step of a grid under a domain mask: every interior node by the general
@@ -566,28 +532,14 @@ __global__ __launch_bounds__(kThreads) void forward_masked(const FwdParams<T> p,
 // then just fit four waves a SIMD (the default packing left it one register
 // over, at three), which measured 18 % faster; every other build keeps the
 // default, as a tighter budget would make it spill.
-#ifndef CW_FRAME_BLOCKS_2D
-#define CW_FRAME_BLOCKS_2D 1
-#endif
-template <typename T, int NDIM, int R, int W, int V, bool STIFF>
+template <typename T, int NDIM, int R, int V>
 __global__ __launch_bounds__(kThreads,
-                             NDIM == 3 && V == 1 && sizeof(T) == 4 ? 4
-                             : NDIM == 2 && sizeof(T) == 4 ? CW_FRAME_BLOCKS_2D : 1) void backward_step(
-    const BwdParams<T> p,
-                                                          const Box box,
-                                                          const int n,
-                                                          const int streams) {
-  if constexpr (NDIM == 2 && W > 0) {
-    if ((int)blockIdx.x < streams) {
-      backward_stream<T, R, W, STIFF, true>(p, box, n, blockIdx.x, streams);
-      return;
-    }
-  }
-  backward_general<T, NDIM, R, V>(p, n, blockIdx.x - streams,
-                                  gridDim.x - streams);
+                             NDIM == 3 && V == 1 && sizeof(T) == 4 ? 4 : 1)
+void backward_step(const BwdParams<T> p, const int n) {
+  backward_general<T, NDIM, R, V>(p, n, blockIdx.x, gridDim.x);
 }
 
-// the core blocks of a 2D step: no layer, no wall, no point, no strip;
+// the core blocks of a 2D step: no layer, no wall, no strip;
 // ILLUM builds in the illumination sum (a separate build, so a step that
 // does not gather it compiles as if it did not exist)
 template <typename T, int R, int W, bool ILLUM>
@@ -597,14 +549,14 @@ __global__ __launch_bounds__(kThreads) void forward_core(const FwdParams<T> p,
   const int t = clocked_step(p, step);
   if (t < 0)
     return;
-  forward_stream<T, R, W, false, ILLUM>(p, box, t, blockIdx.x, gridDim.x);
+  forward_stream<T, R, W, ILLUM>(p, box, t, blockIdx.x, gridDim.x);
 }
 
 template <typename T, int R, int W, bool STIFF>
 __global__ __launch_bounds__(kThreads) void backward_core(const BwdParams<T> p,
                                                           const Box box,
                                                           const int n) {
-  backward_stream<T, R, W, STIFF, false>(p, box, n, blockIdx.x, gridDim.x);
+  backward_stream<T, R, W, STIFF>(p, box, n, blockIdx.x, gridDim.x);
 }
 
 } // namespace cw

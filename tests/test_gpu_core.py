@@ -1,9 +1,8 @@
 """Grids large enough that a 2D sweep runs its core kernels, against the oracle.
 
 A 2D sweep launches two kernels a step: the core kernel streams the blocks
-of the stream box that hold no layer node, no node whose transposed taps
-reach a layer, and no source or sensor; the edge kernel takes every other
-node. The golden grids are too small to hold a core block, so these cases
+of the stream box, which hold no layer node and no node whose transposed
+taps reach a layer; the general kernel takes every other node. The golden grids are too small to hold a core block, so these cases
 build larger ones (sizes chosen so both kernels run, with points inside and
 outside the core rectangle) and compare with the oracle on the same inputs:
 
@@ -130,6 +129,41 @@ def test_a_batched_misfit_gradient_with_core_blocks_matches_the_oracle():
         driver.Sensors(osim, coords), observed)
     assert abs(cost - ocost) <= 1e-5 * abs(ocost)
     assert rel_max(gradient, ogradient) < F32_GRAD
+
+
+@pytest.mark.parametrize("Nx, precision, shots", [((134, 200), "float32", 5),
+                                                  ((100, 560), "float64", 1)])
+def test_points_along_the_edges_of_core_blocks_match_the_oracle(Nx, precision, shots):
+    from oracle import driver
+
+    z, sim, rng = _case(Nx, precision, 32, 19)
+    osim = oracle_sim(z)
+    print(f"case core points {precision} {Nx} {shots} shots", flush=True)
+    sig = rng.standard_normal((sim.N, 1)).astype(sim.np_dtype)
+    # the rows beside the box's first (38) and second block row (70), the columns
+    # beside a point tile (64, 128) and a one-lane block (256); several a node
+    rows, cols = (36, 37, 38, 39, 69, 70), (31, 32, 63, 64, 127, 128)
+    cols += (255, 256, 511, 512) if Nx[1] > 512 else ()
+    sensors = np.array([(r, c) for r in rows for c in cols] + [(38, 64)] * 3,
+                       dtype=np.int32).T
+    sources = [wave.Source(np.array([[rows[k]], [cols[k]]]), sig * (1 + k))
+               for k in range(shots)]
+    fields, records = wave.simulate_shots(sim, sources, z["indicator"], sensors)
+    for k, s in enumerate(sources):
+        f, r = driver.simulate(osim, s.position, s.signal, z["indicator"], sensors)
+        np.testing.assert_array_equal(host(fields[k]), f, err_msg=f"shot {k}")
+        np.testing.assert_array_equal(host(records[k]), r, err_msg=f"shot {k}")
+    # the adjoint, by the comparison and bounds of the batched gradient above
+    coords = sensors.T * np.asarray(sim.dx)
+    observed = [0.1 * rng.standard_normal((sim.N, len(coords))).astype(sim.np_dtype)
+                for _ in sources]
+    cost, gradient = utils.misfit_gradient(sim, sources, z["indicator"],
+                                           utils.Sensors(sim, coords), observed)
+    ocost, ogradient = driver.misfit_gradient(
+        osim, [(s.position, s.signal) for s in sources], z["indicator"],
+        driver.Sensors(osim, coords), observed)
+    assert abs(cost - ocost) <= 1e-5 * abs(ocost)
+    assert rel_max(gradient, ogradient) < (F32_GRAD if precision == "float32" else F64)
 
 
 def test_the_illumination_map_with_core_blocks_matches_the_oracle():
