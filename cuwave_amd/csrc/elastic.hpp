@@ -200,6 +200,37 @@ __device__ Q half_rows(const ElGeom<T> &g, const Line<T, Off> &L, int k, int lo,
                               });
 }
 
+// the stencils away from the walls, at a node (h = 0, of half-point values)
+// or at a half point (h = 1, of nodal ones)
+template <int NDIM, int R, typename Q, typename T, typename Off>
+__device__ __forceinline__ Q inner_derivative(const ElGeom<T> &g, const Line<T, Off> &L, int k,
+                                              int h) {
+  Q acc((T)0);
+#pragma unroll
+  for (int q = 1; q <= R; ++q)
+    acc += g.sg[q - 1] * (line_at<NDIM, Q>(L, k, q - 1 + h) - line_at<NDIM, Q>(L, k, h - q));
+  return acc;
+}
+template <int NDIM, int R, typename Q, typename T, typename Off>
+__device__ __forceinline__ Q inner_divergence(const ElGeom<T> &g, const Line<T, Off> &L, int k,
+                                              int h) {
+  Q acc((T)0);
+#pragma unroll
+  for (int q = 1; q <= R; ++q) {
+    acc += g.sg[q - 1] * line_at<NDIM, Q>(L, k, q - 1 + h);
+    acc -= g.sg[q - 1] * line_at<NDIM, Q>(L, k, h - q);
+  }
+  return acc;
+}
+
+// whether a wall of axis e is near: whether a derivative or divergence along
+// it may be a closure row, or one that is not there
+template <typename T>
+__device__ __forceinline__ bool near_wall(const ElGeom<T> &g, int a, int e) {
+  const int rows = g.nc > g.hc ? g.nc : g.hc, band = rows > 1 ? rows : 1;
+  return a - 1 < band || g.n[e] - 3 - a < band;
+}
+
 // d/dx at node a of a half-point field (common.cuh:247-258)
 template <int NDIM, int R, typename Q, typename T, typename Off>
 __device__ __forceinline__ Q node_derivative(const ElGeom<T> &g, const Line<T, Off> &L, int k, int a,
@@ -207,11 +238,7 @@ __device__ __forceinline__ Q node_derivative(const ElGeom<T> &g, const Line<T, O
   const int lo = a - 1, hi = N - 2 - a;
   if (lo < g.nc || hi < g.nc)
     return node_rows<NDIM, Q>(g, L, k, lo, hi);
-  Q acc((T)0);
-#pragma unroll
-  for (int q = 1; q <= R; ++q)
-    acc += g.sg[q - 1] * (line_at<NDIM, Q>(L, k, q - 1) - line_at<NDIM, Q>(L, k, -q));
-  return acc;
+  return inner_derivative<NDIM, R, Q>(g, L, k, 0);
 }
 
 // d/dx at half point a of a nodal field (common.cuh:261-271)
@@ -221,11 +248,7 @@ __device__ __forceinline__ Q half_derivative(const ElGeom<T> &g, const Line<T, O
   const int lo = a - 1, hi = N - 3 - a;
   if (lo < g.hc || hi < g.hc)
     return half_rows<NDIM, Q>(g, L, k, lo, hi);
-  Q acc((T)0);
-#pragma unroll
-  for (int q = 1; q <= R; ++q)
-    acc += g.sg[q - 1] * (line_at<NDIM, Q>(L, k, q) - line_at<NDIM, Q>(L, k, 1 - q));
-  return acc;
+  return inner_derivative<NDIM, R, Q>(g, L, k, 1);
 }
 
 // the divergence of a nodal stress at half point a (common.cuh:276-288)
@@ -235,13 +258,7 @@ __device__ __forceinline__ Q node_divergence(const ElGeom<T> &g, const Line<T, O
   const int lo = a - 1, hi = N - 3 - a;
   if (lo < g.hc || hi < g.hc)
     return half_rows<NDIM, Q>(g, L, k, lo, hi);
-  Q acc((T)0);
-#pragma unroll
-  for (int q = 1; q <= R; ++q) {
-    acc += g.sg[q - 1] * line_at<NDIM, Q>(L, k, q);
-    acc -= g.sg[q - 1] * line_at<NDIM, Q>(L, k, 1 - q);
-  }
-  return acc;
+  return inner_divergence<NDIM, R, Q>(g, L, k, 1);
 }
 
 // the divergence of a half-point stress at node a (common.cuh:292-304)
@@ -251,13 +268,7 @@ __device__ __forceinline__ Q half_divergence(const ElGeom<T> &g, const Line<T, O
   const int lo = a - 1, hi = N - 2 - a;
   if (lo < g.nc || hi < g.nc)
     return node_rows<NDIM, Q>(g, L, k, lo, hi);
-  Q acc((T)0);
-#pragma unroll
-  for (int q = 1; q <= R; ++q) {
-    acc += g.sg[q - 1] * line_at<NDIM, Q>(L, k, q - 1);
-    acc -= g.sg[q - 1] * line_at<NDIM, Q>(L, k, -q);
-  }
-  return acc;
+  return inner_divergence<NDIM, R, Q>(g, L, k, 0);
 }
 
 // -------------------------------------------------- strains and stresses
@@ -290,6 +301,35 @@ __device__ __forceinline__ Q strain_derivative(const ElGeom<T> &g, const L &line
   if (A[k] > g.n[k] - 3 || A[e] > g.n[e] - 3)
     return Q((T)0);
   return half_derivative<NDIM, R, Q>(g, line, k, A[e], g.n[e]);
+}
+
+// every derivative of u, D[k][e] = d u_k / d x_e: an axis with no wall near
+// takes its NDIM derivatives in one branch, so that the thread waits on memory
+// once for their taps and not once for each derivative. Latency bounds the
+// pair (a third of the instructions issued that could be): with the updates'
+// divergences and the layers' memories taken likewise, an update of 107 x 120 x
+// 131 with two shots went from 150 to 101 us and 136 to 91 registers, the
+// stresses of the same step from 116 to 98 us.
+template <int NDIM, int R, typename Q, typename T, typename Off>
+__device__ __forceinline__ void derivatives(const ElGeom<T> &g, const T *u, Off off, const int *A,
+                                            Q (*D)[NDIM]) {
+#pragma unroll
+  for (int e = 0; e < NDIM; ++e) {
+    const auto line = field_line(u, off, g, e);
+    if (near_wall(g, A[e], e)) {
+#pragma unroll
+      for (int k = 0; k < NDIM; ++k)
+        D[k][e] = strain_derivative<NDIM, R, Q>(g, line, k, e, A);
+    } else {
+#pragma unroll
+      for (int k = 0; k < NDIM; ++k)
+        D[k][e] = inner_derivative<NDIM, R, Q>(g, line, k, k != e);
+#pragma unroll
+      for (int k = 0; k < NDIM; ++k)
+        if (k != e && A[k] > g.n[k] - 3)
+          D[k][e] = Q((T)0);
+    }
+  }
 }
 
 // the normal strains of u at a node, zero on a traction wall (elastic.cu:121-141)
@@ -351,10 +391,10 @@ __device__ __forceinline__ void strains_of(const ElGeom<T> &g, const Q (*D)[NDIM
 }
 
 // the stresses of the strains (elastic.cu:236-263); the shear gamma of the
-// pair points comes prepared (`shear`: the pair rows of prep)
+// pair points comes prepared (`shear`: the node's pair rows of prep)
 template <int NDIM, typename Q, typename T>
 __device__ __forceinline__ void stress_of(const ElGeom<T> &g, const Q *eps, int zeroed, T gn,
-                                          const T *shear, int64_t idx, const int *A, Q *sig) {
+                                          const T *shear, const int *A, Q *sig) {
   const T lam = condensed_lame<NDIM>(g, zeroed);
   Q tr((T)0);
 #pragma unroll
@@ -368,8 +408,7 @@ __device__ __forceinline__ void stress_of(const ElGeom<T> &g, const Q *eps, int 
 #pragma unroll
     for (int l = k + 1; l < NDIM; ++l) {
       const int v = stress_row<NDIM>(k, l);
-      sig[v] = shear_point(g, k, l, A) ? shear[(v - NDIM) * g.nodes + idx] * g.mu * eps[v]
-                                       : Q((T)0);
+      sig[v] = shear_point(g, k, l, A) ? shear[v - NDIM] * g.mu * eps[v] : Q((T)0);
     }
 }
 
@@ -422,7 +461,7 @@ __device__ __forceinline__ void slab_geometry(const ElGeom<T> &g, int e, int lo,
 // the stresses of the memory strains t of axis e (elastic.cu:445-467)
 template <int NDIM, typename Q, typename T>
 __device__ __forceinline__ void add_stress(const ElGeom<T> &g, Q *sig, T gn, const T *shear,
-                                           int64_t idx, int e, const Q *t, const int *A) {
+                                           int e, const Q *t, const int *A) {
   const int zeroed = zeroed_axes<NDIM>(g, A);
   if (!((zeroed >> e) & 1)) {
     const T lam = condensed_lame<NDIM>(g, zeroed);
@@ -436,19 +475,19 @@ __device__ __forceinline__ void add_stress(const ElGeom<T> &g, Q *sig, T gn, con
   for (int k = 0; k < NDIM; ++k)
     if (k != e && A[k] <= g.n[k] - 3 && A[e] <= g.n[e] - 3) {
       const int v = stress_row<NDIM>(k, e);
-      sig[v] += shear[(v - NDIM) * g.nodes + idx] * g.mu * t[k];
+      sig[v] += shear[v - NDIM] * g.mu * t[k];
     }
 }
 
 // the strain memory of axis e (elastic.cu:486-528), D[k] = d u_k / d x_e
-template <int NDIM, int R, int V, typename T, typename Off>
-__device__ __forceinline__ void stress_memory(const ElGeom<T> &g, const ElLayer<T> &P, int e,
-                                              const T *u, const LanesOf<T, V> (*D)[NDIM], T gn,
-                                              const T *shear, int64_t idx, Off place, int lane0,
-                                              const int *A, LanesOf<T, V> *sig) {
+template <int NDIM, int R, int V, int e, typename T, typename Off>
+__device__ __forceinline__ void stress_memory(const ElGeom<T> &g, const ElLayer<T> &P, const T *u,
+                                              const LanesOf<T, V> (*D)[NDIM], T gn,
+                                              const T *shear, Off place, int lane0, const int *A,
+                                              LanesOf<T, V> *sig) {
   using Q = LanesOf<T, V>;
   const int a = A[e], lo = P.lo[e], hi = P.hi[e];
-  if (!in_slab<NDIM>(g, a, e, lo, hi, P.phase ? R : 0))
+  if (!(lo + hi) || !in_slab<NDIM>(g, a, e, lo, hi, P.phase ? R : 0))
     return;
   int64_t plane, size, off;
   slab_geometry<NDIM>(g, e, lo, hi, A, &plane, &size, &off);
@@ -476,37 +515,47 @@ __device__ __forceinline__ void stress_memory(const ElGeom<T> &g, const ElLayer<
   } else {
     const int64_t t = slab_at(a, N, lo, hi, e < NDIM - 1, plane, off);
     T *aux = P.aux[e] + lane0;
+    // the rows read before any is written: one wait for all
+    const T pn = prof[N + a], dn = prof[a], ph = prof[3 * N + a], dh = prof[2 * N + a];
+    Q m[NDIM];
+#pragma unroll
+    for (int k = 0; k < NDIM; ++k)
+      m[k] = lanes_at<Q>(aux, ((int64_t)k * size + t) * g.lanes);
 #pragma unroll
     for (int k = 0; k < NDIM; ++k) {
-      const int at = (k == e ? 0 : 2 * N) + a;
-      const int64_t m = ((int64_t)k * size + t) * g.lanes;
-      q[k] = prof[N + at] * lanes_at<Q>(aux, m) + prof[at] * (g.f[e] * D[k][e]);
-      lanes_put(aux, m, q[k]);
+      q[k] = (k == e ? pn : ph) * m[k] + (k == e ? dn : dh) * (g.f[e] * D[k][e]);
+      lanes_put(aux, ((int64_t)k * size + t) * g.lanes, q[k]);
     }
   }
-  add_stress<NDIM>(g, sig, gn, shear, idx, e, q, A);
+  add_stress<NDIM>(g, sig, gn, shear, e, q, A);
 }
 
-// the divergence memory of component c along axis e (elastic.cu:532-573),
-// `term` the divergence term itself (the forward's)
-template <int NDIM, int R, int V, typename T, typename Off>
-__device__ __forceinline__ LanesOf<T, V> force_memory(const ElGeom<T> &g, const ElLayer<T> &P,
-                                                      const T *sigma, const LanesOf<T, V> &term,
-                                                      const LanesOf<T, V> &u1, Off place,
-                                                      int lane0, int c, int e, const int *A) {
+// the divergence memories of axis e (elastic.cu:532-573) into the components'
+// updates, D[c] the divergences of the axis; `on`: the components that have
+// their point here
+template <int NDIM, int R, int V, int e, typename T, typename Off>
+__device__ __forceinline__ void force_memory(const ElGeom<T> &g, const ElLayer<T> &P,
+                                             const T *sigma, const LanesOf<T, V> (*D)[NDIM],
+                                             const LanesOf<T, V> *w1, const T *mi, const bool *on,
+                                             Off place, int lane0, const int *A,
+                                             LanesOf<T, V> *next) {
   using Q = LanesOf<T, V>;
   const int a = A[e], lo = P.lo[e], hi = P.hi[e];
-  if (!in_slab<NDIM>(g, a, e, lo, hi, P.phase ? R : 0))
-    return Q((T)0);
+  if (!(lo + hi))
+    return;
+  if (!in_slab<NDIM>(g, a, e, lo, hi, P.phase ? R : 0)) {
+#pragma unroll
+    for (int c = 0; c < NDIM; ++c)
+      next[c] += mi[c] * Q((T)0);
+    return;
+  }
   int64_t plane, size, off;
   slab_geometry<NDIM>(g, e, lo, hi, A, &plane, &size, &off);
   const int N = g.n[e];
   const bool slow = e < NDIM - 1;
   const int64_t t = slab_at(a, N, lo, hi, slow, plane, off);
   const T *prof = P.profile[e];
-  const int at = (c == e ? 2 * N : 0) + a;
   T *aux = P.aux[e] + lane0;
-  const int64_t z = ((int64_t)(NDIM + c) * size + t) * g.lanes;
   if (P.phase) {
     Line<T, Off> k = field_line(sigma, place, g, e);
     k.stress = true;
@@ -523,14 +572,33 @@ __device__ __forceinline__ LanesOf<T, V> force_memory(const ElGeom<T> &g, const 
     k.N = N;
     k.own_half = false;
     k.slow = slow;
-    const Q back = g.f[e] * stress_divergence<NDIM, R, Q>(g, k, c, e, c, A);
-    if (t >= 0)
-      lanes_put(aux, z, prof[N + at] * (lanes_at<Q>(aux, z) + u1));
-    return back;
+#pragma unroll
+    for (int c = 0; c < NDIM; ++c) {
+      if (!on[c])
+        continue;
+      next[c] += mi[c] * (g.f[e] * stress_divergence<NDIM, R, Q>(g, k, c, e, c, A));
+      if (t >= 0) {
+        const int at = (c == e ? 3 * N : N) + a;
+        const int64_t z = ((int64_t)(NDIM + c) * size + t) * g.lanes;
+        lanes_put(aux, z, prof[at] * (lanes_at<Q>(aux, z) + w1[c]));
+      }
+    }
+    return;
   }
-  const Q next = prof[N + at] * lanes_at<Q>(aux, z) + prof[at] * term;
-  lanes_put(aux, z, next);
-  return next;
+  // the rows read before any is written: one wait for all
+  const T pn = prof[N + a], dn = prof[a], ph = prof[3 * N + a], dh = prof[2 * N + a];
+  Q m[NDIM];
+#pragma unroll
+  for (int c = 0; c < NDIM; ++c)
+    m[c] = lanes_at<Q>(aux, ((int64_t)(NDIM + c) * size + t) * g.lanes);
+#pragma unroll
+  for (int c = 0; c < NDIM; ++c) {
+    if (!on[c])
+      continue;
+    m[c] = (c == e ? ph : pn) * m[c] + (c == e ? dh : dn) * Q(g.f[e] * D[c][e]);
+    lanes_put(aux, ((int64_t)(NDIM + c) * size + t) * g.lanes, m[c]);
+    next[c] += mi[c] * m[c];
+  }
 }
 
 // the adjoint's strain memory settled into its other block (elastic.cu:577-595)
@@ -666,15 +734,14 @@ stress_node(const ElGeom<T> &g, const ElLayer<T> &P, const T *__restrict__ gamma
   using Q = LanesOf<T, V>;
   constexpr int NV = nvoigt<NDIM>();
   const auto place = place_of<NDIM>(g, idx, lane0);
-  const T *shear = prep + NDIM * g.nodes;
   const T gn = gamma[idx];
+  T shear[NV > NDIM ? NV - NDIM : 1]; // read at every node: used where the pair has its point
+#pragma unroll
+  for (int v = 0; v < NV - NDIM; ++v)
+    shear[v] = prep[(NDIM + v) * g.nodes + idx];
   // each derivative once: the strains and the forward's memory both read it
   Q D[NDIM][NDIM];
-#pragma unroll
-  for (int e = 0; e < NDIM; ++e)
-#pragma unroll
-    for (int k = 0; k < NDIM; ++k)
-      D[k][e] = strain_derivative<NDIM, R, Q>(g, field_line(u1, place, g, e), k, e, A);
+  derivatives<NDIM, R, Q>(g, u1, place, A, D);
   Q eps[NV], sig[NV];
   const int zeroed = zeroed_axes<NDIM>(g, A);
   strains_of<NDIM>(g, D, A, eps);
@@ -693,11 +760,14 @@ stress_node(const ElGeom<T> &g, const ElLayer<T> &P, const T *__restrict__ gamma
         take_off<T, V>(g_shear, (int64_t)(w - NDIM) * g.nodes + idx, d, g.lanes, lane0);
       }
   }
-  stress_of<NDIM, Q>(g, eps, zeroed, gn, shear, idx, A, sig);
-#pragma unroll
-  for (int e = 0; e < NDIM; ++e)
-    if (P.lo[e] + P.hi[e])
-      stress_memory<NDIM, R, V>(g, P, e, u1, D, gn, shear, idx, place, lane0, A, sig);
+  stress_of<NDIM, Q>(g, eps, zeroed, gn, shear, A, sig);
+  // the axis a constant of each: so large a loop is left rolled at the long
+  // stencils, and its arrays go to scratch memory
+  stress_memory<NDIM, R, V, 0>(g, P, u1, D, gn, shear, place, lane0, A, sig);
+  if constexpr (NDIM > 1)
+    stress_memory<NDIM, R, V, 1>(g, P, u1, D, gn, shear, place, lane0, A, sig);
+  if constexpr (NDIM > 2)
+    stress_memory<NDIM, R, V, 2>(g, P, u1, D, gn, shear, place, lane0, A, sig);
 #pragma unroll
   for (int w = 0; w < NV; ++w)
     put_bytes(sigma + w * (g.nodes * g.lanes), place, sig[w]);
@@ -725,37 +795,62 @@ update_node(const ElGeom<T> &g, const ElLayer<T> &P, const T *__restrict__ prep,
             const T *__restrict__ v1, T mf, const int *A, int64_t idx, int lane0) {
   using Q = LanesOf<T, V>;
   const auto place = place_of<NDIM>(g, idx, lane0);
+  // the node's own values (of every component: an update that has no point
+  // here is dropped), then the divergence of component c along axis e, once:
+  // the force (nodal_force, elastic.cu:281-303) and the forward's memory read
+  // it. As in `derivatives`, an axis with no wall near takes its divergences
+  // in one branch.
+  bool on[NDIM];
+  T mi[NDIM];
+  Q w0[NDIM], w1[NDIM], D[NDIM][NDIM], next[NDIM];
 #pragma unroll
   for (int c = 0; c < NDIM; ++c) {
-    if (A[c] > g.n[c] - 3)
-      continue;
-    // the force on component c at its point (nodal_force, elastic.cu:281-303),
-    // each divergence once: the forward's memory reads it too
-    Q D[NDIM];
+    const int64_t comp = c * (g.nodes * g.lanes);
+    on[c] = A[c] <= g.n[c] - 3;
+    mi[c] = prep[(int64_t)c * g.nodes + idx];
+    w0[c] = at_bytes<Q>(u0 + comp, place);
+    w1[c] = at_bytes<Q>(u1 + comp, place);
+  }
 #pragma unroll
-    for (int e = 0; e < NDIM; ++e)
-      D[e] = stress_divergence<NDIM, R, Q>(g, field_line(sigma, place, g, e), c, e,
-                                           stress_row<NDIM>(c, e), A);
-    Q force = g.f[c] * D[c];
+  for (int e = 0; e < NDIM; ++e) {
+    const auto line = field_line(sigma, place, g, e);
+    if (near_wall(g, A[e], e)) {
+#pragma unroll
+      for (int c = 0; c < NDIM; ++c)
+        D[c][e] = on[c] ? stress_divergence<NDIM, R, Q>(g, line, c, e, stress_row<NDIM>(c, e), A)
+                        : Q((T)0);
+    } else {
+#pragma unroll
+      for (int c = 0; c < NDIM; ++c)
+        D[c][e] = inner_divergence<NDIM, R, Q>(g, line, stress_row<NDIM>(c, e), c == e);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < NDIM; ++c) {
+    Q force = g.f[c] * D[c][c];
 #pragma unroll
     for (int l = 0; l < NDIM; ++l)
       if (l != c)
-        force = fmat(g.f[l], D[l], force);
-    const int64_t n = (int64_t)c * g.nodes + idx;
-    const int64_t comp = c * (g.nodes * g.lanes);
-    const T mi = prep[n];
-    const Q w0 = at_bytes<Q>(u0 + comp, place), w1 = at_bytes<Q>(u1 + comp, place);
-    Q next = -w0 + (T)2.f * w1 + mi * force;
+        force = fmat(g.f[l], D[c][l], force);
+    next[c] = -w0[c] + (T)2.f * w1[c] + mi[c] * force;
+  }
+  // the axis a constant of each, as in stress_node
+  force_memory<NDIM, R, V, 0>(g, P, sigma, D, w1, mi, on, place, lane0, A, next);
+  if constexpr (NDIM > 1)
+    force_memory<NDIM, R, V, 1>(g, P, sigma, D, w1, mi, on, place, lane0, A, next);
+  if constexpr (NDIM > 2)
+    force_memory<NDIM, R, V, 2>(g, P, sigma, D, w1, mi, on, place, lane0, A, next);
 #pragma unroll
-    for (int e = 0; e < NDIM; ++e)
-      if (P.lo[e] + P.hi[e])
-        next += mi * force_memory<NDIM, R, V>(g, P, sigma, Q(g.f[e] * D[e]), w1, place, lane0, c,
-                                              e, A);
+  for (int c = 0; c < NDIM; ++c) {
+    if (!on[c])
+      continue;
+    const int64_t comp = c * (g.nodes * g.lanes);
     if constexpr (GRAD) {
       const Q v = at_bytes<Q>(v1 + comp, place);
-      take_off<T, V>(g_mass, n, mf * v * (next - (T)2.f * w1 + w0), g.lanes, lane0);
+      take_off<T, V>(g_mass, (int64_t)c * g.nodes + idx,
+                     mf * v * (next[c] - (T)2.f * w1[c] + w0[c]), g.lanes, lane0);
     }
-    put_bytes(u2 + comp, place, next);
+    put_bytes(u2 + comp, place, next[c]);
   }
   if (P.phase) {
 #pragma unroll
