@@ -31,9 +31,7 @@
 // used to run in the second launch, which tested every block of the box for
 // them and then marched the few 32 rows long on a nearly empty chip: on
 // 1090 x 1090 with 32 shots a step took 201 us and an adjoint level 421,
-// against 173 and 352 now (and 169 and 340 then with no point in the box).
-// The core needs 7 to 8 registers more for it, one wave a SIMD in the forward
-// step, which the memory rate does not show.
+// against 173 and 333 now (and 169 and 340 then with no point in the box).
 //
 // The arithmetic is the general kernels' term by term, in the same order,
 // so both paths give the same bits; the cell weight of every node here is 1.
@@ -273,6 +271,19 @@ __device__ __forceinline__ void forward_stream(const FwdParams<T> &p,
   }
 }
 
+// The adjoint core's parameters as its rows with points read them: from the
+// kernel's argument memory (they are its first argument), where they are
+// needed. Read as `p` they are loaded at the start and kept in scalar registers
+// the march has not got, spilled to lanes of vector ones: 103 registers, four
+// waves a SIMD and 352 us a level of 1090 x 1090 with 32 shots, against 92 (with
+// the five waves asked for), and 333. The forward core keeps `p`: read late, it
+// has eight waves a SIMD for seven and takes 180 us a step for 173.
+template <typename P> __device__ __forceinline__ const P &late_params() {
+  auto q = (const __attribute__((address_space(4))) P *)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(q));
+  return *(const P *)q;
+}
+
 // --------------------------------------------------------------- adjoint
 template <typename T, int R, int W, bool STIFF>
 __device__ __forceinline__ void backward_stream(const BwdParams<T> &p,
@@ -315,10 +326,12 @@ __device__ __forceinline__ void backward_stream(const BwdParams<T> &p,
   const uint32_t e0 = ((((uint32_t)ya * s0 + xl) << SH) + b) * sizeof(T);
   const uint32_t n0 = ((uint32_t)ya * s0 + xl) * sizeof(T);
   const uint32_t nrow = (uint32_t)s0 * sizeof(T);
-  const bool has_rec = chunk_has(p.rec, g, ya, yb, tx);
-  const bool has_src = reverse && chunk_has(p.src, g, ya, yb, tx);
-  const uint32_t rec_rows = has_rec ? point_rows(p.rec, g, ya, yb, tx) : 0u;
-  const uint32_t src_rows = has_src ? point_rows(p.src, g, ya, yb, tx) : 0u;
+  const bool has_rec = chunk_has(late_params<BwdParams<T>>().rec, g, ya, yb, tx);
+  const bool has_src = reverse && chunk_has(late_params<BwdParams<T>>().src, g, ya, yb, tx);
+  const uint32_t rec_rows =
+      has_rec ? point_rows(late_params<BwdParams<T>>().rec, g, ya, yb, tx) : 0u;
+  const uint32_t src_rows =
+      has_src ? point_rows(late_params<BwdParams<T>>().src, g, ya, yb, tx) : 0u;
   const int lane0 = ((xc + R) * W + b);
 
   auto stage_mat = [&](int y) {
@@ -440,13 +453,15 @@ __device__ __forceinline__ void backward_stream(const BwdParams<T> &p,
         cs = cs - p.mf * gsum;
       }
       const int tile = (y / TileShape<2>::TY) * g.tf + tx;
-      if ((rec_rows >> (y - ya)) & 1u)
-        for (int k = p.rec.starts[tile]; k < p.rec.starts[tile + 1]; ++k)
-          if (p.rec.takes(k, nc, b)) {
-            const T load = p.rec.weight[k] * p.adjoint[p.rec.at(m, k, b)];
+      if ((rec_rows >> (y - ya)) & 1u) {
+        const BwdParams<T> &q = late_params<BwdParams<T>>();
+        for (int k = q.rec.starts[tile]; k < q.rec.starts[tile + 1]; ++k)
+          if (q.rec.takes(k, nc, b)) {
+            const T load = q.rec.weight[k] * q.adjoint[q.rec.at(m, k, b)];
             ln += load;
-            cm += -p.mf * uc * load;
+            cm += -q.mf * uc * load;
           }
+      }
       // the gradient as add_gradient forms it, stored below
       if (p.combine) {
         gm_new = accm + shot_sum(p.jm * cm + p.js * cs, W);
@@ -466,10 +481,12 @@ __device__ __forceinline__ void backward_stream(const BwdParams<T> &p,
         div[1] = flux<T, R>(ut1, chi1[0], clo1[0], g.op);
         const T lap = combine_axes<T, 2, R>(div, g.f);
         v = -o.uo + (T)2 * uc + mi * lap;
-        if ((src_rows >> (y - ya)) & 1u)
-          for (int k = p.src.starts[tile]; k < p.src.starts[tile + 1]; ++k)
-            if (p.src.takes(k, nc, b))
-              v += p.src.weight[k] * p.signal[p.src.at(n + 1, k, b)];
+        if ((src_rows >> (y - ya)) & 1u) {
+          const BwdParams<T> &q = late_params<BwdParams<T>>();
+          for (int k = q.src.starts[tile]; k < q.src.starts[tile + 1]; ++k)
+            if (q.src.takes(k, nc, b))
+              v += q.src.weight[k] * q.signal[q.src.at(n + 1, k, b)];
+        }
       }
     }
     // four stores every thread issues (off the box or without a value, out
@@ -553,7 +570,7 @@ __global__ __launch_bounds__(kThreads) void forward_core(const FwdParams<T> p,
 }
 
 template <typename T, int R, int W, bool STIFF>
-__global__ __launch_bounds__(kThreads) void backward_core(const BwdParams<T> p,
+__global__ __launch_bounds__(kThreads, sizeof(T) == 4 && !STIFF ? 5 : 1) void backward_core(const BwdParams<T> p,
                                                           const Box box,
                                                           const int n) {
   backward_stream<T, R, W, STIFF>(p, box, n, blockIdx.x, gridDim.x);
