@@ -73,15 +73,28 @@ __device__ __forceinline__ int64_t shifted(const Image &im, int64_t p, int tap) 
 
 // ------------------------------------------------------------ forward
 // One block: a tile of kTH x kTW pixels of one image and every output channel
-// (BN = cout, 32 / 64 / 128). What bounds it is the LDS, then HBM: a 32 -> 32
-// layer has 36 flops a byte of activations, so the input has to reach the
-// block once. The tile's input with its one-pixel halo is staged KC channels
-// at a time and read nine times from LDS, with the KC channels' weights beside
-// it; the nine taps need no further load and no barrier between them. A wave
-// holds RW rows of 32 pixels by NT tiles of 32 channels and keeps the RW + 2
-// input rows of a column shift in registers for the three taps that share
-// them, so a tap costs a wave NT weight reads and a third of RW + 2 input
-// reads for RW NT matrix instructions.
+// (BN = cout, 32 / 64 / 128). The sums run tap by tap, 16 channels an
+// instruction within a tap: a pre-activation within rounding of zero takes the
+// sign this order gives it, the ReLU's gradient follows that sign, and another
+// order turns some of them (a few in 1e8), each worth up to |dy w| in the
+// gradient at the input.
+//
+// So the tile's input with its one-pixel halo is staged once for all nine taps,
+// every channel of it (KC >= cin; past 128 channels the tile is staged again
+// for each tap, KC at a time), and the weights T taps at a time in two LDS
+// buffers in turn: the next taps' are in registers while these are multiplied,
+// one barrier a turn. KC is the least of 16, 32, 64 and 128 that holds cin
+// (channels past cin are zeros), T is 3 where that is 32 or less and a tap's
+// products are too few to cover a barrier. A wave holds RW rows of 32 pixels
+// by NT tiles of 32 channels: RW + NT 16-byte LDS reads a lane for RW NT matrix
+// instructions, which at two by two is the LDS's rate at the instructions' own.
+// A layer's three passes at 16 x 290 x 304, 64 -> 64: 0.72 ms, and 0.67 with
+// the taps innermost, whose sums are in another order.
+//
+// A plane of LDS holds eight channels of every staged pixel, so a wave's reads
+// are runs of 32 pixels; kPlane keeps the writes (a pixel's planes one after
+// the other) off each other's banks. The weights' channels are permuted by
+// their chunk for the same reason.
 //
 // The matrix instruction's rows are channels and its columns pixels, so a lane
 // ends with runs of four channels of one pixel; the two halves of the wave
@@ -96,15 +109,13 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
-// the 16-byte slot of chunk c of staged pixel p: the chunks of a pixel are
-// permuted by its place among 16, so 16 neighbouring pixels' same chunk sits
-// in 16 different slots of the 64 banks
-template <int S> __device__ __forceinline__ int staged(int p, int c) {
-  return p * S + (c ^ (S == 4 ? (p >> 2) & 3 : (p >> 3) & 1));
+// the 16-byte slots of an LDS plane: 16 / S modulo the 16 slots of the 64 banks
+template <int S> constexpr int plane_slots() {
+  return (kHaloPixels - 16 / S + 15) / 16 * 16 + 16 / S;
 }
 
-template <int BN, int KC>
-__global__ void __launch_bounds__(kThreads)
+template <int BN, int KC, int T>
+__global__ void __launch_bounds__(kThreads, 2)
 conv3x3_fwd(Image im, int tiles_x, int tiles_y, int cin, const uint4 *__restrict__ x,
             const uint4 *__restrict__ wt, const float *__restrict__ bias, int relu,
             uint16_t *__restrict__ y) {
@@ -112,14 +123,18 @@ conv3x3_fwd(Image im, int tiles_x, int tiles_y, int cin, const uint4 *__restrict
   constexpr int WN = BN == 128 ? 2 : 1;         // waves along the channels
   constexpr int RW = kTH * WN / 4;              // pixel rows a wave
   constexpr int NT = BN / WN / 32;              // channel tiles a wave
-  __shared__ uint4 sx[kHaloPixels * S];
-  __shared__ uint4 sw[9 * S * BN];              // [tap][chunk][channel]
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+  constexpr int kPlane = plane_slots<S>();
+  constexpr int kWeights = T * S * BN;          // chunks of weights a stage
+  constexpr int kMine = (kWeights + kThreads - 1) / kThreads;
+  __shared__ uint4 sx[S * kPlane];              // [chunk][pixel]
+  __shared__ uint4 sw[2][kWeights];             // [tap][chunk][channel ^ chunk]
+  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64, half = lane / 32;
   const int tile = cw::xcd_tile(blockIdx.x, gridDim.x);
   const int x0 = tile % tiles_x * kTW, y0 = tile / tiles_x % tiles_y * kTH;
   const int base = tile / (tiles_x * tiles_y) * im.h * im.w;  // the image's first pixel
   const int cin8 = cin / 8, krow8 = 9 * cin8;
   const int row0 = wave / WN * RW, n0 = wave % WN * (32 * NT);
+  const int chunks = T > 1 ? 1 : (cin + KC - 1) / KC, stages = 9 / T * chunks;
   f32x16 acc[RW][NT];
 #pragma unroll
   for (int i = 0; i < RW; ++i)
@@ -128,9 +143,7 @@ conv3x3_fwd(Image im, int tiles_x, int tiles_y, int cin, const uint4 *__restrict
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         acc[i][j][r] = 0.0f;
-  for (int c0 = 0; c0 < cin8; c0 += S) {
-    if (c0)
-      __syncthreads();
+  auto stage_input = [&](int c0) { // chunks c0 .. c0 + S - 1 of the tile and its halo
 #pragma unroll
     for (int k = 0; k < (kHaloPixels * S + kThreads - 1) / kThreads; ++k) {
       const int t = tid + k * kThreads;
@@ -138,46 +151,75 @@ conv3x3_fwd(Image im, int tiles_x, int tiles_y, int cin, const uint4 *__restrict
       const int py = y0 + p / kHaloW - 1, px = x0 + p % kHaloW - 1;
       if (p < kHaloPixels) {
         uint4 v = {0, 0, 0, 0};
-        if (py >= 0 && py < im.h && px >= 0 && px < im.w)
+        if (py >= 0 && py < im.h && px >= 0 && px < im.w && c0 + c < cin8)
           v = x[(int64_t)(base + py * im.w + px) * cin8 + c0 + c];
-        sx[staged<S>(p, c)] = v;
+        sx[c * kPlane + p] = v;
       }
     }
+  };
+  uint4 ahead[kMine];
+  auto fetch_weights = [&](int stage) {
+    const int tap0 = stage / chunks * T, c0 = stage % chunks * S;
 #pragma unroll
-    for (int k = 0; k < (9 * S * BN + kThreads - 1) / kThreads; ++k) {
+    for (int k = 0; k < kMine; ++k) {
       const int t = tid + k * kThreads;
       const int c = t % S, n = t / S % BN, tap = t / (S * BN);
-      if (tap < 9)
-        sw[(tap * S + c) * BN + n] = wt[n * krow8 + tap * cin8 + c0 + c];
+      ahead[k] = uint4{0, 0, 0, 0};
+      if (tap < T && c0 + c < cin8)
+        ahead[k] = wt[n * krow8 + (tap0 + tap) * cin8 + c0 + c];
     }
+  };
+  auto stage_weights = [&](int stage) {
+#pragma unroll
+    for (int k = 0; k < kMine; ++k) {
+      const int t = tid + k * kThreads;
+      const int c = t % S, n = t / S % BN, tap = t / (S * BN);
+      if (tap < T)
+        sw[stage & 1][(tap * S + c) * BN + (n ^ (c & 15))] = ahead[k];
+    }
+  };
+  fetch_weights(0);
+  stage_input(0);
+  stage_weights(0);
+  for (int stage = 0; stage < stages; ++stage) {
     __syncthreads();
+    if (stage + 1 < stages)
+      fetch_weights(stage + 1);
+    const int tap0 = stage / chunks * T;
+    const uint4 *weights = sw[stage & 1];
 #pragma unroll
-    for (int kk = 0; kk < KC / 16; ++kk) {
-      const int c = 2 * kk + lane / 32;
+    for (int t = 0; t < T; ++t) {
+      const uint4 *from = sx + (row0 + (tap0 + t) / 3) * kHaloW + lane % 32 + (tap0 + t) % 3;
 #pragma unroll
-      for (int dw = 0; dw < 3; ++dw) {
-        bf16x8 in[RW + 2];
+      for (int kk = 0; kk < KC / 16; ++kk) {
+        const int c = 2 * kk + half;
+        bf16x8 in[RW], w[NT];
 #pragma unroll
-        for (int i = 0; i < RW + 2; ++i)
-          in[i] = __builtin_bit_cast(
-              bf16x8, sx[staged<S>((row0 + i) * kHaloW + lane % 32 + dw, c)]);
+        for (int i = 0; i < RW; ++i)
+          in[i] = __builtin_bit_cast(bf16x8, from[c * kPlane + i * kHaloW]);
 #pragma unroll
-        for (int dh = 0; dh < 3; ++dh)
+        for (int j = 0; j < NT; ++j)
+          w[j] = __builtin_bit_cast(
+              bf16x8, weights[(t * S + c) * BN + ((n0 + 32 * j + lane % 32) ^ (c & 15))]);
 #pragma unroll
-          for (int j = 0; j < NT; ++j) {
-            const bf16x8 w = __builtin_bit_cast(
-                bf16x8, sw[((3 * dh + dw) * S + c) * BN + n0 + 32 * j + lane % 32]);
+        for (int i = 0; i < RW; ++i)
 #pragma unroll
-            for (int i = 0; i < RW; ++i)
-              acc[i][j] =
-                  __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, in[i + dh], acc[i][j], 0, 0, 0);
-          }
+          for (int j = 0; j < NT; ++j)
+            acc[i][j] =
+                __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[j], in[i], acc[i][j], 0, 0, 0);
       }
+    }
+    if (stage + 1 < stages) {
+      if (chunks > 1) {
+        __syncthreads(); // this stage's input has been read
+        stage_input((stage + 1) % chunks * S);
+      }
+      stage_weights(stage + 1);
     }
   }
   // epilogue: bias, activation, bfloat16; accumulator register r of a lane is
   // channel 8 (r / 4) + 4 (lane / 32) + r % 4 of pixel lane % 32
-  const int px = x0 + lane % 32, half = lane / 32;
+  const int px = x0 + lane % 32;
   const bool wide = (reinterpret_cast<uintptr_t>(y) & 15) == 0; // else two bytes a store
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
@@ -227,9 +269,21 @@ conv3x3_fwd(Image im, int tiles_x, int tiles_y, int cin, const uint4 *__restrict
 template <int BN, int KC>
 void launch_fwd(const cw_conv3x3_args &a, const Image &im, hipStream_t s) {
   const int tx = (a.w + kTW - 1) / kTW, ty = (a.h + kTH - 1) / kTH;
-  hipLaunchKernelGGL((conv3x3_fwd<BN, KC>), dim3(tx * ty * a.n), dim3(kThreads), 0, s, im, tx, ty,
-                     a.cin, (const uint4 *)a.x, (const uint4 *)a.weight, (const float *)a.bias,
-                     a.relu, (uint16_t *)a.y);
+  hipLaunchKernelGGL((conv3x3_fwd<BN, KC, KC <= 32 ? 3 : 1>), dim3(tx * ty * a.n), dim3(kThreads),
+                     0, s, im, tx, ty, a.cin, (const uint4 *)a.x, (const uint4 *)a.weight,
+                     (const float *)a.bias, a.relu, (uint16_t *)a.y);
+}
+
+template <int BN>
+void launch_fwd(const cw_conv3x3_args &a, const Image &im, hipStream_t s) {
+  if (a.cin <= 16)
+    launch_fwd<BN, 16>(a, im, s);
+  else if (a.cin <= 32)
+    launch_fwd<BN, 32>(a, im, s);
+  else if (a.cin <= 64)
+    launch_fwd<BN, 64>(a, im, s);
+  else
+    launch_fwd<BN, 128>(a, im, s);
 }
 
 // ------------------------------------------------------- backward weight
@@ -681,16 +735,10 @@ int cw_conv3x3_bf16_fwd(const cw_conv3x3_args *a, void *stream) {
     return fail("the forward needs x, weight and y");
   const Image im{a->n, a->h, a->w, (int64_t)a->n * a->h * a->w};
   const auto s = (hipStream_t)stream;
-  const bool wide = a->cin % 32 == 0;
   switch (a->cout) {
-  case 32:
-    wide ? launch_fwd<32, 32>(*a, im, s) : launch_fwd<32, 16>(*a, im, s);
-    break;
-  case 64:
-    launch_fwd<64, 16>(*a, im, s);
-    break;
-  default:
-    launch_fwd<128, 16>(*a, im, s);
+  case 32: launch_fwd<32>(*a, im, s); break;
+  case 64: launch_fwd<64>(*a, im, s); break;
+  default: launch_fwd<128>(*a, im, s); break;
   }
   return hip_status("conv3x3_fwd");
 }

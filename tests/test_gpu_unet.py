@@ -185,3 +185,51 @@ def test_the_output_layer_and_its_gradients(shape, outputs):
     assert _rel(ours[1].grad, ref[1].grad) < 1e-5
     assert _rel(ours[2].grad, ref[2].grad) < 1e-5
     assert _rel(ours[0].grad, ref[0].grad) < 4e-3
+
+
+def _summed(x, w, taps_first):
+    """The convolution with one product a 16-channel group (the others are zero), each
+    added in float32: tap by tap, or group by group."""
+    n, h, wd, cin = x.shape
+    cout = w.shape[0]
+    wide = torch.nn.functional.pad(x, (0, 0, 1, 1, 1, 1))
+    wk = w.reshape(cout, 9, cin)
+    acc = torch.zeros(n, h, wd, cout)
+    pairs = [(t, c) for t in range(9) for c in range(0, cin, 16)]
+    for t, c in pairs if taps_first else sorted(pairs, key=lambda p: p[1]):
+        at = wide[:, t // 3:t // 3 + h, t % 3:t % 3 + wd, c:c + 16]
+        term = at[..., None, :] * wk[:, t, c:c + 16]  # exact: eight bits by eight
+        acc = acc + term.sum(-1)                      # one of the sixteen is not zero
+    return acc
+
+
+@pytest.mark.parametrize("cin, cout", [(16, 32), (32, 32), (48, 64), (64, 64), (64, 128),
+                                       (128, 64), (128, 128), (160, 32)])
+def test_a_convolution_adds_its_terms_tap_by_tap(cin, cout):
+    print(f"case order {cin}->{cout}", flush=True)
+    g = torch.Generator().manual_seed(cin + cout)
+    h, w = 11, 45
+
+    def halves(*shape):  # products in quarters: a sum's rounding needs two bits below it
+        return torch.randint(-8, 9, shape, generator=g) * 0.5
+
+    keep = torch.zeros(cin, dtype=torch.bool)
+    keep[[c + (c // 16) % 16 for c in range(0, cin, 16)]] = True
+    x = halves(2, h, w, cin) * keep
+    weight = halves(cout, 9, cin) * keep
+    # a large term at the first tap and its negative at the last: every sum between is
+    # rounded to whole numbers, so the order of the others is in the result
+    x[..., 0] = 4096.0
+    weight[..., 0] = 0.0
+    weight[:, 0, 0], weight[:, 8, 0] = 2048.0, -2048.0
+    weight = weight.reshape(cout, 9 * cin)
+    ref, other = (_summed(x, weight, first) for first in (True, False))
+    if cin > 16:
+        assert float((ref.bfloat16() != other.bfloat16()).float().mean()) > 0.1
+    conv = unet.Conv3x3(cin, cout, False).cuda()
+    with torch.no_grad():
+        conv.weight.copy_(weight)
+        conv.bias.zero_()
+        y = conv(x.cuda().bfloat16())
+    # the same additions in the same order: the same bits
+    torch.testing.assert_close(y.cpu(), ref.bfloat16(), rtol=0, atol=0)
