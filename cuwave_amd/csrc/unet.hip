@@ -80,8 +80,7 @@ __device__ __forceinline__ int64_t shifted(const Image &im, int64_t p, int tap) 
 // gradient at the input.
 //
 // So the tile's input with its one-pixel halo is staged once for all nine taps,
-// every channel of it (KC >= cin; past 128 channels the tile is staged again
-// for each tap, KC at a time), and the weights T taps at a time in two LDS
+// every channel of it (KC >= cin), and the weights T taps at a time in two LDS
 // buffers in turn: the next taps' are in registers while these are multiplied,
 // one barrier a turn. KC is the least of 16, 32, 64 and 128 that holds cin
 // (channels past cin are zeros), T is 3 where that is 32 or less and a tap's
@@ -134,7 +133,6 @@ conv3x3_fwd(Image im, int tiles_x, int tiles_y, int cin, const uint4 *__restrict
   const int base = tile / (tiles_x * tiles_y) * im.h * im.w;  // the image's first pixel
   const int cin8 = cin / 8, krow8 = 9 * cin8;
   const int row0 = wave / WN * RW, n0 = wave % WN * (32 * NT);
-  const int chunks = T > 1 ? 1 : (cin + KC - 1) / KC, stages = 9 / T * chunks;
   f32x16 acc[RW][NT];
 #pragma unroll
   for (int i = 0; i < RW; ++i)
@@ -143,30 +141,15 @@ conv3x3_fwd(Image im, int tiles_x, int tiles_y, int cin, const uint4 *__restrict
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         acc[i][j][r] = 0.0f;
-  auto stage_input = [&](int c0) { // chunks c0 .. c0 + S - 1 of the tile and its halo
-#pragma unroll
-    for (int k = 0; k < (kHaloPixels * S + kThreads - 1) / kThreads; ++k) {
-      const int t = tid + k * kThreads;
-      const int c = t % S, p = t / S;
-      const int py = y0 + p / kHaloW - 1, px = x0 + p % kHaloW - 1;
-      if (p < kHaloPixels) {
-        uint4 v = {0, 0, 0, 0};
-        if (py >= 0 && py < im.h && px >= 0 && px < im.w && c0 + c < cin8)
-          v = x[(int64_t)(base + py * im.w + px) * cin8 + c0 + c];
-        sx[c * kPlane + p] = v;
-      }
-    }
-  };
   uint4 ahead[kMine];
   auto fetch_weights = [&](int stage) {
-    const int tap0 = stage / chunks * T, c0 = stage % chunks * S;
 #pragma unroll
     for (int k = 0; k < kMine; ++k) {
       const int t = tid + k * kThreads;
       const int c = t % S, n = t / S % BN, tap = t / (S * BN);
       ahead[k] = uint4{0, 0, 0, 0};
-      if (tap < T && c0 + c < cin8)
-        ahead[k] = wt[n * krow8 + (tap0 + tap) * cin8 + c0 + c];
+      if (tap < T && c < cin8)
+        ahead[k] = wt[n * krow8 + (stage * T + tap) * cin8 + c];
     }
   };
   auto stage_weights = [&](int stage) {
@@ -179,17 +162,28 @@ conv3x3_fwd(Image im, int tiles_x, int tiles_y, int cin, const uint4 *__restrict
     }
   };
   fetch_weights(0);
-  stage_input(0);
+#pragma unroll
+  for (int k = 0; k < (kHaloPixels * S + kThreads - 1) / kThreads; ++k) {
+    const int t = tid + k * kThreads;
+    const int c = t % S, p = t / S;
+    const int py = y0 + p / kHaloW - 1, px = x0 + p % kHaloW - 1;
+    if (p < kHaloPixels) {
+      uint4 v = {0, 0, 0, 0};
+      if (py >= 0 && py < im.h && px >= 0 && px < im.w && c < cin8)
+        v = x[(int64_t)(base + py * im.w + px) * cin8 + c];
+      sx[c * kPlane + p] = v;
+    }
+  }
   stage_weights(0);
-  for (int stage = 0; stage < stages; ++stage) {
+  for (int stage = 0; stage < 9 / T; ++stage) {
     __syncthreads();
-    if (stage + 1 < stages)
+    if (stage + 1 < 9 / T)
       fetch_weights(stage + 1);
-    const int tap0 = stage / chunks * T;
     const uint4 *weights = sw[stage & 1];
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-      const uint4 *from = sx + (row0 + (tap0 + t) / 3) * kHaloW + lane % 32 + (tap0 + t) % 3;
+      const uint4 *from = sx + (row0 + (stage * T + t) / 3) * kHaloW + lane % 32 +
+                          (stage * T + t) % 3;
 #pragma unroll
       for (int kk = 0; kk < KC / 16; ++kk) {
         const int c = 2 * kk + half;
@@ -209,13 +203,8 @@ conv3x3_fwd(Image im, int tiles_x, int tiles_y, int cin, const uint4 *__restrict
                 __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[j], in[i], acc[i][j], 0, 0, 0);
       }
     }
-    if (stage + 1 < stages) {
-      if (chunks > 1) {
-        __syncthreads(); // this stage's input has been read
-        stage_input((stage + 1) % chunks * S);
-      }
+    if (stage + 1 < 9 / T)
       stage_weights(stage + 1);
-    }
   }
   // epilogue: bias, activation, bfloat16; accumulator register r of a lane is
   // channel 8 (r / 4) + 4 (lane / 32) + r % 4 of pixel lane % 32
@@ -266,6 +255,84 @@ conv3x3_fwd(Image im, int tiles_x, int tiles_y, int cin, const uint4 *__restrict
   }
 }
 
+// What the tiles waste or don't hold: images of a few pixels a side, and more
+// channels than 128. One block: 128 pixels of the whole batch in memory order x
+// BN output channels, wave w the pixels 32 w .. 32 w + 31 and every channel, its
+// input gathered from memory once a tap, 16 channels a barrier: the same sums
+// in the same order.
+constexpr int kBM = 128; // pixels a flat block takes (4 waves x 32)
+constexpr int kBK = 16;  // reduction step: 16 channels of one tap
+
+template <int BN>
+__global__ void __launch_bounds__(kThreads)
+conv3x3_fwd_flat(Image im, int cin, const uint4 *__restrict__ x, const uint4 *__restrict__ wt,
+            const float *__restrict__ bias, int relu, uint16_t *__restrict__ y) {
+  __shared__ uint4 sa[2][kBM * 2];  // [m][k]: 16 bf16 a row, two uint4
+  __shared__ uint4 sb[2][BN * 2];   // [n][k]
+  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+  const int64_t m0 = (int64_t)blockIdx.x * kBM;
+  const int steps = 9 * (cin / kBK);
+  const int cin8 = cin / 8;      // uint4 chunks a pixel
+  const int krow8 = 9 * cin8;    // uint4 chunks a weight row
+  // the chunk this thread stages: pixel am, half ah; weight row bn, half bh
+  const int am = tid / 2, ah = tid % 2;
+  const int bn = tid / 2, bh = tid % 2;
+  uint4 ra = {0, 0, 0, 0}, rb = {0, 0, 0, 0};
+  auto load = [&](int s) {
+    const int tap = s / (cin / kBK), c0 = (s % (cin / kBK)) * kBK;
+    const int64_t p = m0 + am;
+    ra = uint4{0, 0, 0, 0};
+    if (p < im.pixels) {
+      const int64_t q = shifted(im, p, tap);
+      if (q >= 0)
+        ra = x[q * cin8 + c0 / 8 + ah];
+    }
+    if (bn < BN)
+      rb = wt[(int64_t)bn * krow8 + tap * cin8 + c0 / 8 + bh];
+  };
+  f32x16 acc[BN / 32];
+#pragma unroll
+  for (int j = 0; j < BN / 32; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      acc[j][r] = 0.0f;
+  load(0);
+  for (int s = 0; s < steps; ++s) {
+    const int buf = s & 1;
+    sa[buf][am * 2 + ah] = ra;
+    if (bn < BN)
+      sb[buf][bn * 2 + bh] = rb;
+    __syncthreads();
+    if (s + 1 < steps)
+      load(s + 1);
+    const uint4 a = sa[buf][(wave * 32 + lane % 32) * 2 + lane / 32];
+    const bf16x8 av = __builtin_bit_cast(bf16x8, a);
+#pragma unroll
+    for (int j = 0; j < BN / 32; ++j) {
+      const uint4 b = sb[buf][(j * 32 + lane % 32) * 2 + lane / 32];
+      acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, __builtin_bit_cast(bf16x8, b),
+                                                      acc[j], 0, 0, 0);
+    }
+  }
+  // epilogue: bias, activation, bfloat16
+#pragma unroll
+  for (int j = 0; j < BN / 32; ++j) {
+    const int n = j * 32 + lane % 32;
+    const float b = bias ? bias[n] : 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int m = wave * 32 + 8 * (r / 4) + 4 * (lane / 32) + r % 4;
+      const int64_t p = m0 + m;
+      if (p >= im.pixels)
+        continue;
+      float v = acc[j][r] + b;
+      if (relu)
+        v = v > 0.0f ? v : 0.0f;
+      y[p * BN + n] = to_bf16(v);
+    }
+  }
+}
+
 template <int BN, int KC>
 void launch_fwd(const cw_conv3x3_args &a, const Image &im, hipStream_t s) {
   const int tx = (a.w + kTW - 1) / kTW, ty = (a.h + kTH - 1) / kTH;
@@ -274,9 +341,31 @@ void launch_fwd(const cw_conv3x3_args &a, const Image &im, hipStream_t s) {
                      (const float *)a.bias, a.relu, (uint16_t *)a.y);
 }
 
+// Whether the flat kernel takes the layer. It costs a pixel of an image what it
+// costs any other, the tiles a pixel of the padded image a half to a fifth of
+// that: tiles, where they fill the card, from the share of true pixels up at
+// which both took the same time (at 16 channels to 32 in 0.19, 40000 x 6: 31.1
+// and 31.9 us; at 64 to 64 0.38, 25000 x 12: 87 and 90; at 128 to 128 0.63, 256
+// images of 40 x 40: 344 and 337), and tiles always where the card holds all of
+// them at once (4096 images of 8 x 8 at 128 channels 213 and 437 us, one of 8 x
+// 8 51 and 27). Past 128 channels the tile would be staged again for each tap
+// (6 x 200 x 225, 256 to 128: 446 us flat, 697 so).
+bool flat_fwd(const cw_conv3x3_args &a) {
+  if (a.cin > 128)
+    return true;
+  const int64_t tiles = (int64_t)a.n * ((a.h + kTH - 1) / kTH) * ((a.w + kTW - 1) / kTW);
+  const int at_once = a.cin <= 32 ? 1024 : a.cin <= 64 ? 512 : 256;
+  const double least = a.cin <= 32 ? 0.2 : a.cin <= 64 ? 0.38 : 0.65;
+  return tiles > at_once && (double)a.n * a.h * a.w < least * (double)(tiles * (kTH * kTW));
+}
+
 template <int BN>
 void launch_fwd(const cw_conv3x3_args &a, const Image &im, hipStream_t s) {
-  if (a.cin <= 16)
+  if (flat_fwd(a))
+    hipLaunchKernelGGL(conv3x3_fwd_flat<BN>, dim3((int)((im.pixels + kBM - 1) / kBM)),
+                       dim3(kThreads), 0, s, im, a.cin, (const uint4 *)a.x,
+                       (const uint4 *)a.weight, (const float *)a.bias, a.relu, (uint16_t *)a.y);
+  else if (a.cin <= 16)
     launch_fwd<BN, 16>(a, im, s);
   else if (a.cin <= 32)
     launch_fwd<BN, 32>(a, im, s);
