@@ -569,6 +569,114 @@ conv3x3_wgrad(Image im, int strips, int cin, int cout, const uint4 *__restrict__
     }
 }
 
+// What the strips waste: images of a few pixels a side, and layers of so few
+// pixels that a strip's march is one or two blocks long. One block: 128 rows of
+// the (tap, ci) axis x BN output channels, summed over its run of pixels of the
+// whole batch 32 at a time, x gathered from memory once a tap.
+template <int BN>
+__global__ void __launch_bounds__(kThreads)
+conv3x3_wgrad_flat(Image im, int cin, const uint4 *__restrict__ x, const uint4 *__restrict__ dy,
+                   int64_t run, float *__restrict__ part) {
+  constexpr int P = 32; // pixels a step
+  __shared__ __attribute__((aligned(16))) uint16_t sx[2][128][P + 8];
+  __shared__ __attribute__((aligned(16))) uint16_t sd[2][BN][P + 8];
+  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+  const int krows = 9 * cin;
+  const int r0 = blockIdx.x * 128;
+  const int split = blockIdx.y;
+  const int64_t p_begin = (int64_t)split * run;
+  const int64_t p_end = p_begin + run < im.pixels ? p_begin + run : im.pixels;
+  const int cin8 = cin / 8;
+  constexpr int cout8 = BN / 8;
+  constexpr int DPT = (P * cout8 + kThreads - 1) / kThreads; // dy chunks a thread
+  // staging: x chunk (pixel xp, rows xr .. xr + 7) twice; dy chunks (pixel dp,
+  // channels dc .. dc + 7)
+  uint4 rx[2], rd[DPT];
+  auto load = [&](int64_t q0) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int t = tid + h * kThreads;       // 512 chunks: 32 pixels x 16
+      const int xp = t / 16, xr = r0 + (t % 16) * 8;
+      rx[h] = uint4{0, 0, 0, 0};
+      const int64_t p = q0 + xp;
+      if (p < p_end && xr < krows) {
+        const int tap = xr / cin, ci = xr % cin;
+        const int64_t q = shifted(im, p, tap);
+        if (q >= 0)
+          rx[h] = x[q * cin8 + ci / 8];
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < DPT; ++h) {
+      const int t = tid + h * kThreads;
+      const int dp = t / cout8, dc = (t % cout8) * 8;
+      rd[h] = uint4{0, 0, 0, 0};
+      const int64_t p = q0 + dp;
+      if (dp < P && p < p_end)
+        rd[h] = dy[p * cout8 + dc / 8];
+    }
+  };
+  f32x16 acc[BN / 32];
+#pragma unroll
+  for (int j = 0; j < BN / 32; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      acc[j][r] = 0.0f;
+  const int64_t steps = (p_end - p_begin + P - 1) / P;
+  if (steps > 0)
+    load(p_begin);
+  for (int64_t s = 0; s < steps; ++s) {
+    const int buf = (int)(s & 1);
+    // transposed into LDS: [row][pixel], [channel][pixel]
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int t = tid + h * kThreads;
+      const int xp = t / 16, xr = (t % 16) * 8;
+      const uint16_t *v = reinterpret_cast<const uint16_t *>(&rx[h]);
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        sx[buf][xr + i][xp] = v[i];
+    }
+#pragma unroll
+    for (int h = 0; h < DPT; ++h) {
+      const int t = tid + h * kThreads;
+      const int dp = t / cout8, dc = (t % cout8) * 8;
+      if (dp < P) {
+        const uint16_t *v = reinterpret_cast<const uint16_t *>(&rd[h]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          sd[buf][dc + i][dp] = v[i];
+      }
+    }
+    __syncthreads();
+    if (s + 1 < steps)
+      load(p_begin + (s + 1) * P);
+    // rows of P + 8 bfloat16 (80 bytes), so a lane's eight pixels are one
+    // aligned 16-byte LDS read
+#pragma unroll
+    for (int k = 0; k < P; k += 16) {
+      const bf16x8 av = __builtin_bit_cast(
+          bf16x8, *reinterpret_cast<const uint4 *>(&sx[buf][wave * 32 + lane % 32][k + 8 * (lane / 32)]));
+#pragma unroll
+      for (int j = 0; j < BN / 32; ++j) {
+        const bf16x8 bv = __builtin_bit_cast(
+            bf16x8, *reinterpret_cast<const uint4 *>(&sd[buf][j * 32 + lane % 32][k + 8 * (lane / 32)]));
+        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bv, av, acc[j], 0, 0, 0);
+      }
+    }
+  }
+  // the partial: part[split][co][row], dw's own order
+  const int row = r0 + wave * 32 + lane % 32;
+  if (row >= krows)
+    return;
+  float *out = part + (int64_t)split * krows * BN;
+#pragma unroll
+  for (int j = 0; j < BN / 32; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      out[(j * 32 + 8 * (r / 4) + 4 * (lane / 32) + r % 4) * krows + row] = acc[j][r];
+}
+
 // out = the sum over the slices: a thread one value of every fourth slice, eight
 // loads in flight, the four threads' sums then added in order
 __global__ void __launch_bounds__(kThreads)
@@ -746,13 +854,63 @@ head_bwd(int64_t pixels, const uint4 *__restrict__ x, const float *__restrict__ 
 }
 
 template <int CI, int CO>
-void launch_wgrad(const cw_conv3x3_args &a, const Image &im, hipStream_t s) {
+void launch_wgrad(const cw_conv3x3_args &a, const Image &im, int slices, hipStream_t s) {
   const int strips = (a.w + kWStrip - 1) / kWStrip;
   const int64_t rows = (int64_t)a.n * strips * a.h;
-  const int run = (int)((rows + a.splits - 1) / a.splits);
-  hipLaunchKernelGGL((conv3x3_wgrad<CI, CO>), dim3((a.cin + CI - 1) / CI * (a.cout / CO), a.splits),
+  const int run = (int)((rows + slices - 1) / slices);
+  hipLaunchKernelGGL((conv3x3_wgrad<CI, CO>), dim3((a.cin + CI - 1) / CI * (a.cout / CO), slices),
                      dim3(kThreads), 0, s, im, strips, a.cin, a.cout, (const uint4 *)a.x,
                      (const uint4 *)a.dy, run, (float *)a.workspace);
+}
+
+template <int BN>
+void launch_wgrad_flat(const cw_conv3x3_args &a, const Image &im, int slices, hipStream_t s) {
+  const int64_t run = (im.pixels + slices - 1) / slices;
+  hipLaunchKernelGGL(conv3x3_wgrad_flat<BN>, dim3((9 * a.cin + 127) / 128, slices), dim3(kThreads),
+                     0, s, im, a.cin, (const uint4 *)a.x, (const uint4 *)a.dy, run,
+                     (float *)a.workspace);
+}
+
+// Whether the flat kernel takes the weight gradient: where the strips' columns
+// and each march's two rows more than it sums leave fewer than a few true
+// pixels in a hundred (both took the same time at 32 channels at 0.016, 20000
+// images of 2 x 2: 157 and 152 us; at 64 at 0.05, 16384 of 4 x 4: 297 and 336;
+// at 128 at 0.08, 60000 x 4: 681 and 880, 40000 x 6: 677 and 612), and where
+// the layer has so few pixels that the strips' blocks are too few and their
+// marches too short (one image of 16 x 16 at 64 channels 10.5 and 22 us; at 64
+// channels both took 21 us at about 1500 pixels, at 128 at 800).
+bool flat_wgrad(const cw_conv3x3_args &a) {
+  const int most = a.cin > a.cout ? a.cin : a.cout;
+  const double pixels = (double)a.n * a.h * a.w;
+  const double least = most <= 32 ? 0.016 : most <= 64 ? 0.05 : 0.08;
+  const double marched = (double)a.n * (a.h + 2) * ((a.w + kWStrip - 1) / kWStrip * kWStrip);
+  return pixels * most < 1e5 || pixels < least * marched;
+}
+
+// a pass sums fewer slices than it was given room for where a slice would be
+// shorter than six rows of a strip, or 2048 pixels (sixteen always: a small
+// layer's blocks)
+int launch_wgrad(const cw_conv3x3_args &a, const Image &im, hipStream_t s) {
+  if (flat_wgrad(a)) {
+    int64_t slices = im.pixels / 2048;
+    slices = slices < 16 ? 16 : slices > 256 ? 256 : slices;
+    slices = slices < a.splits ? slices : a.splits;
+    switch (a.cout) {
+    case 32: launch_wgrad_flat<32>(a, im, (int)slices, s); break;
+    case 64: launch_wgrad_flat<64>(a, im, (int)slices, s); break;
+    default: launch_wgrad_flat<128>(a, im, (int)slices, s); break;
+    }
+    return (int)slices;
+  }
+  int64_t slices = (int64_t)a.n * a.h * ((a.w + kWStrip - 1) / kWStrip) / 6;
+  slices = slices < 1 ? 1 : slices < a.splits ? slices : a.splits;
+  if (a.cin <= 32)
+    a.cout == 32 ? launch_wgrad<32, 32>(a, im, (int)slices, s)
+                 : launch_wgrad<32, 64>(a, im, (int)slices, s);
+  else
+    a.cout == 32 ? launch_wgrad<64, 32>(a, im, (int)slices, s)
+                 : launch_wgrad<64, 64>(a, im, (int)slices, s);
+  return (int)slices;
 }
 
 // the kernels' weights from the float32 master: wt (cout, 9 cin) as is and
@@ -858,14 +1016,11 @@ int cw_conv3x3_bf16_bwd_weight(const cw_conv3x3_args *a, void *stream) {
     return fail("the backward weight pass needs x, dy, dweight, a workspace and splits");
   const Image im{a->n, a->h, a->w, (int64_t)a->n * a->h * a->w};
   const auto s = (hipStream_t)stream;
-  if (a->cin <= 32)
-    a->cout == 32 ? launch_wgrad<32, 32>(*a, im, s) : launch_wgrad<32, 64>(*a, im, s);
-  else
-    a->cout == 32 ? launch_wgrad<64, 32>(*a, im, s) : launch_wgrad<64, 64>(*a, im, s);
+  const int slices = launch_wgrad(*a, im, s);
   if (int e = hip_status("conv3x3_wgrad"))
     return e;
   const int total = 9 * a->cin * a->cout;
-  launch_slices_sum(total, a->splits, a->workspace, a->dweight, s);
+  launch_slices_sum(total, slices, a->workspace, a->dweight, s);
   return hip_status("slices_sum");
 }
 

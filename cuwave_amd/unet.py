@@ -42,12 +42,13 @@ def _bf16_weights(w: torch.Tensor, cout: int, cin: int, flipped: bool):
 
 
 def _splits(n: int, h: int, w: int, cin: int, cout: int) -> int:
-    """Pixel runs a weight gradient sums apart: its kernel takes two blocks a CU (256 CUs),
-    so 512 blocks over the channel tiles of 64, each of at least 6 rows of a 64-column
-    strip (below that the slices cost more than the CUs they occupy give)."""
+    """The most pixel runs a weight gradient sums apart (the pass takes no more than suit
+    its layer): its kernel takes two blocks a CU (256 CUs), so 512 blocks over the channel
+    tiles of 64, each of at least 6 rows of a 64-column strip, and room for sixteen runs
+    of a small layer."""
     tiles = max(1, -(-cin // 64)) * max(1, cout // 64)
     rows = n * h * -(-w // 64)
-    return max(1, min(512 // tiles, rows // 6))
+    return max(16, min(512 // tiles, rows // 6))
 
 
 def _slices(threads: int) -> int:

@@ -527,7 +527,7 @@ typedef struct cw_conv3x3_args {
   void *dx;                    /* (n, h, w, cin) bfloat16 */
   void *dweight;               /* (cout, 9 cin) float32 */
   void *workspace;             /* splits x 9 cin cout float32 partial sums */
-  int32_t splits;              /* pixel runs the weight gradient sums apart */
+  int32_t splits;              /* the most pixel runs the weight gradient sums apart */
 } cw_conv3x3_args;
 
 /* y = act(bias + conv(x, weight)) */

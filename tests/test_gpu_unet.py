@@ -137,6 +137,9 @@ def test_training_fits_a_target_on_the_gpu():
     (1, 9, 65, 16, 128),    # one past a tile, half a channel chunk
     (2, 17, 33, 48, 64),    # a channel count of the 16-channel chunks only
     (1, 40, 130, 96, 128),  # several tiles and chunks each way
+    (700, 3, 5, 32, 64),    # small images: the flat kernels', runs of pixels across them
+    (400, 4, 6, 128, 128),
+    (1, 1200, 2, 64, 32),
 ])
 def test_a_convolution_at_its_tiles_edges(n, h, w, cin, cout):
     print(f"case conv3x3 {n}x{h}x{w} {cin}->{cout}", flush=True)
