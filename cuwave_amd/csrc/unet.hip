@@ -462,6 +462,7 @@ conv3x3_wgrad(Image im, int strips, int cin, int cout, const uint4 *__restrict__
     at += b - a;
     const int c0 = s % strips * kWStrip;                 // the strip's first column
     const int base = s / strips * im.h * im.w;           // the image's first pixel
+    const bool ragged = im.w - c0 < kWStrip;             // the image ends in the strip
     uint4 v[4], ev;
     // input row r into the x registers, gradient row r + 1 into the dy ones
     auto fetch = [&](int r) {
@@ -515,7 +516,16 @@ conv3x3_wgrad(Image im, int strips, int cin, int cout, const uint4 *__restrict__
         const uint32_t a2 = __builtin_amdgcn_alignbit(m.z, m.y, 16);
         const uint32_t a3 = __builtin_amdgcn_alignbit(m.w, m.z, 16);
         const uint32_t a4 = __builtin_amdgcn_alignbit(right, m.w, 16);
-        const bf16x8 in[3] = {__builtin_bit_cast(bf16x8, uint4{a0, a1, a2, a3}),
+        uint4 before = {a0, a1, a2, a3};
+        if (ragged) { // the column past the last meets the last one's value: no pixel
+          const int d = im.w - c0 - 8 * g;
+          const uint32_t keep = d & 1 ? 0x0000ffffu : 0xffff0000u;
+          before.x &= d >> 1 == 0 ? keep : ~0u;
+          before.y &= d >> 1 == 1 ? keep : ~0u;
+          before.z &= d >> 1 == 2 ? keep : ~0u;
+          before.w &= d >> 1 == 3 ? keep : ~0u;
+        }
+        const bf16x8 in[3] = {__builtin_bit_cast(bf16x8, before),
                               __builtin_bit_cast(bf16x8, m),
                               __builtin_bit_cast(bf16x8, uint4{a1, a2, a3, a4})};
 #pragma unroll

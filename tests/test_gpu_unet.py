@@ -239,3 +239,26 @@ def test_a_convolution_adds_its_terms_tap_by_tap(cin, cout, n, h, w):
         y = conv(x.cuda().bfloat16())
     # the same additions in the same order: the same bits
     torch.testing.assert_close(y.cpu(), ref.bfloat16(), rtol=0, atol=0)
+
+
+@pytest.mark.parametrize("w", [57, 64, 70, 95])  # the last column at places of a run, a strip
+@pytest.mark.parametrize("cin, cout", [(32, 32), (64, 128)])
+def test_an_infinity_in_the_last_column_stays_in_its_taps(w, cin, cout):
+    print(f"case infinity {w} {cin}->{cout}", flush=True)
+    g = torch.Generator().manual_seed(w)
+    x = _bf(torch.randn(2, 40, w, cin, generator=g))
+    dy = _bf(torch.randn(2, 40, w, cout, generator=g))
+    conv = unet.Conv3x3(cin, cout, False)
+    ref_w = conv.weight.detach().clone().double().requires_grad_(True)
+    O.conv3x3(x.double(), ref_w, torch.zeros(cout).double(), False).backward(dy.double())
+    x[1, 17, w - 1, 5] = float("inf")
+    conv = conv.cuda()
+    conv(x.cuda().bfloat16()).backward(dy.cuda().bfloat16())
+    ours = conv.weight.grad.cpu().reshape(cout, 3, 3, cin)
+    met = torch.zeros(3, 3, cin, dtype=torch.bool)
+    met[:, 1:, 5] = True  # no pixel lies right of it: the taps from the left never read it
+    assert bool(torch.isfinite(ours[:, ~met]).all())
+    assert not bool(torch.isfinite(ours[:, met]).any())
+    # the others are the sums without it (float32 sums of 2 x 40 x w products)
+    theirs = ref_w.grad.reshape(cout, 3, 3, cin)
+    assert _rel(ours[:, ~met], theirs[:, ~met]) < 1e-4
