@@ -110,29 +110,53 @@ class _Conv3x3(torch.autograd.Function):
 
 
 class _Head(torch.autograd.Function):
-    """y = x w + b in float32, x (n, h, w, 32) bfloat16, w (32, 1 .. 4)."""
+    """y = x w + b in float32, x (n, h, w, 32) bfloat16, w (32, 1 .. 4) and b float32. A
+    gradient of the gradient and a tangent, which the kernels don't give, come from torch's
+    products, as those of the general path do."""
+
+    @staticmethod
+    def takes(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor) -> bool:
+        """Whether the kernels compute what `x.float() @ w + b` would (not under autocast,
+        which takes that product in its own type)."""
+        return (x.dtype == torch.bfloat16 and w.dtype == b.dtype == torch.float32
+                and x.shape[-1] == w.shape[0] == 32 and 1 <= w.shape[1] <= 4
+                and b.shape == w.shape[1:] and x.device == w.device == b.device
+                and not torch.is_autocast_enabled("cuda"))
 
     @staticmethod
     def forward(ctx, x: torch.Tensor, w: torch.Tensor, b: torch.Tensor):
-        x, w = x.contiguous(), w.contiguous()
+        xc, wc, b = x.contiguous(), w.detach().contiguous(), b.detach().contiguous()
         n, h, wd, _ = x.shape
         y = torch.empty((n, h, wd, w.shape[1]), dtype=torch.float32, device=x.device)
-        _abi.call("cw_head_fwd", n * h * wd, w.shape[1], _abi.ptr(x), _abi.ptr(w.detach()),
-                  _abi.ptr(b.detach()), _abi.ptr(y), _abi.stream())
+        _abi.call("cw_head_fwd", n * h * wd, w.shape[1], _abi.ptr(xc), _abi.ptr(wc), _abi.ptr(b),
+                  _abi.ptr(y), _abi.stream())
         ctx.save_for_backward(x, w)
+        ctx.save_for_forward(x, w)
         return y
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
+    def jvp(ctx, dx, dw, db):
+        x, w = ctx.saved_tensors
+        terms = [dx.float() @ w] if dx is not None else []
+        terms += [x.float() @ dw] if dw is not None else []
+        tangent = sum(terms[1:], terms[0]) if terms else x.new_zeros(
+            (*x.shape[:-1], w.shape[1]), dtype=torch.float32)
+        return tangent if db is None else tangent + db
+
+    @staticmethod
     def backward(ctx, dy: torch.Tensor):
         x, w = ctx.saved_tensors
+        if torch.is_grad_enabled():  # differentiated again
+            dx = (dy @ w.t()).to(x.dtype) if ctx.needs_input_grad[0] else None
+            dw = x.float().reshape(-1, x.shape[-1]).t() @ dy.reshape(-1, dy.shape[-1])
+            return dx, dw, dy.sum((0, 1, 2))
         outputs, pixels = w.shape[1], x.numel() // x.shape[-1]
-        dy = dy.contiguous()
+        x, dy, wc = x.contiguous(), dy.contiguous(), w.contiguous()
         slices = _slices(pixels * 4)
         dx = torch.empty_like(x) if ctx.needs_input_grad[0] else None
         work = torch.empty((slices, 33 * outputs), dtype=torch.float32, device=x.device)
         dwb = torch.empty(33 * outputs, dtype=torch.float32, device=x.device)
-        _abi.call("cw_head_bwd", pixels, outputs, _abi.ptr(x), _abi.ptr(w.detach()), _abi.ptr(dy),
+        _abi.call("cw_head_bwd", pixels, outputs, _abi.ptr(x), _abi.ptr(wc), _abi.ptr(dy),
                   _abi.ptr(dx), _abi.ptr(work), slices, _abi.ptr(dwb), _abi.stream())
         return dx, dwb[:32 * outputs].view(32, outputs), dwb[32 * outputs:]
 
@@ -206,7 +230,7 @@ class UNet(nn.Module):
         m = self.mid(_pool(e2))
         d2 = self.dec2(torch.cat([self.up2(m), e2], -1).contiguous())
         d1 = self.dec1(torch.cat([self.up1(d2), e1], -1).contiguous())
-        if d1.shape[-1] == 32 and self.out_w.shape[1] <= 4 and self.out_w.dtype == torch.float32:
+        if _Head.takes(d1, self.out_w, self.out_b):
             return _Head.apply(d1, self.out_w, self.out_b)
         return d1.float() @ self.out_w + self.out_b
 

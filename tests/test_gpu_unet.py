@@ -262,3 +262,47 @@ def test_an_infinity_in_the_last_column_stays_in_its_taps(w, cin, cout):
     # the others are the sums without it (float32 sums of 2 x 40 x w products)
     theirs = ref_w.grad.reshape(cout, 3, 3, cin)
     assert _rel(ours[:, ~met], theirs[:, ~met]) < 1e-4
+
+
+def test_the_output_layer_is_differentiated_again_as_the_product_is():
+    print("case head, second derivatives and a tangent", flush=True)
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(2, 5, 7, 32, generator=g).bfloat16().cuda()
+    w, t = torch.randn(2, 32, 3, generator=g).cuda()
+    b = torch.randn(3, generator=g).cuda()
+
+    def seconds(layer):
+        p = [v.clone().requires_grad_(True) for v in (x, w, b)]
+        (gw,) = torch.autograd.grad((layer(*p) ** 2).sum(), p[1], create_graph=True)
+        return torch.autograd.grad((gw**2).sum(), p)
+
+    ours = seconds(unet._Head.apply)
+    for a, r in zip(ours, seconds(lambda x, w, b: x.float() @ w + b)):
+        assert a.dtype == r.dtype
+        # float32 products; the one at x rounded to bfloat16
+        assert _rel(a, r) < (4e-3 if a.dtype == torch.bfloat16 else 1e-5)
+    fwd = torch.autograd.forward_ad
+    with fwd.dual_level():
+        y = unet._Head.apply(x, fwd.make_dual(w, t), b)
+        assert _rel(fwd.unpack_dual(y).tangent, x.float() @ t) < 1e-5
+
+
+@pytest.mark.parametrize("how", ["plain", "autocast", "wide bias", "one bias for all"])
+def test_the_output_layer_s_kernels_step_aside_for_other_products(how):
+    print(f"case head {how}", flush=True)
+    torch.manual_seed(5)
+    net = unet.UNet(cout=2).cuda()
+    if how == "wide bias":
+        net.out_b = torch.nn.Parameter(net.out_b.detach().double())
+    if how == "one bias for all":
+        net.out_b = torch.nn.Parameter(net.out_b.detach()[:1])
+    seen = []
+    net.dec1.register_forward_hook(lambda module, args, out: seen.append(out))
+    with torch.no_grad(), torch.autocast("cuda", torch.bfloat16, enabled=how == "autocast"):
+        out = net(torch.randn(1, 8, 12, 2, device="cuda"))
+        ref = seen[0].float() @ net.out_w + net.out_b
+    assert out.dtype == ref.dtype
+    if how == "plain":  # float32 sums of 32 terms
+        assert _rel(out, ref) < 1e-6
+    else:
+        torch.testing.assert_close(out, ref, rtol=0, atol=0)
