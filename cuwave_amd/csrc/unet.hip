@@ -972,6 +972,9 @@ int check_conv(const cw_conv3x3_args *a) {
   return 0;
 }
 
+// the activations are read and written 16 bytes a thread
+bool aligned(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
 int hip_status(const char *where) {
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
@@ -1053,6 +1056,8 @@ int cw_relu_bias_grad(int64_t pixels, int32_t channels, const void *dy, const vo
     return fail("channels must be 32, 64 or 128");
   if (y && !dpre)
     return fail("a masked gradient needs dpre");
+  if (!aligned(dy) || !aligned(y) || (y && !aligned(dpre)))
+    return fail("dy, y and dpre must be 16-byte aligned");
   const int64_t chunks = pixels * (channels / 8);
   const auto s = (hipStream_t)stream;
   const uint4 *d = (const uint4 *)dy, *yy = (const uint4 *)y;
@@ -1072,6 +1077,8 @@ int cw_head_fwd(int64_t pixels, int32_t outputs, const void *x, const void *w, c
                 void *stream) {
   if (pixels < 1 || !x || !w || !b || !y)
     return fail("the output layer needs pixels, x, w, b and y");
+  if (!aligned(x))
+    return fail("x must be 16-byte aligned");
   const int64_t threads = pixels * kHeadG;
   const dim3 grid((int)((threads + kThreads - 1) / kThreads)), block(kThreads);
   const auto s = (hipStream_t)stream;
@@ -1092,6 +1099,8 @@ int cw_head_bwd(int64_t pixels, int32_t outputs, const void *x, const void *w, c
                 void *workspace, int32_t slices, void *dwb, void *stream) {
   if (pixels < 1 || !x || !w || !dy || !workspace || !dwb || slices < 1)
     return fail("the output layer's backward needs pixels, x, w, dy, a workspace, slices and dwb");
+  if (!aligned(x) || !aligned(dx))
+    return fail("x and dx must be 16-byte aligned");
   const dim3 grid(slices), block(kThreads);
   const auto s = (hipStream_t)stream;
   const uint4 *xx = (const uint4 *)x;

@@ -57,6 +57,12 @@ def _slices(threads: int) -> int:
     return max(1, min(1024, -(-threads // 256)))
 
 
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """`t` contiguous at a 16-byte address (a view into another tensor may start anywhere)."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 class _Conv3x3(torch.autograd.Function):
     """y = act(conv3x3(x, w) + b) on NHWC bfloat16, w float32 (cout, 9 cin)."""
 
@@ -81,7 +87,7 @@ class _Conv3x3(torch.autograd.Function):
         x, y = ctx.saved_tensors
         n, h, w, cin = x.shape
         cout = y.shape[-1]
-        dy = dy.to(torch.bfloat16).contiguous()
+        dy = _aligned(dy.to(torch.bfloat16))
         # the gradient before the activation and the bias' gradient, one pass
         pixels = n * h * w
         slices = _slices(pixels * cout // 8)
@@ -125,7 +131,7 @@ class _Head(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x: torch.Tensor, w: torch.Tensor, b: torch.Tensor):
-        xc, wc, b = x.contiguous(), w.detach().contiguous(), b.detach().contiguous()
+        xc, wc, b = _aligned(x), w.detach().contiguous(), b.detach().contiguous()
         n, h, wd, _ = x.shape
         y = torch.empty((n, h, wd, w.shape[1]), dtype=torch.float32, device=x.device)
         _abi.call("cw_head_fwd", n * h * wd, w.shape[1], _abi.ptr(xc), _abi.ptr(wc), _abi.ptr(b),
@@ -151,7 +157,7 @@ class _Head(torch.autograd.Function):
             dw = x.float().reshape(-1, x.shape[-1]).t() @ dy.reshape(-1, dy.shape[-1])
             return dx, dw, dy.sum((0, 1, 2))
         outputs, pixels = w.shape[1], x.numel() // x.shape[-1]
-        x, dy, wc = x.contiguous(), dy.contiguous(), w.contiguous()
+        x, dy, wc = _aligned(x), dy.contiguous(), w.contiguous()
         slices = _slices(pixels * 4)
         dx = torch.empty_like(x) if ctx.needs_input_grad[0] else None
         work = torch.empty((slices, 33 * outputs), dtype=torch.float32, device=x.device)

@@ -557,7 +557,7 @@ int cw_head_fwd(int64_t pixels, int32_t outputs, const void *x, const void *w, c
                 void *stream);
 /* its gradients in one pass: dx (pixels, 32) bfloat16 (or NULL), and in dwb the
  * (32, outputs) gradient at w, then the (outputs) one at b; workspace slices x
- * 33 outputs float32 */
+ * 33 outputs float32; x and dx 16-byte aligned */
 int cw_head_bwd(int64_t pixels, int32_t outputs, const void *x, const void *w, const void *dy, void *dx,
                 void *workspace, int32_t slices, void *dwb, void *stream);
 

@@ -154,3 +154,18 @@ def test_the_product_refuses_to_run_without_its_device(monkeypatch):
         pytest.skip("a GPU is present")
     with pytest.raises(RuntimeError, match="AMD GPU"):
         _abi.require_device()
+
+
+@pytest.mark.parametrize("at", [2, 8])
+def test_the_activation_passes_refuse_a_misaligned_tensor(at):
+    """The passes over bfloat16 activations read 16 bytes a thread: an address that is no
+    multiple of 16 is refused before anything is launched."""
+    good, bad = 1 << 20, (1 << 20) + at  # never read: the checks come first
+    for args in ((bad, good, good), (good, bad, good), (good, good, bad)):
+        with pytest.raises(RuntimeError, match="aligned"):
+            _abi.call("cw_relu_bias_grad", 8, 32, *args, good, 1, good, None)
+    with pytest.raises(RuntimeError, match="aligned"):
+        _abi.call("cw_head_fwd", 8, 1, bad, good, good, good, None)
+    for x, dx in ((bad, good), (good, bad)):
+        with pytest.raises(RuntimeError, match="aligned"):
+            _abi.call("cw_head_bwd", 8, 1, x, good, good, dx, good, 1, good, None)

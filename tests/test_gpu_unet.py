@@ -306,3 +306,21 @@ def test_the_output_layer_s_kernels_step_aside_for_other_products(how):
         assert _rel(out, ref) < 1e-6
     else:
         torch.testing.assert_close(out, ref, rtol=0, atol=0)
+
+
+def test_a_gradient_that_starts_inside_another_tensor():
+    print("case misaligned gradients", flush=True)
+    g = torch.Generator().manual_seed(9)
+    conv = unet.Conv3x3(32, 32).cuda()
+    x = torch.randn(1, 9, 11, 32, generator=g).bfloat16().cuda()
+    flat = torch.randn(x.numel() + 1, generator=g).bfloat16().cuda()
+    w, b = torch.randn(32, 1, generator=g).cuda(), torch.zeros(1, device="cuda")
+    results = []
+    for dy in (flat[1:].clone(), flat[1:]):  # the second two bytes past an aligned address
+        p = x.clone().requires_grad_(True)
+        results.append(torch.autograd.grad(conv(p), [p, conv.weight, conv.bias],
+                                           dy.view(x.shape)))
+    results.append([unet._Head.apply(flat[1:].view(x.shape), w, b)])
+    results.append([unet._Head.apply(flat[1:].clone().view(x.shape), w, b)])
+    for a, c in (*zip(*results[:2]), *zip(*results[2:])):
+        torch.testing.assert_close(a, c, rtol=0, atol=0)
