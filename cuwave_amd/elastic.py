@@ -24,8 +24,8 @@ innermost in every per-shot array as in the pressure path:
 
 The host-side parametrization (point inertia, excitation weights, the norms)
 runs in numpy in the simulation's precision, as the reference computes it, so
-what the kernels read is the reference's to the bit; the chain rule
-(`finalize_gradients`) runs the same operations where the densities are.
+what the kernels read is the reference's to the bit; the chain rule of
+`finalize_gradients` runs the same operations where the densities are.
 """
 
 from __future__ import annotations
@@ -523,25 +523,32 @@ def _pair_average_adjoint(sim: ElasticWave, density: torch.Tensor, field: torch.
     return out
 
 
-def finalize_gradients(sim: ElasticWave, grads: dict, gamma: np.ndarray) -> dict:
-    """The point densities chained through the averages onto the nodal design field
-    (cuwave/elastic.py:716-729, cuwave/wave.py:386-475), on the densities' device."""
+def _chain_rule(sim: ElasticWave, grads: dict, gamma: np.ndarray) -> dict:
+    """`finalize_gradients` as tensors on the densities' device."""
     device = grads["normal"].device
 
     def here(a):
-        return torch.as_tensor(a, device=device)
+        return torch.as_tensor(np.ascontiguousarray(a), device=device)
 
     gamma = here(gamma)
     g_mass = torch.zeros_like(grads["normal"])
-    density = float(sim.np_dtype(sim.density))
     for c in range(sim.ncomp):
-        g_mass += _point_average_adjoint(grads["mass"][c] * here(sim.point_weights((c,))) * density,
-                                         c)
+        density = grads["mass"][c] * here(sim.point_weights((c,)))
+        # a numpy number brings its own precision to the product, a Python one none
+        density = density * (here(sim.density) if isinstance(sim.density, np.generic)
+                             else float(sim.np_dtype(sim.density)))
+        g_mass += _point_average_adjoint(density, c)
     g_stiff = grads["normal"] * here(sim.point_weights(()))
     for p, axes in enumerate(PAIRS[sim.ndim][sim.ndim:]):
         shear = grads["shear"][p] * here(sim.point_weights(axes))
         g_stiff += _pair_average_adjoint(sim, shear, gamma, axes)
     return {"mass": g_mass, "stiff": g_stiff}
+
+
+def finalize_gradients(sim: ElasticWave, grads: dict, gamma: np.ndarray) -> dict:
+    """The point densities chained through the averages onto the nodal design field
+    (cuwave/elastic.py:716-729, cuwave/wave.py:386-475), as host arrays."""
+    return {k: v.cpu().numpy() for k, v in _chain_rule(sim, grads, gamma).items()}
 
 
 def reconstruction_nodes(sim: ElasticWave):
@@ -633,7 +640,7 @@ def sensitivity(sim: ElasticWave, source: Source, indicator, sensors, objective)
         l0, l1 = P[m % 2], P[1 - m % 2]
         back.step(l0, l1, l0, grads, v1, mf)
         adj.adjoint_inject(l0, adjoint, m, grads["mass"], v1, mf)
-    out = finalize_gradients(sim, grads, mat["gamma_host"])
+    out = _chain_rule(sim, grads, mat["gamma_host"])
     if sim.pml is not None:
         layer = torch.as_tensor(pml_nodes(sim), device=eng.device)
         for f in out.values():
@@ -817,7 +824,7 @@ class _Reconstruction:
         return rebuilt / self.seed if self.seed else float("inf")
 
     def gradients(self) -> dict:
-        out = finalize_gradients(self.sim, self.grads, self.mat["gamma_host"])
+        out = _chain_rule(self.sim, self.grads, self.mat["gamma_host"])
         for f in out.values():
             f[~self.inside] = 0.0
         return out
@@ -877,10 +884,12 @@ def misfit_gradient(sim: ElasticWave, sources, indicator, sensors, observed, obj
         else:
             for k in total:
                 total[k] += run.grads[k]
-    out = finalize_gradients(sim, total, mat["gamma_host"])
+    out = _chain_rule(sim, total, mat["gamma_host"])
+
     def chained(jacobian, density):
-        if np.ndim(jacobian) == 0:
-            return float(jacobian) * density
+        if isinstance(jacobian, (int, float)) and not isinstance(jacobian, np.generic):
+            return jacobian * density
+        jacobian = np.ascontiguousarray(as_numpy(jacobian))
         return torch.as_tensor(jacobian, device=density.device) * density
 
     jm, js = sim.parametrization_jacobian(indicator)

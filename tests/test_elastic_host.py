@@ -97,6 +97,25 @@ def test_the_chain_rule_matches_the_oracle(name):
         np.testing.assert_array_equal(ours[k], theirs[k])
 
 
+def test_the_chain_rule_gives_host_arrays_and_takes_any_of_them():
+    z = golden("el_adj_2d_o4_pml_f32")
+    sim, osim = elastic_sim(z), E.sim_from_npz(z)
+    rng = np.random.default_rng(8)
+    gamma = np.ascontiguousarray(z["indicator"], dtype=sim.np_dtype)
+    grads = {"mass": rng.standard_normal((sim.ncomp, *sim.Nx_padded)).astype(sim.np_dtype),
+             "normal": rng.standard_normal(sim.Nx_padded).astype(sim.np_dtype),
+             "shear": rng.standard_normal((sim.npairs, *sim.Nx_padded)).astype(sim.np_dtype)}
+    backwards = np.ascontiguousarray(gamma[::-1])[::-1]  # the same values, a negative stride
+    for density in (sim.density, np.float64(sim.density), np.float32(sim.density)):
+        sim.density = osim.density = density
+        ours = elastic.finalize_gradients(sim, {k: torch.as_tensor(v) for k, v in grads.items()},
+                                          backwards)
+        theirs = E.finalize_gradients(osim, {k: v.copy() for k, v in grads.items()}, gamma)
+        for k in ("mass", "stiff"):
+            assert isinstance(ours[k], np.ndarray) and ours[k].dtype == sim.np_dtype
+            np.testing.assert_array_equal(ours[k], theirs[k])
+
+
 def test_the_abi_grid_carries_the_constants():
     z = golden("el_adj_2d_o4_pml_f32")
     sim = elastic_sim(z)
