@@ -217,7 +217,7 @@ class MaxwellWave(Simulation):
         """The harmonic mean of the two nodes component c sits between
         (cuwave/wave.py:416-425)."""
         tiny = float(np.finfo(self.np_dtype).tiny)
-        inverse = 1.0 / torch.clamp(torch.as_tensor(field), min=tiny)
+        inverse = 1.0 / torch.clamp(torch.as_tensor(np.ascontiguousarray(field)), min=tiny)
         mean = self._point_average(inverse, c)
         return torch.where(mean > 0.0, 1.0 / torch.clamp(mean, min=tiny),
                            torch.zeros((), dtype=self.dtype)).numpy()
@@ -441,7 +441,8 @@ def finalize_gradients(sim: MaxwellWave, grads: dict, mat: dict) -> dict:
     427-475); zero stiffness otherwise."""
     eps = mat["eps"]
     g_mass = grads["mass"].cpu()
-    safe = torch.clamp(torch.as_tensor(eps), min=float(np.finfo(sim.np_dtype).tiny))
+    safe = torch.clamp(torch.as_tensor(np.ascontiguousarray(eps)),
+                       min=float(np.finfo(sim.np_dtype).tiny))
     square = safe * safe
     total = torch.zeros(sim.Nx_padded, dtype=sim.dtype)
     for c in range(sim.ncomp):

@@ -22,6 +22,7 @@ import math
 
 import numpy as np
 import pytest
+import torch
 
 from helpers import ROOT
 
@@ -366,3 +367,16 @@ def test_the_reverse_march_refuses_a_damped_field():
     with pytest.raises(NotImplementedError, match="damped"):
         S.reconstruction_sensitivity(sim, source, np.zeros(sim.Nx_padded),
                                      np.array([[1], [5], [7]]), lambda u: (0.0, u))
+
+
+def test_the_materials_take_a_permittivity_of_any_strides():
+    sim = MX.DielectricWave((9, 11), (0.1, 0.1), 4, 0.01, permittivity1=1.0, permittivity2=4.0)
+    rng = np.random.default_rng(2)
+    eps = (1.0 + 3.0 * rng.random(sim.Nx_padded)).astype(sim.np_dtype)
+    backwards = np.ascontiguousarray(eps[::-1])[::-1]  # the same values, a negative stride
+    np.testing.assert_array_equal(sim.point_inverse_inertia(backwards),
+                                  sim.point_inverse_inertia(eps))
+    grads = {"mass": torch.as_tensor(rng.standard_normal((sim.ncomp, *sim.Nx_padded))
+                                     .astype(sim.np_dtype))}
+    ours, theirs = (MX.finalize_gradients(sim, grads, {"eps": e}) for e in (backwards, eps))
+    np.testing.assert_array_equal(ours["mass"], theirs["mass"])
