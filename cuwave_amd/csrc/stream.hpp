@@ -278,11 +278,18 @@ __device__ __forceinline__ void forward_stream(const FwdParams<T> &p,
 // waves a SIMD and 352 us a level of 1090 x 1090 with 32 shots, against 92 (with
 // the five waves asked for), and 333. The forward core keeps `p`: read late, it
 // has eight waves a SIMD for seven and takes 180 us a step for 173.
+// The launch asserts that they are its first argument (FirstArg).
 template <typename P> __device__ __forceinline__ const P &late_params() {
   auto q = (const __attribute__((address_space(4))) P *)__builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(q));
   return *(const P *)q;
 }
+
+// the type of a kernel's first argument
+template <typename F> struct FirstArg;
+template <typename A, typename... Rest> struct FirstArg<void(A, Rest...)> {
+  using type = A;
+};
 
 // --------------------------------------------------------------- adjoint
 template <typename T, int R, int W, bool STIFF>
