@@ -123,3 +123,21 @@ class Receivers:
 
     def traces(self, record):
         return record
+
+
+def plain_waves(sim, nbatch: int, margin, axes=None) -> int:
+    """The waves of a launch over a vector family's interior whose every node lies `margin`
+    (low, high) nodes or more off the walls of `axes` (every axis by default): those that
+    run without a test a tap. Threads take the rows' nodes in order, a node's lanes in
+    groups of 16 bytes; the order of the rows is the plane's in 2D (in 3D ask for the fast
+    axis alone, which no order of rows changes)."""
+    lanes = 1 << (nbatch - 1).bit_length()
+    group = min(lanes, 16 // np.dtype(sim.np_dtype).itemsize)
+    inner = [n - 2 for n in sim.Nx]
+    place = np.indices(inner).reshape(sim.ndim, -1) + 1
+    off = np.ones(place.shape[1], dtype=bool)
+    for d in range(sim.ndim) if axes is None else axes:
+        off &= (place[d] >= 1 + margin[0]) & (place[d] <= sim.Nx[d] - 2 - margin[1])
+    threads = np.repeat(off, lanes // group)
+    whole = threads[:threads.size // 64 * 64].reshape(-1, 64)
+    return int(whole.all(axis=1).sum())

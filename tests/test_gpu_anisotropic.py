@@ -365,3 +365,37 @@ def test_a_damped_misfit_gradient_sums_the_stored_gradients():
     assert abs(cost - want_cost) <= 1e-12 * want_cost
     got = gradient.cpu().numpy()
     assert np.linalg.norm(got - want) <= 1e-10 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("count", [1, 5, 16])
+@pytest.mark.parametrize("precision", ["float32", "float64"])
+def test_waves_off_the_walls_march_to_the_oracles_bits(precision, count):
+    # rows long enough for waves that hold no node by a wall, which load the nodes around
+    # once and test no cell; the rows by the walls and their ends take the other branch
+    from helpers import plain_waves
+
+    print(f"anisotropic plain waves {precision} {count} shots", flush=True)
+    sim = aniso_sim((17, 150), "mixed", precision=precision, C=ORTHO, N=12)
+    assert plain_waves(sim, count, (1, 1)) > 10
+    rng = np.random.default_rng(count)
+    gamma = (0.5 + rng.random(sim.Nx_padded)).astype(sim.np_dtype)
+    sources = shots(sim, rng, count)
+    sensors = sensor_points(sim, rng)
+    field, record = AN.simulate_shots(sim, sources, gamma, sensors)
+    for b, source in enumerate(sources):
+        last, traces = oracle_march(sim, gamma, source, sensors)
+        assert np.array_equal(field[b].cpu().numpy(), last), f"shot {b}"
+        assert np.array_equal(record[b].cpu().numpy(), traces), f"shot {b}"
+
+
+@pytest.mark.parametrize("precision", ["float32", "float64"])
+def test_damped_waves_off_the_walls_march_to_the_oracles_bits(precision):
+    from helpers import plain_waves
+
+    assert plain_waves(aniso_sim((17, 150), precision=precision), 2, (1, 1)) > 10
+    test_a_damped_march_is_the_oracles_bit_for_bit((17, 150), "mixed", precision)
+
+
+@pytest.mark.parametrize("Nx", [(17, 150), (11, 12, 90)])
+def test_the_gradient_kernel_on_long_rows_is_the_oracles(Nx):
+    test_the_gradient_kernel_is_the_oracles(Nx)

@@ -517,3 +517,45 @@ def test_a_damped_misfit_gradient_sums_the_stored_gradients():
     assert abs(cost - want_cost) <= 1e-12 * want_cost
     got = gradient.cpu().numpy()
     assert np.linalg.norm(got - want) <= 1e-10 * np.linalg.norm(want)
+
+
+LONG = [((17, 150), 2), ((19, 150), 8), ((10, 11, 150), 4), ((14, 15, 150), 6)]
+
+
+@pytest.mark.parametrize("precision, count", [("float32", 1), ("float32", 5), ("float64", 1),
+                                              ("float64", 5)])
+@pytest.mark.parametrize("Nx, order", LONG)
+def test_waves_off_the_walls_march_to_the_oracles_bits(Nx, order, precision, count):
+    # rows long enough for waves whose taps along them all stay inside the walls, which
+    # take them as they lie; the rows' ends find images
+    from helpers import plain_waves
+
+    print(f"maxwell plain waves {Nx} order {order} {precision} {count} shots", flush=True)
+    sim = vector_sim(Nx, order, "mixed", precision=precision, N=12)
+    assert plain_waves(sim, count, (sim.radius, sim.radius), axes=(sim.ndim - 1,)) > 10
+    rng = np.random.default_rng(order + count)
+    gamma = rng.random(sim.Nx_padded).astype(sim.np_dtype)
+    sources = shots(sim, rng, count)
+    sensors = sensor_points(sim, rng)
+    field, record = MX.simulate_shots(sim, sources, gamma, sensors)
+    for b, source in enumerate(sources):
+        last, traces = oracle_march(sim, gamma, source, sensors)
+        assert np.array_equal(field[b].cpu().numpy(), last), f"shot {b}"
+        assert np.array_equal(record[b].cpu().numpy(), traces), f"shot {b}"
+
+
+@pytest.mark.parametrize("Nx, order", LONG)
+def test_waves_off_the_walls_step_the_adjoint_as_the_oracle(Nx, order):
+    # the adjoint step with its inertia density, and with a designed permeability's
+    test_the_adjoint_step_is_the_oracles_gradient_step(Nx, order)
+    test_the_permeability_density_is_the_oracles(Nx, order)
+
+
+@pytest.mark.parametrize("Nx, order, precision", [((17, 150), 4, "float32"),
+                                                  ((14, 15, 150), 2, "float64")])
+def test_damped_waves_off_the_walls_march_to_the_oracles_bits(Nx, order, precision):
+    test_a_damped_march_is_the_oracles_bit_for_bit(Nx, order, precision)
+
+
+def test_a_designed_permeability_on_long_rows_marches_to_the_oracles_bits():
+    test_a_designed_permeability_march_is_the_oracles_bit_for_bit((10, 11, 150), 4, "mixed")
