@@ -378,6 +378,7 @@ SIGNATURES = {
     "cw_scalar_gradient": ([ctypes.POINTER(GradientArgs), VP], I32),
     "cw_elastic_prepare": ([ctypes.POINTER(ElasticGrid), ctypes.POINTER(ElasticMaterial), VP], I32),
     "cw_elastic_step": ([ctypes.POINTER(ElasticStepArgs), VP], I32),
+    "cw_elastic_core_nodes": ([ctypes.POINTER(ElasticStepArgs)], I64),
     "cw_elastic_gradient": ([ctypes.POINTER(ElasticGradientArgs), VP], I32),
     "cw_elastic_points": ([ctypes.POINTER(ElasticGrid), ctypes.POINTER(ElasticPointArgs), VP], I32),
     "cw_maxwell_step": ([ctypes.POINTER(MaxwellStepArgs), VP], I32),

@@ -150,6 +150,15 @@ int cw_elastic_step(const cw_elastic_step_args *args, void *stream) {
   return dispatch<Step>(args->grid, *args, (hipStream_t)stream);
 }
 
+int64_t cw_elastic_core_nodes(const cw_elastic_step_args *args) {
+  if (!args || check_grid(&args->grid) || check_layer(args->grid, args->pml) || args->g_mass)
+    return 0;
+  cwe::ElBox box{};
+  if (!cweh::core_box(args->grid, args->pml, cweh::core_shape(args->grid), &box))
+    return 0;
+  return (int64_t)(box.y1 - box.y0) * (box.x1 - box.x0);
+}
+
 int cw_elastic_gradient(const cw_elastic_gradient_args *args, void *stream) {
   if (!args)
     return fail("args is NULL");

@@ -394,6 +394,9 @@ typedef struct cw_elastic_point_args {
 int cw_elastic_prepare(const cw_elastic_grid *grid, const cw_elastic_material *mat,
                        void *stream);
 int cw_elastic_step(const cw_elastic_step_args *args, void *stream);
+/* the nodes a 2D step without accumulators takes through its fused core, 0 where
+ * the pair of kernels takes them all (the fields' pointers are not read) */
+int64_t cw_elastic_core_nodes(const cw_elastic_step_args *args);
 int cw_elastic_gradient(const cw_elastic_gradient_args *args, void *stream);
 int cw_elastic_points(const cw_elastic_grid *grid, const cw_elastic_point_args *args,
                       void *stream);

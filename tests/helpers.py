@@ -3,6 +3,7 @@ product (`cuwave_amd`) and for the CPU oracle (`oracle/driver.py`)."""
 
 from __future__ import annotations
 
+import ctypes
 import sys
 from pathlib import Path
 
@@ -141,3 +142,17 @@ def plain_waves(sim, nbatch: int, margin, axes=None) -> int:
     threads = np.repeat(off, lanes // group)
     whole = threads[:threads.size // 64 * 64].reshape(-1, 64)
     return int(whole.all(axis=1).sum())
+
+
+def elastic_core_nodes(sim, nbatch: int, adjoint: bool = False) -> int:
+    """The nodes a step of `nbatch` shots takes through the fused elastic core."""
+    from cuwave_amd import _abi, boundary
+
+    a = _abi.ElasticStepArgs()
+    a.grid = sim.abi_grid(nbatch)
+    if sim.pml is not None:
+        for d, (lo, hi) in enumerate(boundary.pml_widths(sim)):
+            a.pml.lo[d], a.pml.hi[d] = lo, hi
+            a.pml.profile[d] = a.pml.memory[d] = 1 << 12  # not read
+        a.pml.phase = int(adjoint)
+    return _abi.call_value("cw_elastic_core_nodes", ctypes.byref(a))

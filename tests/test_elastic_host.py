@@ -16,7 +16,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import elastic_sim, golden, golden_names
+from helpers import elastic_core_nodes, elastic_sim, golden, golden_names
 
 from cuwave_amd import boundary, elastic, sbp
 from cuwave_amd.stencils import staggered_weights
@@ -143,3 +143,23 @@ def test_elastic_faces_and_layers_are_validated():
                             wavespeed_s=1.5)
     with pytest.raises(NotImplementedError):
         elastic.ElasticWave((40, 40), (1.0, 1.0), 10, 0.1, relaxation=object(), **kw)
+
+
+@pytest.mark.parametrize("n, order, shots, precision, layer, want", [
+    # closure rows 5 deep at order 4 (6 at the high end, whose last half point is past the
+    # last node), 2 ghosts and one wall node, and 2 nodes more each side for the update
+    ((131, 157), 4, 3, "float32", 0, (131 - 17) * (157 - 17)),
+    ((131, 157), 4, 33, "float32", 0, (131 - 17) * (157 - 17)),
+    # a layer of 9, 2 ghosts and the update's 2 each side
+    ((131, 157), 4, 20, "float64", 9, (131 - 24) * (157 - 24)),
+    ((131, 157), 4, 33, "float64", 0, 0),  # 64 lanes of doubles: the pair
+    ((131, 157), 8, 33, "float32", 0, 0),  # and of floats at the long stencils
+    ((40, 41), 4, 3, "float32", 9, 0),     # a core of less than half the nodes
+    ((40, 41, 42), 4, 2, "float32", 0, 0),
+])
+def test_the_core_takes_the_steps_its_rule_says(n, order, shots, precision, layer, want):
+    pml = boundary.Pml(layer, 2.0, 1e-6, 2.0) if layer else None
+    sim = elastic.ElasticWave(n, (1.0,) * len(n), 4, 0.1, precision=precision, space_order=order,
+                              density=1.0, wavespeed_p=2.0, wavespeed_s=1.0, pml=pml,
+                              boundary=boundary.Clamped)
+    assert elastic_core_nodes(sim, shots) == want

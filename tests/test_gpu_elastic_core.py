@@ -13,7 +13,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from helpers import Receivers, host, rel_max
+from helpers import Receivers, elastic_core_nodes, host, rel_max
 
 pytestmark = pytest.mark.gpu
 
@@ -82,3 +82,47 @@ def test_the_core_s_gradient_matches_the_oracle(precision, tol):
                                      sensors, observed)
     assert abs(cost - ocost) <= 1e-5 * ocost
     assert rel_max(gradient, ograd) < tol
+
+
+# the shapes of a core block the cases above leave out: 32 lanes (512 threads) in both
+# precisions, 16 of doubles, and 16 and 32 at the long stencils
+SHAPES = [
+    ((131, 150), 4, 20, 8, "float32", LINED, 8, (1, 2, 3)),
+    ((150, 146), 8, 20, 8, "float32", LINED, 6, (1, 2, 3)),
+    ((140, 137), 6, 16, 8, "float32", ((T, C), (C, T)), 0, ()),
+    ((128, 140), 4, 12, 8, "float64", LINED, 8, (1, 2, 3)),
+    ((131, 133), 4, 20, 8, "float64", LINED, 7, (1, 2, 3)),
+    ((129, 131), 2, 20, 8, "float64", ((C, T), (T, T)), 0, ()),
+]
+
+
+def _id(a):
+    return f"{a[0][0]}x{a[0][1]}-o{a[1]}-b{a[2]}-{a[4]}"
+
+
+@pytest.mark.parametrize("args", CASES + SHAPES, ids=_id)
+def test_a_case_runs_through_the_core(args):
+    assert elastic_core_nodes(_case(*args)[0], args[2]) > 0
+
+
+@pytest.mark.parametrize("args", SHAPES, ids=_id)
+def test_every_shape_of_the_core_steps_to_the_oracle_s_bits(args):
+    test_the_core_steps_to_the_oracle_s_bits(args)
+
+
+@pytest.mark.parametrize("n, order, shots, precision", [
+    ((121, 149), 2, 5, "float32"), ((133, 149), 8, 6, "float32"), ((125, 141), 4, 16, "float32"),
+    ((125, 141), 4, 20, "float32"), ((121, 137), 6, 5, "float64"), ((121, 137), 4, 20, "float64")])
+def test_the_core_s_gradient_matches_the_oracle_at_other_shapes(n, order, shots, precision):
+    from oracle import elastic as E
+
+    print(f"case gradient {n} order {order} {shots} shots {precision}", flush=True)
+    sim, osim, gamma, sources, sensors = _case(n, order, shots, 24, precision, LINED, 6, (1, 2, 3))
+    assert elastic_core_nodes(sim, shots) > 0
+    _, records = wave.simulate_shots(sim, sources, gamma, sensors)
+    observed = [host(r) * 0.9 for r in records]
+    cost, gradient = utils.misfit_gradient(sim, sources, gamma, Receivers(sensors), observed)
+    ocost, ograd = E.misfit_gradient(osim, [(s.position, s.signal) for s in sources], gamma,
+                                     sensors, observed)
+    assert abs(cost - ocost) <= 1e-5 * ocost
+    assert rel_max(gradient, ograd) < (1e-4 if precision == "float32" else 1e-10)
