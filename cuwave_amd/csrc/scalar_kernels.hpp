@@ -642,10 +642,13 @@ __device__ __forceinline__ void forward_general(const FwdParams<T> &p,
     col = p.strip.map[idx];
   const T *__restrict__ u1 = p.u.at(t - 1);
   // the layer memory this node owns and its profile: in flight with the taps
-  // where a lane group is small (a one-shot 298 x 298 step 6.0 us without, 5.2
-  // with), and only when it is used in 3D or where a group is 16 bytes (held
-  // through the taps it would halve the waves a SIMD holds)
-  constexpr bool kEarly = NDIM < 3 && sizeof(Q) <= 8;
+  // in 1D and 2D for a single float lane (a 298 x 298 step of order 8 6.0 us
+  // without, 5.2 with), and only when it is used elsewhere: held through the
+  // taps it costs a group of 8 bytes a third of its waves (two floats at order
+  // 8 77 -> 105 registers, 6 waves a SIMD -> 4) and gives it nothing (300 steps
+  // of 298 x 298, two shots: 2.66 ms either way; of 700 x 900 in double, order
+  // 8, one shot: 6.19 ms with, 5.61 without)
+  constexpr bool kEarly = NDIM < 3 && sizeof(Q) <= 4;
   Q mem[NDIM][3];
   T pr[NDIM][6];
   uint64_t own[NDIM];
