@@ -9,14 +9,18 @@
 // optimiser and in bfloat16 for the kernels.
 //
 // - forward: y[p][co] = act(bias[co] + sum_{tap, ci} x[p + off(tap)][ci] w[co][tap][ci]),
-//   a GEMM of M = pixels, N = cout, K = 9 cin; the x tile is gathered per
-//   tap (zero off the image) and staged in LDS with the weight tile.
-// - backward data: the same kernel on dy with the weights flipped in space
+//   added tap by tap. A block takes a tile of 8 x 32 pixels, whose input with
+//   its halo is in LDS once for all nine taps (conv3x3_fwd); images of a few
+//   pixels a side and more than 128 channels take runs of 128 pixels, gathered
+//   a tap at a time (conv3x3_fwd_flat): the same sums in the same order.
+// - backward data: the same kernels on dy with the weights flipped in space
 //   and transposed in channels (wd[ci][tap][co] = w[co][8 - tap][ci]).
-// - backward weight: dw[co][tap][ci] = sum_p dy[p][co] x[p + off(tap)][ci],
-//   a GEMM of M = 9 cin, N = cout reduced over the pixels: each block sums a
-//   contiguous run of pixels into a float32 partial, and a second kernel
-//   adds the partials in a fixed order (deterministic, no atomics).
+// - backward weight: dw[co][tap][ci] = sum_p dy[p][co] x[p + off(tap)][ci].
+//   A block marches down the rows of a strip of 64 columns with every tap's
+//   sums in registers (conv3x3_wgrad); small images and layers take runs of
+//   pixels a block (conv3x3_wgrad_flat). Either writes its float32 partial to a
+//   slice, and slices_sum adds the slices in a fixed order (deterministic, no
+//   atomics).
 //
 // MFMA v_mfma_f32_32x32x16_bf16: lane l holds A[l % 32][8 (l / 32) + i] and
 // B[8 (l / 32) + i][l % 32], i = 0 .. 7, and D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32]
@@ -50,10 +54,6 @@ __device__ __forceinline__ uint16_t to_bf16(float v) {
   return (uint16_t)((bits + 0x7fffu + ((bits >> 16) & 1u)) >> 16);
 }
 
-__device__ __forceinline__ float from_bf16(uint16_t b) {
-  return __uint_as_float((uint32_t)b << 16);
-}
-
 struct Image {
   int n, h, w; // batch, height, width
   int64_t pixels;
@@ -73,7 +73,11 @@ __device__ __forceinline__ int64_t shifted(const Image &im, int64_t p, int tap) 
 
 // ------------------------------------------------------------ forward
 // One block: a tile of kTH x kTW pixels of one image and every output channel
-// (BN = cout, 32 / 64 / 128). The sums run tap by tap, 16 channels an
+// (BN = cout, 32 / 64 / 128). A 32 -> 32 layer has 144 flops a byte of
+// activations read and written, so the input has to reach the block once; what
+// bounds it then is the LDS, its bandwidth and, from 64 channels up, its size:
+// two blocks a CU at 64, one at 128 (which has eight waves for it: with four
+// 128 -> 64 at 16 x 290 x 304 took 526 us). The sums run tap by tap, 16 channels an
 // instruction within a tap: a pre-activation within rounding of zero takes the
 // sign this order gives it, the ReLU's gradient follows that sign, and another
 // order turns some of them (a few in 1e8), each worth up to |dy w| in the
@@ -87,8 +91,11 @@ __device__ __forceinline__ int64_t shifted(const Image &im, int64_t p, int tap) 
 // products are too few to cover a barrier. A wave holds RW rows of 32 pixels
 // by NT tiles of 32 channels: RW + NT 16-byte LDS reads a lane for RW NT matrix
 // instructions, which at two by two is the LDS's rate at the instructions' own.
-// A layer's three passes at 16 x 290 x 304, 64 -> 64: 0.72 ms, and 0.67 with
-// the taps innermost, whose sums are in another order.
+//
+// At 16 x 580 x 608: 32 -> 32 220 us (279 with the taps innermost and the
+// channels staged in turn, 611 by the flat kernel), 64 -> 32 405 (417, 1240);
+// at half that 64 -> 64 199 (183, 424), 128 -> 64 363 (319, 841); 128 -> 128 at
+// a quarter 133 (180, 306).
 //
 // A plane of LDS holds eight channels of every staged pixel, so a wave's reads
 // are runs of 32 pixels; kPlane keeps the writes (a pixel's planes one after
@@ -113,18 +120,19 @@ template <int S> constexpr int plane_slots() {
   return (kHaloPixels - 16 / S + 15) / 16 * 16 + 16 / S;
 }
 
-template <int BN, int KC, int T>
-__global__ void __launch_bounds__(kThreads, 2)
+template <int BN, int KC, int T, int THREADS>
+__global__ void __launch_bounds__(THREADS, 2)
 conv3x3_fwd(Image im, int tiles_x, int tiles_y, int cin, const uint4 *__restrict__ x,
             const uint4 *__restrict__ wt, const float *__restrict__ bias, int relu,
             uint16_t *__restrict__ y) {
   constexpr int S = KC / 8;                     // 16-byte chunks a pixel a stage
+  constexpr int WAVES = THREADS / 64;
   constexpr int WN = BN == 128 ? 2 : 1;         // waves along the channels
-  constexpr int RW = kTH * WN / 4;              // pixel rows a wave
+  constexpr int RW = kTH * WN / WAVES;          // pixel rows a wave
   constexpr int NT = BN / WN / 32;              // channel tiles a wave
   constexpr int kPlane = plane_slots<S>();
   constexpr int kWeights = T * S * BN;          // chunks of weights a stage
-  constexpr int kMine = (kWeights + kThreads - 1) / kThreads;
+  constexpr int kMine = (kWeights + THREADS - 1) / THREADS;
   __shared__ uint4 sx[S * kPlane];              // [chunk][pixel]
   __shared__ uint4 sw[2][kWeights];             // [tap][chunk][channel ^ chunk]
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64, half = lane / 32;
@@ -145,7 +153,7 @@ conv3x3_fwd(Image im, int tiles_x, int tiles_y, int cin, const uint4 *__restrict
   auto fetch_weights = [&](int stage) {
 #pragma unroll
     for (int k = 0; k < kMine; ++k) {
-      const int t = tid + k * kThreads;
+      const int t = tid + k * THREADS;
       const int c = t % S, n = t / S % BN, tap = t / (S * BN);
       ahead[k] = uint4{0, 0, 0, 0};
       if (tap < T && c < cin8)
@@ -155,7 +163,7 @@ conv3x3_fwd(Image im, int tiles_x, int tiles_y, int cin, const uint4 *__restrict
   auto stage_weights = [&](int stage) {
 #pragma unroll
     for (int k = 0; k < kMine; ++k) {
-      const int t = tid + k * kThreads;
+      const int t = tid + k * THREADS;
       const int c = t % S, n = t / S % BN, tap = t / (S * BN);
       if (tap < T)
         sw[stage & 1][(tap * S + c) * BN + (n ^ (c & 15))] = ahead[k];
@@ -163,8 +171,8 @@ conv3x3_fwd(Image im, int tiles_x, int tiles_y, int cin, const uint4 *__restrict
   };
   fetch_weights(0);
 #pragma unroll
-  for (int k = 0; k < (kHaloPixels * S + kThreads - 1) / kThreads; ++k) {
-    const int t = tid + k * kThreads;
+  for (int k = 0; k < (kHaloPixels * S + THREADS - 1) / THREADS; ++k) {
+    const int t = tid + k * THREADS;
     const int c = t % S, p = t / S;
     const int py = y0 + p / kHaloW - 1, px = x0 + p % kHaloW - 1;
     if (p < kHaloPixels) {
@@ -336,26 +344,28 @@ conv3x3_fwd_flat(Image im, int cin, const uint4 *__restrict__ x, const uint4 *__
 template <int BN, int KC>
 void launch_fwd(const cw_conv3x3_args &a, const Image &im, hipStream_t s) {
   const int tx = (a.w + kTW - 1) / kTW, ty = (a.h + kTH - 1) / kTH;
-  hipLaunchKernelGGL((conv3x3_fwd<BN, KC, KC <= 32 ? 3 : 1>), dim3(tx * ty * a.n), dim3(kThreads),
-                     0, s, im, tx, ty, a.cin, (const uint4 *)a.x, (const uint4 *)a.weight,
+  constexpr int threads = KC == 128 ? 512 : 256;
+  hipLaunchKernelGGL((conv3x3_fwd<BN, KC, KC <= 32 ? 3 : 1, threads>), dim3(tx * ty * a.n),
+                     dim3(threads), 0, s, im, tx, ty, a.cin, (const uint4 *)a.x, (const uint4 *)a.weight,
                      (const float *)a.bias, a.relu, (uint16_t *)a.y);
 }
 
 // Whether the flat kernel takes the layer. It costs a pixel of an image what it
-// costs any other, the tiles a pixel of the padded image a half to a fifth of
+// costs any other, the tiles a pixel of the padded image a third to a fifth of
 // that: tiles, where they fill the card, from the share of true pixels up at
-// which both took the same time (at 16 channels to 32 in 0.19, 40000 x 6: 31.1
-// and 31.9 us; at 64 to 64 0.38, 25000 x 12: 87 and 90; at 128 to 128 0.63, 256
-// images of 40 x 40: 344 and 337), and tiles always where the card holds all of
-// them at once (4096 images of 8 x 8 at 128 channels 213 and 437 us, one of 8 x
-// 8 51 and 27). Past 128 channels the tile would be staged again for each tap
-// (6 x 200 x 225, 256 to 128: 446 us flat, 697 so).
+// which both took the same time (at 16 channels to 32 in 0.19, 40000 x 6: 31
+// and 32 us; at 64 to 64 0.30, 2048 images of 12 x 12 (0.28): 82 and 92, of 4 x
+// 40 (0.31): 88 and 83; at 128 to 128 0.33, the same two: 235 and 289, 266 and
+// 280, 25000 x 12 (0.38): 266 and 239), and tiles always where the card holds
+// all of them at once (4096 images of 8 x 8 at 128 channels 214 and 280 us, one
+// of 8 x 8 51 and 16). Past 128 channels the tile would be staged again for
+// each tap (6 x 200 x 225, 256 to 128: 446 us flat, 697 so).
 bool flat_fwd(const cw_conv3x3_args &a) {
   if (a.cin > 128)
     return true;
   const int64_t tiles = (int64_t)a.n * ((a.h + kTH - 1) / kTH) * ((a.w + kTW - 1) / kTW);
   const int at_once = a.cin <= 32 ? 1024 : a.cin <= 64 ? 512 : 256;
-  const double least = a.cin <= 32 ? 0.2 : a.cin <= 64 ? 0.38 : 0.65;
+  const double least = a.cin <= 32 ? 0.2 : a.cin <= 64 ? 0.3 : 0.33;
   return tiles > at_once && (double)a.n * a.h * a.w < least * (double)(tiles * (kTH * kTW));
 }
 
