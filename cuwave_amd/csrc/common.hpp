@@ -26,8 +26,10 @@ template <int NDIM> struct TileShape {
 };
 
 // division of an unsigned under 2^31 by a number the host knows: a product's
-// high half, an addition and a shift where the general division takes about
-// twenty instructions, three times over to find a node
+// high half, an addition and a shift (the rounded-up multiplier of Granlund and
+// Montgomery, Division by Invariant Integers using Multiplication, 1994) where
+// the general division takes about twenty instructions, three times over to
+// find a node
 struct Div {
   uint32_t m, s, d;
 };
