@@ -125,7 +125,7 @@ class _Head(torch.autograd.Function):
         """Whether the kernels compute what `x.float() @ w + b` would (not under autocast,
         which takes that product in its own type)."""
         return (x.dtype == torch.bfloat16 and w.dtype == b.dtype == torch.float32
-                and x.shape[-1] == w.shape[0] == 32 and 1 <= w.shape[1] <= 4
+                and w.ndim == 2 and x.shape[-1] == w.shape[0] == 32 and 1 <= w.shape[1] <= 4
                 and b.shape == w.shape[1:] and x.device == w.device == b.device
                 and not torch.is_autocast_enabled("cuda"))
 

@@ -287,7 +287,7 @@ def test_the_output_layer_is_differentiated_again_as_the_product_is():
         assert _rel(fwd.unpack_dual(y).tangent, x.float() @ t) < 1e-5
 
 
-@pytest.mark.parametrize("how", ["plain", "autocast", "wide bias", "one bias for all"])
+@pytest.mark.parametrize("how", ["plain", "autocast", "wide bias", "one bias for all", "vector"])
 def test_the_output_layer_s_kernels_step_aside_for_other_products(how):
     print(f"case head {how}", flush=True)
     torch.manual_seed(5)
@@ -296,6 +296,9 @@ def test_the_output_layer_s_kernels_step_aside_for_other_products(how):
         net.out_b = torch.nn.Parameter(net.out_b.detach().double())
     if how == "one bias for all":
         net.out_b = torch.nn.Parameter(net.out_b.detach()[:1])
+    if how == "vector":
+        net.out_w = torch.nn.Parameter(net.out_w.detach()[:, 0])
+        net.out_b = torch.nn.Parameter(net.out_b.detach()[0])
     seen = []
     net.dec1.register_forward_hook(lambda module, args, out: seen.append(out))
     with torch.no_grad(), torch.autocast("cuda", torch.bfloat16, enabled=how == "autocast"):
@@ -324,3 +327,19 @@ def test_a_gradient_that_starts_inside_another_tensor():
     results.append([unet._Head.apply(flat[1:].clone().view(x.shape), w, b)])
     for a, c in (*zip(*results[:2]), *zip(*results[2:])):
         torch.testing.assert_close(a, c, rtol=0, atol=0)
+
+
+@pytest.mark.parametrize("most", [1, 3, 40])
+@pytest.mark.parametrize("n, h, w", [(2, 40, 70), (700, 3, 5)])  # the strips', the flat kernel's
+def test_a_weight_gradient_keeps_to_the_slices_it_is_given(n, h, w, most, monkeypatch):
+    print(f"case slices {n}x{h}x{w} most {most}", flush=True)
+    g = torch.Generator().manual_seed(most)
+    x = _bf(torch.randn(n, h, w, 32, generator=g))
+    dy = _bf(torch.randn(n, h, w, 64, generator=g))
+    conv = unet.Conv3x3(32, 64, False)
+    ref_w = conv.weight.detach().clone().double().requires_grad_(True)
+    O.conv3x3(x.double(), ref_w, torch.zeros(64).double(), False).backward(dy.double())
+    monkeypatch.setattr(unet, "_splits", lambda *a: most)
+    conv = conv.cuda()
+    conv(x.cuda().bfloat16()).backward(dy.cuda().bfloat16())
+    assert _rel(conv.weight.grad, ref_w.grad) < 1e-4
